@@ -104,12 +104,13 @@ class Batch:
 
     def groups(self) -> list:
         """The current plan's launch groups (kind: wave / lds / global / lane /
-        gwave, the last one shot per wavefront on global amplitudes)."""
+        gwave, one shot per wavefront on global amplitudes, / shared, many
+        shots per workgroup on shared states; set_tuning names the others)."""
         n = ctypes.c_uint32()
         _lib.check(_lib.lib().clifft_svm_batch_info(self.handle, 0, None, ctypes.byref(n)), "batch_info")
         arr = (_lib.BatchGroupInfo * max(n.value, 1))()
         _lib.check(_lib.lib().clifft_svm_batch_info(self.handle, n.value, arr, ctypes.byref(n)), "batch_info")
-        kinds = ["wave", "lds", "global", "lane", "gwave"]
+        kinds = ["wave", "lds", "global", "lane", "gwave", "shared"]
         out = []
         for g in arr[:n.value]:
             d = {f: getattr(g, f) for f, _ in g._fields_}

@@ -24,7 +24,7 @@ INCLUDE = os.path.join(ROOT, "include")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 LIB_SVM = os.path.join(HERE, "libclifft_svm.so")
-SVM_SOURCES = ["svm_kernels.hip", "svm_host.cpp"]
+SVM_SOURCES = ["svm_kernels.hip", "svm_tree.hip", "svm_host.cpp"]
 LIB_PROBE = os.path.join(HERE, "libclifft_probe.so")
 
 HIP_FLAGS = [
@@ -39,14 +39,26 @@ def _run(cmd):
     subprocess.run(cmd, check=True)
 
 
+def _run_all(cmds):
+    """Independent compilations, side by side."""
+    procs = []
+    for cmd in cmds:
+        print(" ".join(cmd), flush=True)
+        procs.append((cmd, subprocess.Popen(cmd)))
+    for cmd, p in procs:
+        if p.wait():
+            raise subprocess.CalledProcessError(p.returncode, cmd)
+
+
 def build_svm(verbose: bool = True) -> str:
-    objs = []
+    objs, cmds = [], []
     os.makedirs(os.path.join(HERE, "_build"), exist_ok=True)
     for src in SVM_SOURCES:
         obj = os.path.join(HERE, "_build", src + ".o")
         lang = [] if src.endswith(".hip") else ["-x", "hip"]
-        _run([HIPCC, *HIP_FLAGS, *lang, "-I", INCLUDE, "-I", CSRC, "-c", os.path.join(CSRC, src), "-o", obj])
+        cmds.append([HIPCC, *HIP_FLAGS, *lang, "-I", INCLUDE, "-I", CSRC, "-c", os.path.join(CSRC, src), "-o", obj])
         objs.append(obj)
+    _run_all(cmds)
     tmp = LIB_SVM + ".tmp"
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, *objs])
     os.replace(tmp, LIB_SVM)

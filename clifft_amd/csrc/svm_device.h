@@ -28,6 +28,7 @@
 #include <type_traits>
 
 #include "clifft_svm.h"
+#include "svm_tree_args.h"
 
 #define CSVM_INLINE __device__ __forceinline__
 
@@ -126,6 +127,12 @@ struct DevProgram {
     uint32_t hz_buckets;  // 0: no guide (no sites or zero total hazard)
     uint32_t pad0;
     double hz_scale;      // hz_buckets / hazards[num_sites - 1]
+    // shared-state executor: its bytecode copy, passes and phases (tree_n 0: none)
+    const clifft_instruction* tree_bc;
+    const TreePass* tree_passes;
+    const TreePhase* tree_phases;
+    uint32_t tree_n;
+    uint32_t pad1;
 };
 
 // Host-visible state blob for single-shot execution from a preset state.
@@ -182,6 +189,8 @@ struct ShotArgs {
     const KfTables* kf;               // MODE_KFAULT
     uint32_t amp_slices;              // global tier: amplitude slices per team (2: fused runs; 3: and candidate folds)
     uint32_t pend_defer;              // with amp_slices >= 2: measurement passes read through pending expansions
+    uint32_t tree_chunk;              // shared-state executor: shots per team (amp_elems: entries of each of its two buffers)
+    uint32_t pad0;
 };
 
 // Opcodes that never read or write amplitudes nor depend on them, so

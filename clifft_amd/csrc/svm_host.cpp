@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "svm_internal.h"
+#include "svm_tree_plan.h"
 
 using namespace csvm;
 
@@ -314,6 +315,11 @@ struct clifft_svm_program {
     int64_t kf_k = -1;
     // launch planning
     LaunchShape base_shape;
+    // shared-state executor: (bits that may part the shots, rank) of every
+    // writing pass (empty: the program has no plan), and its code length
+    std::vector<std::pair<uint32_t, uint32_t>> tree_sizes;
+    uint32_t tree_n = 0;
+    bool tree_choices = false;  // frame bits, not outcomes alone, part the shots
     // staging for host outputs (grown on demand)
     void* out_dev = nullptr;
     size_t out_dev_bytes = 0;
@@ -683,10 +689,9 @@ void pack_array_fanouts(clifft_instruction* code, uint64_t n) {
     }
 }
 
-void lane_inline_operands(const clifft_program_view* v, clifft_instruction* code, const std::vector<uint8_t>& idle) {
-    const uint64_t n = v->num_instructions;
+void lane_inline_operands(const clifft_program_view* v, clifft_instruction* code, uint64_t n, const std::vector<uint8_t>& idle) {
     pack_frame_runs(code, n, idle);  // first, so the runs never hold the opcodes below
-    for (uint64_t i = 0; i < v->num_instructions; ++i) {
+    for (uint64_t i = 0; i < n; ++i) {
         clifft_instruction& in = code[i];
         uint64_t w2 = 0, w3 = 0;
         if (in.opcode == CLIFFT_OP_APPLY_PAULI) {
@@ -743,8 +748,8 @@ void lane_inline_operands(const clifft_program_view* v, clifft_instruction* code
 // A dormant measurement immediately followed by the APPLY_PAULI that its
 // record conditions (the reset after a measurement) becomes one lane
 // instruction (kLaneMeasPauli); the APPLY_PAULI's masks are already inline.
-void lane_fuse_meas_pauli(const clifft_program_view* v, clifft_instruction* code) {
-    for (uint64_t i = 0; i + 1 < v->num_instructions; ++i) {
+void lane_fuse_meas_pauli(clifft_instruction* code, uint64_t n) {
+    for (uint64_t i = 0; i + 1 < n; ++i) {
         clifft_instruction& m = code[i];
         const clifft_instruction& a = code[i + 1];
         if ((m.opcode != CLIFFT_OP_MEAS_DORMANT_STATIC && m.opcode != CLIFFT_OP_MEAS_DORMANT_RANDOM) ||
@@ -756,6 +761,53 @@ void lane_fuse_meas_pauli(const clifft_program_view* v, clifft_instruction* code
         std::memcpy(m.p.raw + 8, a.p.raw + 8, 16);
         ++i;
     }
+}
+
+// Drop the instructions that packed runs, fans and measurement + reset pairs
+// cover (a DETECTOR run reads its covered instructions and keeps them), so
+// the walk reads consecutive memory.
+std::vector<clifft_instruction> compact_covered(const std::vector<clifft_instruction>& code) {
+    std::vector<clifft_instruction> out;
+    for (size_t i = 0; i < code.size(); ++i) {
+        out.push_back(code[i]);
+        const uint32_t op = code[i].opcode;
+        if (op != kLaneFrameRun && op != kLaneFrameFan && op != kLaneMeasPauli) continue;
+        i += out.back().axis_2;
+        out.back().axis_2 = 0;
+    }
+    return out;
+}
+
+uint8_t forced_opcode(uint8_t op) {
+    return op >= CLIFFT_OP_MEAS_DORMANT_STATIC && op <= CLIFFT_OP_SWAP_MEAS_INTERFERE
+               ? (uint8_t)(op + (CLIFFT_OP_MEAS_DORMANT_STATIC_FORCED - CLIFFT_OP_MEAS_DORMANT_STATIC))
+               : op;
+}
+
+// The shared-state executor's bytecode for the sampled and the forced walk.
+void tree_bytecode(const clifft_program_view* v, const TreePlan& plan, std::vector<clifft_instruction>& sample,
+                   std::vector<clifft_instruction>& forced) {
+    std::vector<clifft_instruction> code = plan.code;
+    const std::vector<uint8_t> idle = frame_prune_enabled() ? plan.idle : std::vector<uint8_t>(code.size(), 0);
+    lane_inline_operands(v, code.data(), code.size(), idle);
+    forced = code;
+    for (clifft_instruction& in : forced) {
+        if (in.opcode == kTreeMeas) in.reserved |= 2u;
+        in.opcode = forced_opcode(in.opcode);
+    }
+    lane_fuse_meas_pauli(code.data(), code.size());
+    sample = compact_covered(code);
+    forced = compact_covered(forced);
+}
+
+// CLIFFT_SHARED_STATE: 0 turns the shared-state executor off, 2 uses it
+// wherever it can run; unset, tree_shape decides from its cost estimate.
+int shared_state_mode() {
+    static int v = [] {
+        const char* e = std::getenv("CLIFFT_SHARED_STATE");
+        return e ? std::atoi(e) : 1;
+    }();
+    return v;
 }
 
 // Highest peak rank run one shot per lane (CLIFFT_LANE_MAX_RANK overrides;
@@ -1026,6 +1078,17 @@ int choose_global_team(LaunchShape& L, uint64_t shots, uint32_t peak_rank) {
     return CLIFFT_OK;
 }
 
+// Bytes a launch's global amplitudes may take: what the device has free
+// (less 40% or 16 GiB headroom, whichever is larger), at most 192 GiB.
+size_t global_budget(hipStream_t st) {
+    size_t free_b = 0, total_b = 0;
+    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 8ull << 30;
+    size_t budget = free_b + arena_bytes(st);
+    const size_t headroom = std::max<size_t>(budget * 2 / 5, 16ull << 30);
+    budget = budget > headroom ? budget - headroom : (size_t)1 << 30;
+    return std::min<size_t>(budget, 192ull << 30);
+}
+
 int finalize_shape(clifft_svm_program* p, LaunchShape& L, uint64_t shots, hipStream_t st, void** gscratch) {
     DeviceInfo& di = device_info();
     int trc = choose_global_team(L, shots, p->peak_rank);
@@ -1038,14 +1101,7 @@ int finalize_shape(clifft_svm_program* p, LaunchShape& L, uint64_t shots, hipStr
     uint32_t per_cu = (uint32_t)std::max(per_cu_i, 1);
     uint64_t cap = (uint64_t)di.num_cus * per_cu;
     if (L.global_amps) {
-        // bound the global scratch by what the device has free (keep 40% or
-        // 16 GiB headroom, whichever is larger), at most 192 GiB
-        size_t free_b = 0, total_b = 0;
-        if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 8ull << 30;
-        size_t budget = free_b + arena_bytes(st);
-        size_t headroom = std::max<size_t>(budget * 2 / 5, 16ull << 30);
-        budget = budget > headroom ? budget - headroom : (size_t)1 << 30;
-        budget = std::min<size_t>(budget, 192ull << 30);
+        const size_t budget = global_budget(st);
         size_t per_team = ((size_t)16 << p->peak_rank) * L.amp_slices;
         uint64_t max_teams = std::max<uint64_t>(1, budget / per_team);
         cap = std::min<uint64_t>(cap, std::max<uint64_t>(1, max_teams / tpb));
@@ -1068,6 +1124,135 @@ int finalize_shape(clifft_svm_program* p, LaunchShape& L, uint64_t shots, hipStr
         if (rc) return rc;
     }
     return CLIFFT_OK;
+}
+
+// Entries of each amplitude buffer of a team of `chunk` shots, and the
+// entries all its passes visit: a pass over N nodes of rank r writes N 2^r,
+// and before it at most min(chunk, 2^bits) groups of shots can have parted.
+struct TreeWork {
+    uint64_t elems = 1, visited = 0;
+};
+TreeWork tree_work(const clifft_svm_program* p, uint32_t chunk) {
+    TreeWork w;
+    for (const auto& sr : p->tree_sizes) {
+        const uint64_t nodes = sr.first < 12 ? std::min<uint64_t>(chunk, 1ull << sr.first) : chunk;
+        w.elems = std::max(w.elems, nodes << sr.second);
+        w.visited += nodes << sr.second;
+    }
+    return w;
+}
+
+// A team shape of the shared-state executor for `chunk` shots on `threads`
+// threads; false where its tables do not fit.
+bool tree_team(const clifft_svm_program* p, uint32_t threads, uint32_t chunk, LaunchShape& L) {
+    const TreeWork w = tree_work(p, chunk);
+    if (w.elems > (1ull << 31)) return false;
+    const uint32_t rec_words = lane_words(p->total_slots) + lane_words(p->num_det) + lane_words(p->num_obs);
+    L = LaunchShape();
+    L.tree = true;
+    L.tree_chunk = chunk;
+    L.tree_elems = (uint32_t)w.elems;
+    L.block = threads;
+    L.lane_narrow = p->frame32;
+    L.lds_bytes = tree_team_lds(threads, chunk, rec_words);
+    L.global_amps = w.elems > kTreeLdsElems;
+    if (!L.global_amps) L.lds_bytes += 32u * (size_t)w.elems;
+    return L.lds_bytes <= kTreeMaxDynLds;
+}
+
+// Estimated time (us) of one chunk on a team of shape L, alone on its CU:
+// the walk, the passes' fixed part, and the entries visited at what the
+// team's wavefronts reach (fitted to a sweep of team sizes and chunks at
+// peak 6 to 16 on one MI355X).
+double tree_team_us(const clifft_svm_program* p, const LaunchShape& L) {
+    const double visited = (double)tree_work(p, L.tree_chunk).visited;
+    const double entry = (L.global_amps ? 0.32e-3 : 0.25e-3) * std::max(1.0, 512.0 / L.block);
+    return 15.0 + 0.2 * p->tree_n + 2.2 * p->tree_sizes.size() + 2.0e-3 * L.block + visited * entry;
+}
+// ... and of `shots` shots.
+double tree_cost(const clifft_svm_program* p, const LaunchShape& L, uint64_t shots) {
+    const double cus = device_info().num_cus;
+    const double teams = std::ceil((double)shots / L.tree_chunk);
+    const double per_cu = std::max(1.0, std::floor(std::min((double)kLdsBytes / (double)L.lds_bytes, 1024.0 / L.block)));
+    const double rounds = std::ceil(teams / (cus * per_cu));
+    const double visited = (double)tree_work(p, L.tree_chunk).visited;
+    // all teams together move 32 B an entry beyond the caches
+    const double bytes = L.global_amps ? std::min(teams, cus * per_cu) * 32.0 * (double)L.tree_elems : 0.0;
+    const double memory = bytes > 64e6 ? teams * visited * 32.0 / 4.0e6 : 0.0;
+    return std::max(rounds * tree_team_us(p, L) * (1.0 + 0.25 * (std::min(per_cu, std::ceil(teams / cus)) - 1.0)), memory);
+}
+
+// Whether `shots` shots of a program are better off sharing their states.
+// Measured on one MI355X, per-shot executors against this one (24-qubit
+// Clifford+T, and random programs with noise and frame-dependent phases,
+// where almost no shots share): from peak 11 on it is 1.3 to 48 times
+// faster from 100 shots up; at peak 7 to 10 it wins 2.6 to 66 times from
+// 10000 shots, 1.1 to 1.3 times at 100 to 1000 shots where only outcomes
+// part the shots, and loses up to a quarter at 100 to 1000 shots of a random
+// program; lanes keep peak 6 and below (1.45 and 2.9 times slower at peak 5
+// and 6 with 100000 shots, but faster up to 10000).
+bool tree_better(const clifft_svm_program* p, uint64_t shots) {
+    if (p->tree_sizes.empty() || shared_state_mode() == 0) return false;
+    if (shared_state_mode() == 2) return true;
+    const uint32_t k = p->peak_rank;
+    if (k >= 11) return true;
+    if (k >= 7) return shots >= 4096 || (!p->tree_choices && shots >= 100);
+    return k >= 5 && !p->tree_choices && shots >= 65536;
+}
+
+// The shared-state shape for a launch of `shots` shots: the team size and
+// the shots per team of the lowest estimate.  False: the program has no
+// plan, or the per-shot executors are faster.
+bool tree_shape(const clifft_svm_program* p, uint64_t shots, LaunchShape& best) {
+    if (!tree_better(p, shots)) return false;
+    double cost = 0.0;
+    bool found = false;
+    for (uint32_t threads : {256u, 512u, 1024u})
+        for (uint32_t chunk = threads; chunk >= 1; chunk /= 2) {
+            if (chunk > 2 * shots && chunk > 1) continue;
+            LaunchShape L;
+            if (!tree_team(p, threads, chunk, L)) continue;
+            const double c = tree_cost(p, L, shots);
+            if (!found || c < cost) {
+                best = L;
+                cost = c;
+                found = true;
+            }
+        }
+    return found;
+}
+
+// The shape in a batch, where other programs fill the device: the least
+// time of a compute unit, each team taking its part of one.
+bool tree_batch_shape(const clifft_svm_program* p, uint64_t shots, LaunchShape& best) {
+    if (p->peak_rank < 7 || !tree_better(p, std::max<uint64_t>(shots, 4096))) return false;
+    double cost = 0.0;
+    bool found = false;
+    for (uint32_t threads : {256u, 512u, 1024u})
+        for (uint32_t chunk = threads; chunk >= 64; chunk /= 2) {
+            if (chunk > 64 && chunk >= 2 * shots) continue;
+            LaunchShape L;
+            if (!tree_team(p, threads, chunk, L)) continue;
+            const double part = std::max((double)threads / 1024.0, (double)L.lds_bytes / (double)kLdsBytes);
+            const double c = std::ceil((double)shots / chunk) * part * tree_team_us(p, L);
+            if (!found || c < cost) {
+                best = L;
+                cost = c;
+                found = true;
+            }
+        }
+    return found;
+}
+
+int tree_finalize(LaunchShape& L, uint64_t shots, hipStream_t st, void** gscratch) {
+    int per_cu = 0;
+    HIP_TRY(shot_occupancy(L, &per_cu));
+    uint64_t cap = (uint64_t)device_info().num_cus * (uint64_t)std::max(per_cu, 1);
+    *gscratch = nullptr;
+    const size_t per_team = 32u * (size_t)L.tree_elems;
+    if (L.global_amps) cap = std::min<uint64_t>(cap, std::max<size_t>(1, global_budget(st) / per_team));
+    L.grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((shots + L.tree_chunk - 1) / L.tree_chunk, cap));
+    return L.global_amps ? ensure_scratch(st, L.grid * per_team, gscratch) : CLIFFT_OK;
 }
 
 void fill_common_args(clifft_svm_program* p, ShotArgs& A, void* gscratch, bool kfault = false) {
@@ -1248,6 +1433,24 @@ int clifft_svm_program_create(const clifft_program_view* view, clifft_svm_progra
     size_t o_u2 = add(view->u2_nodes, view->num_u2 * sizeof(clifft_u2_node));
     size_t o_u4 = add(view->u4_nodes, view->num_u4 * sizeof(clifft_u4_node));
     size_t o_eo = add(view->expected_observables, view->num_expected_observables);
+    // the shared-state executor's tables
+    TreePlan plan;
+    std::vector<clifft_instruction> tree_code, tree_forced;
+    if (!has_forced && shared_state_mode() != 0) {
+        TreePlanner planner(view, khist);
+        plan = planner.run();
+        if (plan.ok && !plan.passes.empty()) {
+            tree_bytecode(view, plan, tree_code, tree_forced);
+            p->tree_sizes = plan.sizes;
+            p->tree_n = (uint32_t)tree_code.size();
+            for (const clifft_instruction& in : tree_code) p->tree_choices |= in.opcode == kTreeChoice;
+        }
+    }
+    size_t o_trb = add(tree_code.data(), tree_code.size() * sizeof(clifft_instruction));
+    size_t o_trf = add(tree_forced.data(), tree_forced.size() * sizeof(clifft_instruction));
+    plan.passes.resize(plan.passes.size() + 1);  // the executor reads one ahead
+    size_t o_trp = add(plan.passes.data(), plan.passes.size() * sizeof(TreePass));
+    size_t o_trh = add(plan.phases.data(), plan.phases.size() * sizeof(TreePhase));
     size_t o_dp = add(nullptr, 2 * sizeof(DevProgram));
 
     std::vector<uint8_t> staging(total, 0);
@@ -1267,7 +1470,7 @@ int clifft_svm_program_create(const clifft_program_view* view, clifft_svm_progra
         auto* lbc = reinterpret_cast<clifft_instruction*>(staging.data() + o_lbc);
         std::memcpy(lbc, view->bytecode, view->num_instructions * sizeof(clifft_instruction));
         const std::vector<uint8_t> idle = identity_frame_ops(view);
-        if (view->words == 1) lane_inline_operands(view, lbc, idle);
+        if (view->words == 1) lane_inline_operands(view, lbc, view->num_instructions, idle);
         auto* lfbc = reinterpret_cast<clifft_instruction*>(staging.data() + o_lfbc);
         std::memcpy(lfbc, lbc, view->num_instructions * sizeof(clifft_instruction));
         for (uint64_t i = 0; i < view->num_instructions; ++i) {
@@ -1275,7 +1478,7 @@ int clifft_svm_program_create(const clifft_program_view* view, clifft_svm_progra
             if (op >= CLIFFT_OP_MEAS_DORMANT_STATIC && op <= CLIFFT_OP_SWAP_MEAS_INTERFERE)
                 op = (uint8_t)(op + (CLIFFT_OP_MEAS_DORMANT_STATIC_FORCED - CLIFFT_OP_MEAS_DORMANT_STATIC));
         }
-        if (view->words == 1) lane_fuse_meas_pauli(view, lbc);  // sampling copy only
+        if (view->words == 1) lane_fuse_meas_pauli(lbc, view->num_instructions);  // sampling copy only
         // the team interpreter's copies: frame runs packed (one-word frames)
         auto* tbc = reinterpret_cast<clifft_instruction*>(staging.data() + o_tbc);
         auto* tfbc = reinterpret_cast<clifft_instruction*>(staging.data() + o_tfbc);
@@ -1340,11 +1543,17 @@ int clifft_svm_program_create(const clifft_program_view* view, clifft_svm_progra
     d.num_ev = view->num_exp_vals;
     d.num_sites = view->num_sites;
     d.n_expected_obs = view->num_expected_observables;
+    d.tree_bc = reinterpret_cast<const clifft_instruction*>(base + o_trb);
+    d.tree_passes = reinterpret_cast<const TreePass*>(base + o_trp);
+    d.tree_phases = reinterpret_cast<const TreePhase*>(base + o_trh);
+    d.tree_n = (uint32_t)tree_code.size();
     {
         DevProgram both[2] = {d, d};
         both[1].bc = p->forced_bc;
         both[1].lane_bc = reinterpret_cast<const clifft_instruction*>(base + o_lfbc);
         both[1].team_bc = reinterpret_cast<const clifft_instruction*>(base + o_tfbc);
+        both[1].tree_bc = reinterpret_cast<const clifft_instruction*>(base + o_trf);
+        both[1].tree_n = (uint32_t)tree_forced.size();
         e = hipMemcpy(base + o_dp, both, sizeof(both), hipMemcpyHostToDevice);
         if (e != hipSuccess) {
             std::string msg = std::string("program upload: ") + hipGetErrorString(e);
@@ -1405,15 +1614,26 @@ static int run_shots(clifft_svm_program* p, uint64_t shots, uint64_t seed, uint3
     for (uint64_t base = 0; base < shots; base += chunk_max) {
         const uint64_t n = std::min(chunk_max, shots - base);
         const bool kfault = mode == MODE_KFAULT;
-        LaunchShape L = kfault ? plan_shape(p, false, true) : p->base_shape;
-        if (L.lds_bytes > kLdsBytes)
-            return fail(CLIFFT_E_UNSUPPORTED, "records and k-fault scratch do not fit the LDS of a team");
+        LaunchShape L;
         void* gs = nullptr;
-        int rc = finalize_shape(p, L, n, st, &gs);
+        int rc;
+        const bool tree = !kfault && tree_shape(p, n, L);
+        if (tree) {
+            rc = tree_finalize(L, n, st, &gs);
+        } else {
+            L = kfault ? plan_shape(p, false, true) : p->base_shape;
+            if (L.lds_bytes > kLdsBytes)
+                return fail(CLIFFT_E_UNSUPPORTED, "records and k-fault scratch do not fit the LDS of a team");
+            rc = finalize_shape(p, L, n, st, &gs);
+        }
         if (rc) return rc;
         ShotArgs A;
         fill_common_args(p, A, gs, kfault);
         A.amp_slices = L.global_amps ? L.amp_slices : 1u;
+        if (tree) {
+            A.amp_elems = L.tree_elems;
+            A.tree_chunk = L.tree_chunk;
+        }
         A.kf = kf;
         A.shot_begin = base;
         A.shot_count = n;
@@ -1884,6 +2104,7 @@ struct clifft_svm_batch {
     std::vector<clifft_svm_records> outs;
     uint32_t flags = 0;
     clifft_svm_batch_tuning tuning{};
+    bool shared = true;  // shared-state groups; off once the caller sets a tuning
     std::vector<BatchGroup> groups;
     std::vector<uint32_t> group_of;  // per program
     std::vector<ShotArgs> args;      // per program, for the current plan
@@ -1998,7 +2219,7 @@ bool batch_shape(const clifft_svm_program* p, const clifft_svm_batch_tuning& t, 
 }
 
 bool same_kernel(const LaunchShape& a, const LaunchShape& b) {
-    return a.lane == b.lane && a.lane_narrow == b.lane_narrow && a.nw == b.nw && a.block_team == b.block_team &&
+    return a.tree == b.tree && a.lane == b.lane && a.lane_narrow == b.lane_narrow && a.nw == b.nw && a.block_team == b.block_team &&
            a.global_amps == b.global_amps && a.block == b.block;
 }
 
@@ -2017,6 +2238,11 @@ size_t group_lds(const BatchGroup& g) {
 }
 
 void group_sizes(BatchGroup& g, const std::vector<clifft_svm_program*>& progs) {
+    if (g.L.tree) {  // each team holds two buffers; LDS as of the largest member
+        g.amp_elems = g.L.tree_elems;
+        g.amp_slices = 2;
+        return;
+    }
     g.amp_elems = 1;
     g.rec_stride = 0;
     g.wave_stride = 0;
@@ -2065,7 +2291,9 @@ int batch_group(clifft_svm_batch* b, uint64_t cap) {
     std::vector<uint32_t> group_of(b->progs.size());
     std::vector<LaunchShape> shape(b->progs.size());
     for (size_t i = 0; i < b->progs.size(); ++i) {
-        if (!batch_shape(b->progs[i], t, shape[i]))
+        if (b->shared && tree_batch_shape(b->progs[i], b->shots[i], shape[i])) {
+            // (grouped by kernel and team size below)
+        } else if (!batch_shape(b->progs[i], t, shape[i]))
             return fail(CLIFFT_E_UNSUPPORTED, "batch: the records of program " + std::to_string(i) +
                                                   " do not fit the LDS of a 256-thread team");
         size_t gi = 0;
@@ -2075,12 +2303,14 @@ int batch_group(clifft_svm_batch* b, uint64_t cap) {
             groups.back().L = shape[i];
         }
         groups[gi].progs.push_back((uint32_t)i);
+        groups[gi].L.lds_bytes = std::max(groups[gi].L.lds_bytes, shape[i].lds_bytes);  // (team tiers: group_sizes)
+        groups[gi].L.tree_elems = std::max(groups[gi].L.tree_elems, shape[i].tree_elems);
     }
     // A team group whose largest amplitudes and largest records do not fit
     // together hands its largest-record members to the global group.
     std::vector<uint32_t> evicted;
     for (BatchGroup& g : groups) {
-        if (g.L.lane || g.L.global_amps) continue;
+        if (g.L.lane || g.L.global_amps || g.L.tree) continue;
         std::stable_sort(g.progs.begin(), g.progs.end(), [&](uint32_t x, uint32_t y) {
             return rec_stride_of(b->progs[x]) > rec_stride_of(b->progs[y]);
         });
@@ -2128,9 +2358,14 @@ int batch_group(clifft_svm_batch* b, uint64_t cap) {
         for (uint32_t i : g.progs) {
             group_of[i] = (uint32_t)gi;
             const uint64_t n = std::min<uint64_t>(b->shots[i], cap);
-            const double c = shot_cost(b->progs[i], g.L);
-            for (uint64_t lo = 0; lo < n; lo += chunk) {
-                const uint64_t hi = std::min<uint64_t>(n, lo + chunk);
+            const uint32_t step = g.L.tree ? shape[i].tree_chunk : chunk;
+            const double c = g.L.tree ? tree_team_us(b->progs[i], shape[i]) / step : shot_cost(b->progs[i], g.L);
+            if (g.L.tree) {
+                b->args[i].tree_chunk = shape[i].tree_chunk;
+                b->args[i].amp_elems = shape[i].tree_elems;
+            }
+            for (uint64_t lo = 0; lo < n; lo += step) {
+                const uint64_t hi = std::min<uint64_t>(n, lo + step);
                 Pending w;
                 w.it.prog = i;
                 w.it.shot_lo = (uint32_t)lo;
@@ -2158,7 +2393,7 @@ int batch_audit(const clifft_svm_batch* b) {
         const std::string where = "batch plan, group " + std::to_string(gi) + ": ";
         if (L.lds_bytes > kBatchMaxDynLds) return fail(CLIFFT_E_INVALID, where + "LDS over the limit");
         if (L.block == 0 || L.block > 1024 || L.block % 64) return fail(CLIFFT_E_INVALID, where + "bad block");
-        if (!L.block_team && !L.lane && L.block > 256) return fail(CLIFFT_E_INVALID, where + "bad wave-team block");
+        if (!L.block_team && !L.lane && !L.tree && L.block > 256) return fail(CLIFFT_E_INVALID, where + "bad wave-team block");
         if (L.global_amps && !g.gscratch) return fail(CLIFFT_E_INVALID, where + "global group without scratch");
         if (L.global_amps && (size_t)g.teams_resident * g.amp_elems * g.amp_slices * 16 > g.gscratch_bytes)
             return fail(CLIFFT_E_INVALID, where + "global slices exceed the scratch");
@@ -2169,6 +2404,16 @@ int batch_audit(const clifft_svm_batch* b) {
             const ShotArgs& A = b->args[it.prog];
             if (it.shot_lo >= it.shot_hi || it.shot_hi > b->shots[it.prog])
                 return fail(CLIFFT_E_INVALID, where + "item shot range outside the program's shots");
+            if (L.tree) {
+                LaunchShape one;
+                if (it.shot_hi - it.shot_lo > A.tree_chunk || A.tree_chunk > L.block || A.tree_chunk == 0)
+                    return fail(CLIFFT_E_INVALID, where + "item over the team's shots");
+                if (!tree_team(p, L.block, A.tree_chunk, one) || one.lds_bytes > L.lds_bytes || one.global_amps != L.global_amps)
+                    return fail(CLIFFT_E_INVALID, where + "team tables exceed the launch's LDS");
+                if (A.amp_elems != one.tree_elems || one.tree_elems > g.amp_elems)
+                    return fail(CLIFFT_E_INVALID, where + "amplitude buffers exceed the team's");
+                continue;
+            }
             if (L.lane) {
                 const size_t need = lane_wave_bytes(p->peak_rank, p->total_slots, p->num_det, p->num_obs);
                 if (need > g.wave_stride || (size_t)(L.block / 64) * g.wave_stride > L.lds_bytes)
@@ -2268,6 +2513,7 @@ int batch_plan(clifft_svm_batch* b, uint64_t cap, hipStream_t st) {
         clifft_svm_program* p = b->progs[i];
         const BatchGroup& g = b->groups[b->group_of[i]];
         ShotArgs& A = b->args[i];
+        const uint32_t tree_chunk = A.tree_chunk, tree_elems = A.amp_elems;  // batch_group's
         fill_common_args(p, A, nullptr);
         A.shot_begin = 0;
         A.shot_count = b->shots[i];
@@ -2278,7 +2524,10 @@ int batch_plan(clifft_svm_batch* b, uint64_t cap, hipStream_t st) {
         A.out_obs = b->outs[i].observables;
         A.out_ev = b->outs[i].exp_vals;
         A.out_disc = b->outs[i].discarded;
-        if (!g.L.lane) {
+        if (g.L.tree) {
+            A.tree_chunk = tree_chunk;
+            A.amp_elems = tree_elems;
+        } else if (!g.L.lane) {
             A.amp_elems = g.amp_elems;
             A.rec_stride = g.rec_stride;
             A.amp_slices = g.L.global_amps && g.amp_slices >= 2 && mono_eligible(p)
@@ -2486,11 +2735,14 @@ int clifft_svm_batch_set_tuning(clifft_svm_batch* b, const clifft_svm_batch_tuni
     int rc = batch_check_tuning(*t);
     if (rc) return rc;
     clifft_svm_batch_tuning old = b->tuning;
+    const bool old_shared = b->shared;
     b->tuning = *t;
+    b->shared = false;  // the tuning names every program's group
     rc = batch_plan(b, ~0ull, library_stream());
     if (rc) {
         std::string msg = g_last_error;
         b->tuning = old;
+        b->shared = old_shared;
         (void)batch_plan(b, ~0ull, library_stream());
         return fail(rc, msg);
     }
@@ -2510,7 +2762,7 @@ int clifft_svm_batch_info(const clifft_svm_batch* b, uint32_t max_groups, clifft
     for (uint32_t gi = 0; gi < max_groups && gi < b->groups.size() && info; ++gi) {
         const BatchGroup& g = b->groups[gi];
         clifft_svm_batch_group_info& o = info[gi];
-        o.kind = g.L.lane ? 3u : (g.L.global_amps ? (g.L.block_team ? 2u : 4u) : (g.L.block_team ? 1u : 0u));
+        o.kind = g.L.tree ? 5u : g.L.lane ? 3u : (g.L.global_amps ? (g.L.block_team ? 2u : 4u) : (g.L.block_team ? 1u : 0u));
         o.programs = (uint32_t)g.progs.size();
         o.items = (uint32_t)g.items.size();
         o.grid = g.L.grid;

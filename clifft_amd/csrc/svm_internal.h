@@ -24,10 +24,13 @@ struct LaunchShape {
     bool lane_narrow = false;  // lane kernel with 32-bit frame words (at most 32 qubits)
     uint32_t amp_slices = 1;   // global-amplitude slices per team (2: fused permutation/phase runs, 3: and candidate folds)
     uint32_t rec_stride = 0;   // LDS bytes of one wavefront's record block (team tiers)
+    bool tree = false;         // shared-state executor (svm_tree.h); global_amps, lane_narrow, block and lds_bytes apply
+    uint32_t tree_chunk = 0;   // its shots per team
+    uint32_t tree_elems = 0;   // entries of each of a team's two amplitude buffers
     uint32_t block = 256;      // threads per workgroup
     uint32_t grid = 1;         // workgroups
     size_t lds_bytes = 0;      // dynamic LDS per workgroup
-    uint32_t teams_per_block() const { return lane ? block : (block_team ? 1u : block / 64u); }
+    uint32_t teams_per_block() const { return lane ? block : (block_team || tree ? 1u : block / 64u); }
 };
 
 // Resident workgroups per compute unit for the shape's kernel.
@@ -51,6 +54,16 @@ hipError_t batch_occupancy(const LaunchShape& L, int* blocks_per_cu);
 hipError_t launch_batch_group(const LaunchShape& L, const BatchArgs* B, hipStream_t st);
 // Zero n queue heads with a fill kernel (never a memset: graph-capturable).
 hipError_t clear_counters(uint32_t* counters, uint32_t n, hipStream_t st);
+
+// Amplitude buffers up to this many entries (each of a team's two) stay in LDS.
+constexpr uint64_t kTreeLdsElems = 2048;
+// Dynamic LDS limit of its kernels (less the queue head and the block-wide
+// "or" the runtime's library keeps in static LDS).
+constexpr size_t kTreeMaxDynLds = 158 * 1024;
+// Shared-state executor (svm_tree.hip): a shape's kernel, plain or batched,
+// and the LDS of a team apart from LDS amplitudes.
+const void* tree_kernel_fn(const LaunchShape& L, bool batch);
+uint32_t tree_team_lds(uint32_t threads, uint32_t chunk, uint32_t rec_words);
 
 // Adjoint-gradient executor (P and A are device memory).
 hipError_t adjoint_occupancy(bool global_amps, uint32_t block, size_t lds_bytes, int* blocks_per_cu);

@@ -295,39 +295,7 @@ __device__ __forceinline__ void lane_range(cptr<DevProgram> Pg, cptr<ShotArgs> A
 
             A = opaque(Ag);
             P = opaque(Pg);
-            const bool packed = (A->flags & CLIFFT_REC_PACKED) != 0;
-            const uint32_t n_exp = P->n_expected_obs;
-            cptr<uint8_t> expo = cp(P->expected_obs);
-            // record bits -> rows (bytes of 0/1, or little-endian bit-packed)
-            auto emit = [&](uint8_t* out, const lds_col_u32* src, uint32_t n, bool xor_expected) {
-                if (!out || n == 0) return;
-                if (packed) {
-                    const uint32_t nb = (n + 7u) / 8u;
-                    for (uint32_t j = 0; j < nb; ++j) {
-                        uint32_t byte = (src[(j >> 2) << 6] >> ((j & 3u) * 8u)) & 0xFFu;
-                        if (xor_expected) {
-                            uint32_t em = 0;
-                            for (uint32_t b = 0; b < 8; ++b)
-                                if (8 * j + b < n_exp) em |= (load_u8(expo, 8 * j + b) ? 1u : 0u) << b;
-                            byte ^= em;
-                        }
-                        if (8 * j + 8 > n) byte &= (1u << (n - 8 * j)) - 1u;
-                        out[s * nb + j] = (uint8_t)byte;
-                    }
-                } else {
-                    for (uint32_t i = 0; i < n; ++i) {
-                        uint32_t v = LaneInterp<FW>::rget(src, i);
-                        if (xor_expected && i < n_exp) v ^= load_u8(expo, i) ? 1u : 0u;
-                        out[s * n + i] = (uint8_t)v;
-                    }
-                }
-            };
-            emit(A->out_meas, S.rm, P->num_meas, false);
-            emit(A->out_det, S.rd, ndet, false);
-            emit(A->out_obs, S.ro, nobs, true);
-            if (A->out_disc) A->out_disc[s] = (uint8_t)S.discarded;
-            if (mode == MODE_FORCED && A->out_logp) A->out_logp[s] = S.reachable ? S.logp : kUnreachable;
-            if (S.dust && A->dust_counter) atomicAdd(A->dust_counter, (unsigned long long)S.dust);
+            lane_write_rows(P, A, S, s);
         }
     }
 }
@@ -543,14 +511,23 @@ static const void* shot_fn_fk(const LaunchShape& L) {
 }
 
 hipError_t shot_occupancy(const LaunchShape& L, int* blocks_per_cu) {
-    const void* fn = L.lane ? lane_fn(L)
+    const void* fn = L.tree ? tree_kernel_fn(L, false)
+                     : L.lane ? lane_fn(L)
                             : (L.nw == 1 ? shot_fn_fk<FRAME_W1>(L) : shot_fn_fk<FRAME_LANES>(L));
-    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    // (the tree kernels hold a few bytes of static LDS)
+    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       L.tree ? (int)kTreeMaxDynLds : 160 * 1024);
     if (e != hipSuccess) return e;
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, fn, (int)L.block, L.lds_bytes);
 }
 
+// (a tree shape's dynamic-LDS attribute is set by shot_occupancy, which
+// sizes its grid)
 hipError_t launch_shots(const LaunchShape& L, const DevProgram* P, const ShotArgs* A, hipStream_t st) {
+    if (L.tree) {
+        void* args[] = {&P, &A};
+        return hipLaunchKernel(tree_kernel_fn(L, false), dim3(L.grid), dim3(L.block), args, L.lds_bytes, st);
+    }
     if (L.lane) return launch_lane(L, P, A, st);
     switch (L.nw) {
         case 1: return launch_fk<FRAME_W1>(L, P, A, st);
@@ -568,6 +545,7 @@ static const void* batch_team_fn(bool block_team, bool global_amps) {
 }
 
 static const void* batch_fn(const LaunchShape& L) {
+    if (L.tree) return tree_kernel_fn(L, true);
     if (L.lane) {
         if (L.lane_narrow)
             return L.lane_dense ? reinterpret_cast<const void*>(batch_lane_kernel<6, uint32_t>)
@@ -582,7 +560,8 @@ static const void* batch_fn(const LaunchShape& L) {
 hipError_t batch_occupancy(const LaunchShape& L, int* blocks_per_cu) {
     const void* fn = batch_fn(L);
     // dynamic LDS may use what the static queue head leaves
-    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kBatchMaxDynLds);
+    hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                       (int)(L.tree ? kTreeMaxDynLds : kBatchMaxDynLds));
     if (e != hipSuccess) return e;
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, fn, (int)L.block, L.lds_bytes);
 }

@@ -301,6 +301,118 @@ struct LaneInterp {
         return res;
     }
 
+    // ------------------------------------------- opcodes without amplitudes
+    // a packed run of frame opcodes (kLaneFrameRun)
+    CSVM_INLINE void frame_run(uint32_t count, uint64_t w1, uint64_t w2, uint64_t w3) {
+        for (uint32_t j = 0; j < count; ++j) {
+            const uint64_t w = j < 4 ? w1 : (j < 8 ? w2 : w3);
+            const uint32_t f = (uint32_t)(w >> (16 * (j & 3u)));
+            const uint32_t fop = f & 7u, fa = (f >> 3) & 63u, fb = (f >> 9) & 63u;
+            if (fop == CLIFFT_OP_FRAME_CNOT) frame_cnot(fa, fb);
+            else if (fop == CLIFFT_OP_FRAME_CZ) frame_cz(fa, fb);
+            else if (fop == CLIFFT_OP_FRAME_SWAP) frame_swap(fa, fb);
+            else if (fop == CLIFFT_OP_FRAME_H) frame_h(fa);
+            else frame_s(fa);
+        }
+    }
+    // frame CZs or CNOTs sharing qubit p (kLaneFrameFan, svm_device.h)
+    CSVM_INLINE void frame_fan(uint32_t kind, uint32_t p, uint64_t mask) {
+        const FW m = (FW)mask, pb = (FW)1 << p;
+        if (kind == kFanCz) {
+            const FW xp = (px >> p) & 1u;
+            const FW par = (FW)(__popcll((uint64_t)(px & m)) & 1);
+            pz ^= (xp ? m : (FW)0) ^ (par ? pb : (FW)0);
+        } else if (kind == kFanControl) {
+            const FW xp = (px >> p) & 1u;
+            const FW par = (FW)(__popcll((uint64_t)(pz & m)) & 1);
+            px ^= xp ? m : (FW)0;
+            pz ^= par ? pb : (FW)0;
+        } else {
+            const FW zp = (pz >> p) & 1u;
+            const FW par = (FW)(__popcll((uint64_t)(px & m)) & 1);
+            px ^= par ? pb : (FW)0;
+            pz ^= zp ? m : (FW)0;
+        }
+    }
+    // DETECTORs with inline parities, each from its own words
+    CSVM_INLINE void detector_run(cptr<uint64_t> code, uint32_t pc, uint32_t more) {
+        for (uint32_t j = 0; j <= more; ++j) {
+            const uint64_t x0 = code[4 * (pc + j)], x1 = code[4 * (pc + j) + 1];
+            const uint64_t x2 = code[4 * (pc + j) + 2], x3 = code[4 * (pc + j) + 3];
+            const uint32_t e = (((uint32_t)(x0 >> 16) & 0xFF) & CLIFFT_FLAG_EXPECTED_ONE) ? 1u : 0u;
+            rset(rd, (uint32_t)(x1 >> 32), e ^ inline_parity(x2, x3));
+        }
+    }
+    // a dormant measurement; returns the record written
+    CSVM_INLINE uint32_t meas_dormant(uint32_t op, uint32_t a, uint32_t idx, uint32_t flags) {
+        const uint32_t sign = flags & CLIFFT_FLAG_SIGN;
+        uint32_t rec;
+        if (op == CLIFFT_OP_MEAS_DORMANT_STATIC) {
+            rec = (flags & CLIFFT_FLAG_IDENTITY) ? sign : (gx(a) ^ sign);
+        } else {
+            const uint32_t m = rng_double(rng) < 0.5 ? 0u : 1u;
+            set_x(a, m);
+            set_z(a, 0);
+            rec = m ^ sign;
+        }
+        rset(rm, idx, rec);
+        return rec;
+    }
+    // the forced kinds; false: the record is unreachable
+    CSVM_INLINE bool meas_dormant_forced(uint32_t op, uint32_t a, uint32_t idx, uint32_t flags) {
+        const uint32_t sign = flags & CLIFFT_FLAG_SIGN, req = forced[idx] ? 1u : 0u;
+        if (op == CLIFFT_OP_MEAS_DORMANT_STATIC_FORCED) {
+            if (req != ((flags & CLIFFT_FLAG_IDENTITY) ? sign : (gx(a) ^ sign))) {
+                reachable = 0;
+                return false;
+            }
+        } else {
+            logp += log(0.5);
+            set_x(a, req ^ sign);
+            set_z(a, 0);
+        }
+        rset(rm, idx, req);
+        return true;
+    }
+    CSVM_INLINE void noise_block(cptr<DevProgram> Pg, uint32_t begin, uint32_t end) {
+        if (next_noise >= begin && next_noise < end) {
+            cptr<DevProgram> P = opaque(Pg);
+            while (next_noise >= begin && next_noise < end) noise(P, next_noise);
+        }
+    }
+    CSVM_INLINE void readout_noise(cptr<DevProgram> P, uint32_t entry) {
+        if (rng_double(rng) < cp(P->ro_prob)[entry]) {
+            const uint32_t mi = cp(P->ro_meas_idx)[entry];
+            rset(rm, mi, rget(rm, mi) ^ 1u);
+        }
+    }
+    // DETECTOR, POSTSELECT, OBSERVABLE; false: the shot is discarded
+    CSVM_INLINE bool record_parity(cptr<DevProgram> Pg, uint32_t op, uint32_t flags, uint32_t list, uint32_t slot,
+                                   uint64_t w2, uint64_t w3) {
+        const bool observable = op == CLIFFT_OP_OBSERVABLE;
+        uint32_t par = !observable && (flags & CLIFFT_FLAG_EXPECTED_ONE) ? 1u : 0u;
+        if ((uint32_t)(w2 & 0xFFFF) == kLaneInlineParity) {
+            par ^= inline_parity(w2, w3);
+        } else {
+            cptr<DevProgram> P = opaque(Pg);
+            cptr<uint32_t> off = cp(observable ? P->obs_off : P->det_off), tgt = cp(observable ? P->obs_tgt : P->det_tgt);
+            const uint32_t j1 = off[list + 1];
+            for (uint32_t j = off[list]; j < j1; ++j) par ^= rget(rm, tgt[j]);
+        }
+        if (observable) {
+            rset(ro, slot, rget(ro, slot) ^ par);
+        } else if (op == CLIFFT_OP_DETECTOR) {
+            rset(rd, slot, par);
+        } else {
+            rset(rd, slot, 0);
+            if (par) {
+                discarded = 1;
+                return false;
+            }
+        }
+        return true;
+    }
+
     // ------------------------------------------------------------- dispatch
     // Runs this lane's shot over the lane copy of the bytecode (operands
     // inlined, superinstructions for runs of frame opcodes, detector runs and
@@ -344,60 +456,12 @@ struct LaneInterp {
                 continue;
             }
             switch (op) {
-                case kLaneFrameRun:  // a packed run of frame opcodes
-                    for (uint32_t j = 0; j < a1; ++j) {
-                        const uint64_t w = j < 4 ? w1 : (j < 8 ? w2 : w3);
-                        const uint32_t f = (uint32_t)(w >> (16 * (j & 3u)));
-                        const uint32_t fop = f & 7u, fa = (f >> 3) & 63u, fb = (f >> 9) & 63u;
-                        if (fop == CLIFFT_OP_FRAME_CNOT) frame_cnot(fa, fb);
-                        else if (fop == CLIFFT_OP_FRAME_CZ) frame_cz(fa, fb);
-                        else if (fop == CLIFFT_OP_FRAME_SWAP) frame_swap(fa, fb);
-                        else if (fop == CLIFFT_OP_FRAME_H) frame_h(fa);
-                        else frame_s(fa);
-                    }
+                case kLaneFrameRun: frame_run(a1, w1, w2, w3); break;
+                case kLaneFrameFan: frame_fan((uint32_t)(w0 >> 8) & 0xFFu, a1, w1); break;
+                case kLaneDetectorRun: detector_run(code, pc, a2); break;
+                case kLaneMeasPauli:
+                    if (meas_dormant((uint32_t)(w0 >> 8) & 0xFFu, a1, i0, flags)) apply_pauli(w2, w3);
                     break;
-                case kLaneFrameFan: {  // frame CZs or CNOTs sharing qubit a1 (svm_device.h)
-                    const FW m = (FW)w1, pb = (FW)1 << a1;
-                    const uint32_t kind = (uint32_t)(w0 >> 8) & 0xFFu;
-                    if (kind == kFanCz) {
-                        const FW xp = (px >> a1) & 1u;
-                        const FW par = (FW)(__popcll((uint64_t)(px & m)) & 1);
-                        pz ^= (xp ? m : (FW)0) ^ (par ? pb : (FW)0);
-                    } else if (kind == kFanControl) {
-                        const FW xp = (px >> a1) & 1u;
-                        const FW par = (FW)(__popcll((uint64_t)(pz & m)) & 1);
-                        px ^= xp ? m : (FW)0;
-                        pz ^= par ? pb : (FW)0;
-                    } else {
-                        const FW zp = (pz >> a1) & 1u;
-                        const FW par = (FW)(__popcll((uint64_t)(px & m)) & 1);
-                        px ^= par ? pb : (FW)0;
-                        pz ^= zp ? m : (FW)0;
-                    }
-                    break;
-                }
-                case kLaneDetectorRun:  // DETECTORs with inline parities, each from its own words
-                    for (uint32_t j = 0; j <= a2; ++j) {
-                        const uint64_t x0 = code[4 * (pc + j)], x1 = code[4 * (pc + j) + 1];
-                        const uint64_t x2 = code[4 * (pc + j) + 2], x3 = code[4 * (pc + j) + 3];
-                        const uint32_t e = (((uint32_t)(x0 >> 16) & 0xFF) & CLIFFT_FLAG_EXPECTED_ONE) ? 1u : 0u;
-                        rset(rd, (uint32_t)(x1 >> 32), e ^ inline_parity(x2, x3));
-                    }
-                    break;
-                case kLaneMeasPauli: {  // dormant measurement, then the APPLY_PAULI on its record
-                    uint32_t rec;
-                    if (((w0 >> 8) & 0xFF) == CLIFFT_OP_MEAS_DORMANT_STATIC) {
-                        rec = (flags & CLIFFT_FLAG_IDENTITY) ? sign : (gx(a1) ^ sign);
-                    } else {
-                        const uint32_t m = rng_double(rng) < 0.5 ? 0u : 1u;
-                        set_x(a1, m);
-                        set_z(a1, 0);
-                        rec = m ^ sign;
-                    }
-                    rset(rm, i0, rec);
-                    if (rec) apply_pauli(w2, w3);
-                    break;
-                }
                 case CLIFFT_OP_FRAME_CNOT: frame_cnot(a1, a2); break;
                 case CLIFFT_OP_FRAME_CZ: frame_cz(a1, a2); break;
                 case CLIFFT_OP_FRAME_H: frame_h(a1); break;
@@ -589,37 +653,14 @@ struct LaneInterp {
                     break;
                 }
                 case CLIFFT_OP_MEAS_DORMANT_STATIC:
-                    rset(rm, i0, (flags & CLIFFT_FLAG_IDENTITY) ? sign : (gx(a1) ^ sign));
-                    break;
-                case CLIFFT_OP_MEAS_DORMANT_RANDOM: {
-                    const uint32_t m = rng_double(rng) < 0.5 ? 0u : 1u;
-                    set_x(a1, m);
-                    set_z(a1, 0);
-                    rset(rm, i0, m ^ sign);
-                    break;
-                }
+                case CLIFFT_OP_MEAS_DORMANT_RANDOM: meas_dormant(op, a1, i0, flags); break;
                 case CLIFFT_OP_MEAS_ACTIVE_DIAGONAL: meas_diagonal(a1, i0, sign, false); break;
                 case CLIFFT_OP_MEAS_ACTIVE_INTERFERE: meas_interfere(a1, i0, sign, false); break;
                 case CLIFFT_OP_SWAP_MEAS_INTERFERE: swap_meas_interfere(a1, a2, i0, sign, false); break;
-                case CLIFFT_OP_MEAS_DORMANT_STATIC_FORCED: {
-                    const uint32_t det_v = (flags & CLIFFT_FLAG_IDENTITY) ? sign : (gx(a1) ^ sign);
-                    if ((forced[i0] ? 1u : 0u) != det_v) {
-                        reachable = 0;
-                        live = 0;
-                        break;
-                    }
-                    rset(rm, i0, det_v);
+                case CLIFFT_OP_MEAS_DORMANT_STATIC_FORCED:
+                case CLIFFT_OP_MEAS_DORMANT_RANDOM_FORCED:
+                    if (!meas_dormant_forced(op, a1, i0, flags)) live = 0;
                     break;
-                }
-                case CLIFFT_OP_MEAS_DORMANT_RANDOM_FORCED: {
-                    const uint32_t req = forced[i0] ? 1u : 0u;
-                    const uint32_t m = req ^ sign;
-                    logp += log(0.5);
-                    set_x(a1, m);
-                    set_z(a1, 0);
-                    rset(rm, i0, req);
-                    break;
-                }
                 case CLIFFT_OP_MEAS_ACTIVE_DIAGONAL_FORCED:
                     if (!meas_diagonal(a1, i0, sign, true)) live = 0;
                     break;
@@ -635,57 +676,13 @@ struct LaneInterp {
                 case CLIFFT_OP_NOISE:
                     if (i0 == next_noise) noise(opaque(Pg), i0);
                     break;
-                case CLIFFT_OP_NOISE_BLOCK: {
-                    const uint32_t end = i0 + i1;
-                    if (next_noise >= i0 && next_noise < end) {
-                        cptr<DevProgram> P = opaque(Pg);
-                        while (next_noise >= i0 && next_noise < end) noise(P, next_noise);
-                    }
-                    break;
-                }
-                case CLIFFT_OP_READOUT_NOISE: {
-                    cptr<DevProgram> P = opaque(Pg);
-                    if (rng_double(rng) < cp(P->ro_prob)[i0]) {
-                        const uint32_t mi = cp(P->ro_meas_idx)[i0];
-                        rset(rm, mi, rget(rm, mi) ^ 1u);
-                    }
-                    break;
-                }
+                case CLIFFT_OP_NOISE_BLOCK: noise_block(Pg, i0, i0 + i1); break;
+                case CLIFFT_OP_READOUT_NOISE: readout_noise(opaque(Pg), i0); break;
                 case CLIFFT_OP_DETECTOR:
-                case CLIFFT_OP_POSTSELECT: {
-                    uint32_t par = (flags & CLIFFT_FLAG_EXPECTED_ONE) ? 1u : 0u;
-                    if ((uint32_t)(w2 & 0xFFFF) == kLaneInlineParity) {
-                        par ^= inline_parity(w2, w3);
-                    } else {
-                        cptr<DevProgram> P = opaque(Pg);
-                        cptr<uint32_t> off = cp(P->det_off), tgt = cp(P->det_tgt);
-                        const uint32_t j1 = off[i0 + 1];
-                        for (uint32_t j = off[i0]; j < j1; ++j) par ^= rget(rm, tgt[j]);
-                    }
-                    if (op == CLIFFT_OP_DETECTOR) {
-                        rset(rd, i1, par);
-                    } else {
-                        rset(rd, i1, 0);
-                        if (par) {
-                            discarded = 1;
-                            live = 0;
-                        }
-                    }
+                case CLIFFT_OP_POSTSELECT:
+                case CLIFFT_OP_OBSERVABLE:
+                    if (!record_parity(Pg, op, flags, i0, i1, w2, w3)) live = 0;
                     break;
-                }
-                case CLIFFT_OP_OBSERVABLE: {
-                    uint32_t par = 0;
-                    if ((uint32_t)(w2 & 0xFFFF) == kLaneInlineParity) {
-                        par = inline_parity(w2, w3);
-                    } else {
-                        cptr<DevProgram> P = opaque(Pg);
-                        cptr<uint32_t> off = cp(P->obs_off), tgt = cp(P->obs_tgt);
-                        const uint32_t j1 = off[i0 + 1];
-                        for (uint32_t j = off[i0]; j < j1; ++j) par ^= rget(rm, tgt[j]);
-                    }
-                    rset(ro, i1, rget(ro, i1) ^ par);
-                    break;
-                }
                 case CLIFFT_OP_EXP_VAL: {
                     cptr<DevProgram> P = opaque(Pg);
                     const double r = exp_val(cp(P->ev_x)[i0], cp(P->ev_z)[i0], load_u8(cp(P->ev_sign), i0) ? 1u : 0u);
@@ -697,5 +694,44 @@ struct LaneInterp {
         }
     }
 };
+
+// A finished shot's rows: record bits as bytes of 0/1 or little-endian
+// bit-packed, the discard flag, the log-probability; s is the shot's index
+// within the launch.
+template <class L>
+CSVM_INLINE void lane_write_rows(cptr<DevProgram> P, cptr<ShotArgs> A, const L& S, uint64_t s) {
+    const bool packed = (A->flags & CLIFFT_REC_PACKED) != 0;
+    const uint32_t n_exp = P->n_expected_obs;
+    cptr<uint8_t> expo = cp(P->expected_obs);
+    auto emit = [&](uint8_t* out, const lds_col_u32* src, uint32_t n, bool xor_expected) {
+        if (!out || n == 0) return;
+        if (packed) {
+            const uint32_t nb = (n + 7u) / 8u;
+            for (uint32_t j = 0; j < nb; ++j) {
+                uint32_t byte = (src[(j >> 2) << 6] >> ((j & 3u) * 8u)) & 0xFFu;
+                if (xor_expected) {
+                    uint32_t em = 0;
+                    for (uint32_t b = 0; b < 8; ++b)
+                        if (8 * j + b < n_exp) em |= (load_u8(expo, 8 * j + b) ? 1u : 0u) << b;
+                    byte ^= em;
+                }
+                if (8 * j + 8 > n) byte &= (1u << (n - 8 * j)) - 1u;
+                out[s * nb + j] = (uint8_t)byte;
+            }
+        } else {
+            for (uint32_t i = 0; i < n; ++i) {
+                uint32_t v = L::rget(src, i);
+                if (xor_expected && i < n_exp) v ^= load_u8(expo, i) ? 1u : 0u;
+                out[s * n + i] = (uint8_t)v;
+            }
+        }
+    };
+    emit(A->out_meas, S.rm, P->num_meas, false);
+    emit(A->out_det, S.rd, P->num_det, false);
+    emit(A->out_obs, S.ro, P->num_obs, true);
+    if (A->out_disc) A->out_disc[s] = (uint8_t)S.discarded;
+    if (A->mode == MODE_FORCED && A->out_logp) A->out_logp[s] = S.reachable ? S.logp : kUnreachable;
+    if (S.dust && A->dust_counter) atomicAdd(A->dust_counter, (unsigned long long)S.dust);
+}
 
 }  // namespace csvm

@@ -1,0 +1,778 @@
+// svm_tree.h -- shared-state executor: many shots of one program per
+// workgroup, one copy of the amplitudes per group of shots that agree on
+// everything the amplitudes depend on.
+//
+// One shot per thread holds the Pauli frame, the xoshiro256++ state and its
+// record bits exactly as the lane interpreter does (svm_lane.h); every
+// thread walks the same bytecode.  Shots whose random
+// outcomes (and frame bits at phase opcodes) agreed so far have the same
+// amplitudes, bit for bit, so the team keeps one state per such group
+// ("node") and sweeps all nodes as one flat array: entry i of node n at
+// n 2^r + i.  An active measurement writes both outcomes' folded states of
+// every node and sums both probabilities; each shot then draws its own
+// outcome from its own stream, and the (node, outcome) pairs that occur
+// become the next nodes.  Nothing is approximated or carried over from one
+// launch to the next: a shot's record is the one the per-shot executors
+// give it.
+//
+// Why.  The per-shot tiers move the whole state once or twice per
+// measurement and shot and dispatch every opcode per shot.  Here a level
+// with N nodes of rank r moves N 2^r entries for all the shots together,
+// and N doubles at most while r falls by one: a team of 1000 shots at peak
+// 16 moves about 12 x 2^16 entries instead of 1000 x 2 x 2^16, and every
+// opcode is dispatched once per 64 shots.
+//
+// Measured on one MI355X (per launch, before -> after; before: the per-shot
+// tiers): 24-qubit Clifford+T, peak 10 x 20000 shots 2307 -> 82 us, peak 13
+// x 20000 2250 -> 147 us, peak 16 x 2000 1808 -> 291 us; 34 qubits, peak 25
+// x 64 shots 750 -> 67 ms; 512 programs x 1000 shots 54.3 -> 1.4 ms.  What
+// bounds it: up to peak 12 the bytecode walk (about 0.35 us a dispatch), from
+// peak 14 the passes (16 instructions and 32 bytes an entry).
+//
+// The array work itself is planned on the host (svm_tree_plan.h): each pass
+// gathers through a linear map over GF(2), so a lane's source index is the
+// XOR of a per-lane part, fixed for the pass, and a uniform part that
+// changes by one column between its entries.
+#pragma once
+
+#include "svm_lane.h"
+#include "svm_tree_args.h"
+#include "svm_sweeps.h"
+
+namespace csvm {
+
+struct TreeStage {  // the running pass's expansion products
+    double tab[1u << kTreeMaxExpand][2];
+};
+constexpr uint32_t kTreeParts = 128;  // partial sums of a pass with several per node
+constexpr uint32_t kTreeWindow = 256;  // bytecode instructions held in LDS
+
+// LDS of one team of `threads` threads and at most `chunk` shots: per-wave
+// record columns, two node tables (source node, choice word), per-node
+// sums, partial sums, two key bitmaps (and the rescale flag), the stage, the
+// bytecode window.
+__host__ __device__ inline uint32_t tree_flag_words(uint32_t chunk) { return (chunk + 1u) / 2u + 2u; }
+__host__ __device__ inline uint32_t tree_lds_bytes(uint32_t threads, uint32_t chunk, uint32_t rec_words) {
+    uint32_t b = (threads >> 6) * rec_words * 256u;
+    b += (16u * chunk + 15u) / 16u * 16u;  // 4 x u32 tables
+    b += 16u * chunk + 16u * kTreeParts;
+    b += (8u * tree_flag_words(chunk) + 15u) / 16u * 16u;
+    return b + (uint32_t)sizeof(TreeStage) + 32u * kTreeWindow;
+}
+
+template <class FW, class AmpT>
+struct TreeInterp : LaneInterp<FW> {
+    typedef LaneInterp<FW> L;
+    typedef __attribute__((address_space(3))) uint32_t lds_u32;
+    typedef __attribute__((address_space(3))) TreeStage lds_stage;
+    typedef __attribute__((address_space(3))) uint64_t lds_u64;
+    static constexpr uint32_t G = 4;  // pairs in flight per lane: eight 16-byte loads
+
+    uint32_t tid, lane, wave, nthreads, nwaves;
+    AmpT *src, *dst;
+    lds_u32 *nsrc, *nsrc2;  // node -> stored node
+    lds_u32 *nch, *nch2;    // node -> choice word
+    lds_u32 *flags, *flags2;
+    uint32_t scale_word;    // index of the rescale flag behind the bitmaps' words
+    lds_f64 *psum, *part;
+    lds_stage* stage;
+    lds_u64* window;        // bytecode instructions [.., ..) of the walk
+    uint32_t N;             // nodes
+    // the next pass's words (svm_tree_args.h), loaded while the one before
+    // it runs: lane b of `wa` the header, of the halves of `wa`, `wb`, `wc`
+    // the columns
+    uint32_t next, wa, wb, wc;
+    uint32_t node, live;    // this thread's shot
+
+    // ------------------------------------------------------------- splitting
+    // The live shots' keys (below nkeys) become the new node numbers, in key
+    // order.  Returns through `id` this shot's number and leaves N nodes.
+    // A node's old tables are still readable until the caller swaps them.
+    CSVM_INLINE uint32_t renumber(uint32_t key, uint32_t nkeys, uint32_t rescale) {
+        const uint32_t words = (nkeys + 31u) >> 5;
+        for (uint32_t w = tid; w < words; w += nthreads) flags[w] = 0u;
+        if (tid == 0) flags[scale_word] = 0u;
+        __syncthreads();
+        if (live) {
+            __hip_atomic_fetch_or(flags + (key >> 5), 1u << (key & 31u), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            if (rescale) flags[scale_word] = 1u;
+        }
+        __syncthreads();
+        if (words == 1u) {
+            const uint32_t w = flags[0];
+            N = uni((uint32_t)__popc(w));
+            return (uint32_t)__popc(w & ((1u << (key & 31u)) - 1u));
+        }
+        uint32_t total = 0, id = 0;
+        for (uint32_t base = 0; base < words; base += 64u) {
+            const uint32_t v = base + lane < words ? flags[base + lane] : 0u;
+            uint32_t incl = (uint32_t)__popc(v);
+#pragma unroll
+            for (int off = 1; off < 64; off <<= 1) {
+                const uint32_t up = (uint32_t)__shfl_up((int)incl, off, 64);
+                if (lane >= (uint32_t)off) incl += up;
+            }
+            const uint32_t at = (key >> 5) - base;  // wraps where the key lies before this block
+            const uint32_t excl = incl - (uint32_t)__popc(v);
+            const uint32_t e = (uint32_t)__shfl((int)excl, (int)(at & 63u), 64);
+            const uint32_t w = (uint32_t)__shfl((int)v, (int)(at & 63u), 64);
+            if (at < 64u) id = total + e + (uint32_t)__popc(w & ((1u << (key & 31u)) - 1u));
+            total += uni((uint32_t)__shfl((int)incl, 63, 64));
+        }
+        N = uni(total);
+        return id;
+    }
+    CSVM_INLINE void swap_tables() {
+        lds_u32* t = nsrc;
+        nsrc = nsrc2;
+        nsrc2 = t;
+        t = nch;
+        nch = nch2;
+        nch2 = t;
+        t = flags;
+        flags = flags2;
+        flags2 = t;
+    }
+    // kTreeChoice: part the shots of every node by `bits` frame bits
+    CSVM_INLINE void choice_split(uint32_t c, uint32_t bits, uint32_t at) {
+        if (!__syncthreads_or((int)(live && c != 0u))) return;  // every bit 0: nodes and choice words stay
+        const uint32_t id = renumber((node << bits) | c, N << bits, 0u);
+        if (live) {
+            nsrc2[id] = nsrc[node];
+            nch2[id] = nch[node] | (c << at);
+            node = id;
+        }
+        swap_tables();
+    }
+
+    // ----------------------------------------------------------------- passes
+    // The words of a coordinate index (svm_tree_args.h): the source offset,
+    // the written offset, the relative signs and the general-phase word.
+    struct Words {
+        uint32_t x, o, s, g;
+        CSVM_INLINE Words operator^(const Words& w) const { return Words{x ^ w.x, o ^ w.o, s ^ w.s, g ^ w.g}; }
+    };
+    // The running pass: its header in scalar registers, its columns spread
+    // over the wavefront's lanes.
+    struct Pass {
+        uint32_t type, r0, r, quarter, ngen, gen_off, sign0, ez_choices, lo;
+        uint32_t wa, wb, wc;
+        CSVM_INLINE static uint32_t at(uint32_t w, uint32_t i) { return (uint32_t)__builtin_amdgcn_readlane(w, i); }
+        CSVM_INLINE uint32_t head(uint32_t i) const { return at(wa, i); }
+        template <bool FULL>
+        CSVM_INLINE Words column(uint32_t b) const {
+            return Words{at(wa, 32u + b), at(wb, b), at(wb, 32u + b), FULL ? at(wc, b) : 0u};
+        }
+    };
+    CSVM_INLINE void load_pass(cptr<DevProgram> Pg, uint32_t i) {
+        const uint32_t* w = reinterpret_cast<const uint32_t*>(opaque(Pg)->tree_passes + i);
+        next = i;
+        wa = w[lane];
+        wb = w[64u + lane];
+        wc = w[128u + (lane & 31u)];
+    }
+    CSVM_INLINE static uint32_t odd(uint32_t i, uint32_t m) { return (uint32_t)__popc(i & m) & 1u; }
+    CSVM_INLINE static double flip(double a, uint32_t sign) {
+        return __longlong_as_double(__double_as_longlong(a) ^ ((long long)((unsigned long long)sign << 32)));
+    }
+    CSVM_INLINE static const AmpT* at(const AmpT* p, uint32_t off) {
+        return (const AmpT*)((const __attribute__((address_space(std::is_same<AmpT, lds_d2>::value ? 3 : 1))) char*)p + off);
+    }
+    CSVM_INLINE static AmpT* at(AmpT* p, uint32_t off) { return const_cast<AmpT*>(at(const_cast<const AmpT*>(p), off)); }
+
+    // sum over the 2^t lanes (t <= 6) that share the lane bits above t; every
+    // lane of them gets it
+    template <int CTRL>
+    CSVM_INLINE static double dpp_add(double a) {
+        const long long b = __double_as_longlong(a);
+        const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xF, 0xF, true);
+        const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xF, 0xF, true);
+        return a + __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+    }
+    CSVM_INLINE static void lanes_sum(double& a, double& b, uint32_t t) {
+        if (t >= 1u) a = dpp_add<0xB1>(a), b = dpp_add<0xB1>(b);    // quad_perm 1,0,3,2
+        if (t >= 2u) a = dpp_add<0x4E>(a), b = dpp_add<0x4E>(b);    // quad_perm 2,3,0,1
+        if (t >= 3u) a = dpp_add<0x141>(a), b = dpp_add<0x141>(b);  // row_half_mirror
+        if (t >= 4u) a = dpp_add<0x140>(a), b = dpp_add<0x140>(b);  // row_mirror
+        if (t >= 5u) a += __shfl_xor(a, 16, 64), b += __shfl_xor(b, 16, 64);
+        if (t >= 6u) a += __shfl_xor(a, 32, 64), b += __shfl_xor(b, 32, 64);
+    }
+
+    // K pairs whose words (pair bit clear) are w[], `pair` those of the pair
+    // bit: load, and (FULL) pending expansions and general phases.
+    template <uint32_t K, bool FULL>
+    CSVM_INLINE void gather(cptr<DevProgram> Pg, const Pass& q, const AmpT* sp, uint32_t ch, const Words& pair,
+                            const Words (&w)[K], dv2 (&p)[K], dv2 (&h)[K]) {
+        if (!FULL || q.r0 == q.r) {
+#pragma unroll
+            for (uint32_t e = 0; e < K; ++e) {
+                p[e] = *at(sp, w[e].x);
+                h[e] = *at(sp, w[e].x ^ pair.x);
+            }
+        } else {
+#pragma unroll
+            for (uint32_t e = 0; e < K; ++e) {
+                p[e] = *at(sp, w[e].x & q.lo);
+                h[e] = *at(sp, (w[e].x ^ pair.x) & q.lo);
+            }
+            if (!q.ez_choices) {
+#pragma unroll
+                for (uint32_t e = 0; e < K; ++e) {
+                    const uint32_t a = w[e].x >> (q.r0 + 4u), b = (w[e].x ^ pair.x) >> (q.r0 + 4u);
+                    p[e] = cmul(p[e], mk(stage->tab[a][0], stage->tab[a][1]));
+                    h[e] = cmul(h[e], mk(stage->tab[b][0], stage->tab[b][1]));
+                }
+            } else {
+                cptr<TreePass> T = cp(opaque(Pg)->tree_passes) + next;
+                for (uint32_t b = 0; b < q.r - q.r0; ++b) {
+                    const uint32_t s = q.r0 + 4u + b, cb = (pair.x >> s) & 1u;
+                    const int32_t c = T->ez_choice[b];
+                    const double zi = T->ez[b][1];
+                    const dv2 z = mk(T->ez[b][0], (c >= 0 && ((ch >> (c & 31)) & 1u)) ? -zi : zi);
+#pragma unroll
+                    for (uint32_t e = 0; e < K; ++e) {
+                        const uint32_t xb = (w[e].x >> s) & 1u;
+                        if (xb) p[e] = cmul(p[e], z);
+                        if (xb ^ cb) h[e] = cmul(h[e], z);
+                    }
+                }
+            }
+        }
+        if (FULL && q.ngen) {
+            cptr<TreePhase> ph = cp(opaque(Pg)->tree_phases) + q.gen_off;
+            for (uint32_t j = 0; j < q.ngen; ++j) {
+                const int32_t c = ph[j].choice;
+                const double zi = ph[j].pi;
+                const dv2 z = mk(ph[j].pr, (c >= 0 && ((ch >> (c & 31)) & 1u)) ? -zi : zi);
+                const uint32_t cb = (pair.g >> j) & 1u;
+#pragma unroll
+                for (uint32_t e = 0; e < K; ++e) {
+                    const uint32_t b = (w[e].g >> j) & 1u;
+                    if (b) p[e] = cmul(p[e], z);
+                    if (b ^ cb) h[e] = cmul(h[e], z);
+                }
+            }
+        }
+    }
+    // what the pass makes of its pairs: writes at dp (and dh, half a state
+    // on), and sums into v0, v1; i[] + il (il per lane): their coordinates
+    template <uint32_t K, bool FULL>
+    CSVM_INLINE void finish(cptr<DevProgram> Pg, const Pass& q, AmpT* dp, AmpT* dh, uint32_t ch, const Words (&w)[K],
+                            const uint32_t (&i)[K], uint32_t il, bool ok, dv2 (&p)[K], dv2 (&h)[K], double& v0, double& v1) {
+        const uint32_t type = q.type;
+        if (type == TREE_INTERFERE || type == TREE_H) {
+            // the relative sign goes into the additions: +-1 times h
+#pragma unroll
+            for (uint32_t e = 0; e < K; ++e) {
+                const double sg = __hiloint2double((int)(0x3FF00000u | (w[e].s & 0x80000000u)), 0);
+                dv2 s, d;
+                if (q.quarter) {  // uniform: times +-i
+                    s = mk(__fma_rn(h[e].y, -sg, p[e].x), __fma_rn(h[e].x, sg, p[e].y));
+                    d = mk(__fma_rn(h[e].y, sg, p[e].x), __fma_rn(h[e].x, -sg, p[e].y));
+                } else {
+                    s = mk(__fma_rn(h[e].x, sg, p[e].x), __fma_rn(h[e].y, sg, p[e].y));
+                    d = mk(__fma_rn(h[e].x, -sg, p[e].x), __fma_rn(h[e].y, -sg, p[e].y));
+                }
+                if (ok) {
+                    *at(dp, w[e].o) = cscale(s, kInvSqrt2);
+                    *at(dh, w[e].o) = cscale(d, kInvSqrt2);
+                }
+                v0 = __fma_rn(s.x, s.x, __fma_rn(s.y, s.y, v0));
+                v1 = __fma_rn(d.x, d.x, __fma_rn(d.y, d.y, v1));
+            }
+            return;
+        }
+        if (type != TREE_COPY) {
+            // (the quarter turn of a diagonal measurement's upper half is a
+            // phase of the whole outcome, but U2 and EXP_VAL need it)
+#pragma unroll
+            for (uint32_t e = 0; e < K; ++e) {
+                const uint32_t s = w[e].s & 0x80000000u;
+                if (q.quarter && FULL) h[e] = mk(-h[e].y, h[e].x);
+                h[e] = mk(flip(h[e].x, s), flip(h[e].y, s));
+            }
+        }
+        if (FULL && type >= TREE_EV) {
+            const uint32_t evz = q.head(12), half = 1u << (q.r - 1u);
+            const bool imag = q.head(13) != 0u;
+#pragma unroll
+            for (uint32_t e = 0; e < K; ++e) {
+                const double zl = odd(i[e] + il, evz) ? -1.0 : 1.0, zh = odd(i[e] + half + il, evz) ? -1.0 : 1.0;
+                const double np = p[e].x * p[e].x + p[e].y * p[e].y, nh = h[e].x * h[e].x + h[e].y * h[e].y;
+                v1 += np + nh;
+                if (type == TREE_EV0) {
+                    v0 += zl * np + zh * nh;
+                } else {
+                    const double re = h[e].x * p[e].x + h[e].y * p[e].y, im = h[e].x * p[e].y - h[e].y * p[e].x;
+                    v0 += imag ? -(zl * im - zh * im) : (zl + zh) * re;
+                }
+            }
+            return;
+        }
+        if (FULL && type == TREE_U2) {
+            const double* m = &opaque(Pg)->u2[q.head(10)].matrices[(ch >> q.head(11)) & 3u][0][0];
+            const dv2 m00 = mk(m[0], m[1]), m01 = mk(m[2], m[3]), m10 = mk(m[4], m[5]), m11 = mk(m[6], m[7]);
+#pragma unroll
+            for (uint32_t e = 0; e < K; ++e) {
+                const dv2 a = p[e], b = h[e];
+                p[e] = cadd(cmul(m00, a), cmul(m01, b));
+                h[e] = cadd(cmul(m10, a), cmul(m11, b));
+            }
+        }
+#pragma unroll
+        for (uint32_t e = 0; e < K; ++e) {
+            if (ok) {
+                *at(dp, w[e].o) = p[e];
+                *at(dh, w[e].o) = h[e];
+            }
+            v0 = __fma_rn(p[e].x, p[e].x, __fma_rn(p[e].y, p[e].y, v0));
+            v1 = __fma_rn(h[e].x, h[e].x, __fma_rn(h[e].y, h[e].y, v1));
+        }
+    }
+    // a times the relative turn of a quad's corner (bit 31: corner 1, ...)
+    CSVM_INLINE static dv2 corner(dv2 a, const Pass& q, uint32_t s, uint32_t bit) {
+        const uint32_t f = (s >> bit) << 31;
+        if ((q.quarter >> bit) & 1u) a = mk(-a.y, a.x);
+        return mk(flip(a.x, f), flip(a.y, f));
+    }
+    // U4: quads of the top two coordinate bits, one at a time per lane
+    CSVM_INLINE void pass_u4(cptr<DevProgram> Pg, const Pass& q) {
+        const uint32_t s = q.r - 2u, n4 = 1u << s;
+        const size_t total = (size_t)N << s;
+        const Words c2 = q.template column<true>(q.r - 2u), c3 = q.template column<true>(q.r - 1u);
+        for (size_t f0 = (size_t)wave << 6; f0 < total; f0 += (size_t)nwaves << 6) {
+            const bool in = f0 + lane < total;
+            const size_t f = in ? f0 + lane : 0;  // lanes past the end repeat the first quad
+            const uint32_t n = (uint32_t)(f >> s), i = (uint32_t)f & (n4 - 1u);
+            Words x = {0u, 0u, q.sign0, 0u};
+            for (uint32_t b = 0; b < s; ++b) {
+                const Words c = q.template column<true>(b);
+                if ((i >> b) & 1u) x = x ^ c;
+            }
+            const uint32_t ch = nch[n];
+            // the pairs (bit r-2 clear, bit r-1 free) and (bit r-2 set, bit r-1 free)
+            const Words w[2] = {x, x ^ c2};
+            dv2 lo[2], hi[2];
+            gather<2, true>(Pg, q, src + ((size_t)nsrc[n] << q.r0), ch, c3, w, lo, hi);
+            lo[1] = corner(lo[1], q, x.s, 31u);
+            hi[0] = corner(hi[0], q, x.s, 30u);
+            hi[1] = corner(hi[1], q, x.s, 29u);
+            if (in) {
+                const double* m = &opaque(Pg)->u4[q.head(10)].entries[(ch >> q.head(11)) & 15u].matrix[0][0][0];
+                AmpT* dp = dst + ((size_t)n << q.r);
+#pragma unroll 1
+                for (uint32_t row = 0; row < 4; ++row) {
+                    const double* e = m + 8 * row;
+                    dv2 acc = cmul(mk(e[0], e[1]), lo[0]);
+                    acc = cadd(acc, cmul(mk(e[2], e[3]), lo[1]));
+                    acc = cadd(acc, cmul(mk(e[4], e[5]), hi[0]));
+                    acc = cadd(acc, cmul(mk(e[6], e[7]), hi[1]));
+                    dp[i + row * n4] = acc;
+                }
+            }
+        }
+    }
+    // A unit of a node: 2^ub wavefront steps of 64 pairs in Gray order from
+    // coordinate i0 (words wu, uniform) on, K pairs per lane at a time.
+    template <uint32_t K, bool FULL>
+    CSVM_INLINE void unit(cptr<DevProgram> Pg, const Pass& q, const AmpT* sp, AmpT* dp, AmpT* dh, uint32_t ch,
+                          const Words& pair, const Words& wl, Words wu, uint32_t i0, uint32_t steps, double& v0, double& v1) {
+        for (uint32_t j0 = 0; j0 < steps; j0 += K) {
+            uint32_t i[K];
+            Words w[K];
+#pragma unroll
+            for (uint32_t e = 0; e < K; ++e) {
+                if (j0 + e != 0u) {  // one coordinate bit flips
+                    const uint32_t b = 6u + (uint32_t)__builtin_ctz(j0 + e);
+                    i0 ^= 1u << b;
+                    wu = wu ^ q.template column<FULL>(b);
+                }
+                i[e] = i0;
+                w[e] = wl ^ wu;
+            }
+            dv2 p[K], h[K];
+            gather<K, FULL>(Pg, q, sp, ch, pair, w, p, h);
+            finish<K, FULL>(Pg, q, dp, dh, ch, w, i, lane, true, p, h, v0, v1);
+        }
+    }
+    // The pass over nodes of 64 pairs or more: a wavefront takes a unit at a
+    // time.  A node's units are dealt to 2^pb sums.
+    template <uint32_t K, bool FULL>
+    CSVM_INLINE void units(cptr<DevProgram> Pg, const Pass& q, const Words& pair, const Words& wl, uint32_t ub, uint32_t upn,
+                           uint32_t pb) {
+        const uint32_t t = q.r - 1u, steps = 1u << ub, items = N << pb, pp = 1u << pb;
+        for (uint32_t item = wave; item < items; item += nwaves) {
+            const uint32_t n = item >> pb;
+            const AmpT* sp = src + ((size_t)uni(nsrc[n]) << q.r0);
+            AmpT* dp = dst + ((size_t)n << q.r);
+            AmpT* dh = dp + (1u << t);
+            const uint32_t ch = uni(nch[n]);
+            double v0 = 0.0, v1 = 0.0;
+            Words wu = {0u, 0u, 0u, 0u};
+            uint32_t before = 0;
+            for (uint32_t u = item & (pp - 1u); u < upn; u += pp) {
+                for (uint32_t d = u ^ before; d; d &= d - 1u)
+                    wu = wu ^ q.template column<FULL>(6u + ub + (uint32_t)__builtin_ctz(d));
+                before = u;
+                unit<K, FULL>(Pg, q, sp, dp, dh, ch, pair, wl, wu, u << (6u + ub), steps, v0, v1);
+            }
+            lanes_sum(v0, v1, 6u);
+            if (lane == 0u) {
+                lds_f64* o = pb == 0u ? psum : part;
+                o[2 * item] = v0;
+                o[2 * item + 1] = v1;
+            }
+        }
+    }
+
+    // The next pass over every node.  Afterwards psum holds the nodes' sums
+    // (pairs (v0, v1)), written states are in src, and every wavefront sees
+    // both.  Returns the pass's rank and type through the arguments.
+    CSVM_INLINE void pass(cptr<DevProgram> Pg, uint32_t& rank, int32_t& ev_sign) {
+        Pass q;
+        q.wa = wa;
+        q.wb = wb;
+        q.wc = wc;
+        q.type = q.head(0);
+        q.r0 = q.head(1);
+        q.r = q.head(3);
+        q.quarter = q.head(4);
+        q.ngen = q.head(5);
+        q.gen_off = q.head(6);
+        q.sign0 = q.head(7);
+        q.ez_choices = q.head(8);
+        q.lo = (16u << q.r0) - 1u;
+        rank = q.r;
+        ev_sign = (int32_t)q.head(14);
+        const uint32_t reset = q.head(9), t = q.r - 1u;
+        const bool full = q.r0 != q.r || q.ngen || q.type > TREE_H;
+        if (q.r0 != q.r && !q.ez_choices && tid < (1u << (q.r - q.r0))) {
+            cptr<TreePass> T = cp(opaque(Pg)->tree_passes) + next;
+            stage->tab[tid][0] = T->ez_tab[tid][0];
+            stage->tab[tid][1] = T->ez_tab[tid][1];
+        }
+        __syncthreads();  // the stage, and the node tables of the last split
+        uint32_t pb = 0;  // sums per node: 2^pb
+        if (q.type == TREE_U4) {
+            pass_u4(Pg, q);
+        } else {
+            const Words pair = q.template column<true>(t);
+            // the part of the words that a lane's own coordinate bits give
+            Words wl = {0u, 0u, q.sign0, 0u};
+            const uint32_t lb = t < 6u ? t : 6u;
+            for (uint32_t b = 0; b < lb; ++b) {
+                const Words c = q.template column<true>(b);
+                if ((lane >> b) & 1u) wl = wl ^ c;
+            }
+            if (t <= 6u) {
+                // one pair per lane, 2^(6-t) nodes per wavefront step
+                const uint32_t total = N << t, il = lane & ((1u << t) - 1u), zero[1] = {0u};
+                const Words w[1] = {wl};
+                for (uint32_t f0 = wave << 6; f0 < total; f0 += nwaves << 6) {
+                    const bool ok = f0 + lane < total;
+                    const uint32_t n = ok ? (f0 + lane) >> t : 0u;  // lanes past the end repeat node 0
+                    const uint32_t ch = nch[n];
+                    dv2 p[1], h[1];
+                    double v0 = 0.0, v1 = 0.0;
+                    AmpT* dp = dst + ((size_t)n << q.r);
+                    gather<1, true>(Pg, q, src + ((size_t)nsrc[n] << q.r0), ch, pair, w, p, h);
+                    finish<1, true>(Pg, q, dp, dp + (1u << t), ch, w, zero, il, ok, p, h, v0, v1);
+                    lanes_sum(v0, v1, t);
+                    if (ok && il == 0u) {
+                        psum[2 * n] = v0;
+                        psum[2 * n + 1] = v1;
+                    }
+                }
+            } else {
+                const uint32_t ub = t - 6u < 3u ? t - 6u : 3u, upn = 1u << (t - 6u - ub);
+                // about kTreeParts sums for the team to work on
+                while ((1u << pb) < upn && pb < 6u && (2u << pb) * N <= kTreeParts) ++pb;
+                if (full || ub == 1u)
+                    units<2, true>(Pg, q, pair, wl, ub, upn, pb);
+                else
+                    units<G, false>(Pg, q, pair, wl, ub, upn, pb);
+            }
+        }
+        load_pass(Pg, next + 1u);  // the table ends with a spare entry
+        __syncthreads();
+        if (pb) {  // a node's partial sums, in order
+            if (tid < N) {
+                const lds_f64* o = part + ((2u * tid) << pb);
+                double v0 = o[0], v1 = o[1];
+                for (uint32_t j = 1; j < (1u << pb); ++j) {
+                    v0 += o[2 * j];
+                    v1 += o[2 * j + 1];
+                }
+                psum[2 * tid] = v0;
+                psum[2 * tid + 1] = v1;
+            }
+            __syncthreads();
+        }
+        if (q.type < TREE_EV) {
+            AmpT* w = src;
+            src = dst;
+            dst = w;
+            if (q.type != TREE_DIAG && q.type != TREE_INTERFERE)
+                for (uint32_t n = tid; n < N; n += nthreads) {
+                    nsrc[n] = n;
+                    if (reset) nch[n] = 0u;
+                }
+        }
+    }
+
+    // The measurement's shots draw (or are told) their outcomes and part.
+    CSVM_INLINE void measure(uint32_t rank, uint32_t axis, uint32_t idx, uint32_t sign, bool interfere, bool forced_op) {
+        uint32_t b = 0, need = 0;
+        double pb = 0.0;
+        if (live) {
+            const double p0 = psum[2 * node], p1 = psum[2 * node + 1], total = p0 + p1;
+            uint32_t m_abs, rec;
+            if (this->choose(p0, p1, total, interfere ? this->gz(axis) : this->gx(axis), sign, idx, forced_op, b, m_abs, rec)) {
+                pb = b ? p1 : p0;
+                this->set_x(axis, m_abs);
+                this->set_z(axis, 0u);
+                L::rset(this->rm, idx, rec);
+                // svm.h:177-186 rescales the array once |gamma|, the inverse of
+                // its norm, leaves [1e-100, 1e100]
+                need = (pb < 1e-200 && pb > 0.0) || pb > 1e200;
+            } else {
+                live = 0;
+            }
+        }
+        const uint32_t key = 2u * node + b, id = renumber(key, 2u * N, need);
+        if (live) {
+            nsrc2[id] = key;
+            nch2[id] = 0u;
+            node = id;
+        }
+        const bool rescale = uni(flags[scale_word]) != 0u;
+        swap_tables();
+        if (rescale) {  // a node's shots have the same pb
+            __syncthreads();
+            if (live) psum[node] = need ? 1.0 / sqrt(pb) : 1.0;
+            __syncthreads();
+            for (uint32_t n = 0; n < N; ++n) {
+                const double s = unid(psum[n]);
+                AmpT* a = src + ((size_t)uni(nsrc[n]) << (rank - 1u));
+                if (s != 1.0)
+                    for (uint32_t i = tid; i < (1u << (rank - 1u)); i += nthreads) a[i] = cscale(a[i], s);
+            }
+            __syncthreads();
+        }
+    }
+
+    // ---------------------------------------------------------------- dispatch
+    // Walks the tree copy of the bytecode.  Tree opcodes are run by every
+    // thread (they hold barriers); the others by the live shots.
+    CSVM_INLINE void run(cptr<DevProgram> Pg, double* ev_row) {
+        cptr<DevProgram> P0 = opaque(Pg);
+        cptr<uint64_t> code = cp(reinterpret_cast<const uint64_t*>(P0->tree_bc));
+        const uint32_t n_instr = P0->tree_n;
+        uint32_t skip = 0, wbegin = 0, wend = 0;
+        for (uint32_t pc = 0; pc < n_instr; pc += 1 + skip) {
+            if (pc >= wend) {  // the next instructions into LDS: a scalar load from L2 each would cost more
+                wbegin = pc;
+                wend = pc + kTreeWindow < n_instr ? pc + kTreeWindow : n_instr;
+                const uint64_t* from = reinterpret_cast<const uint64_t*>(opaque(Pg)->tree_bc) + 4 * (size_t)pc;
+                __syncthreads();
+                for (uint32_t e = tid; e < 4u * (wend - wbegin); e += nthreads) window[e] = from[e];
+                __syncthreads();
+            }
+            const lds_u64* ins = window + 4u * (pc - wbegin);
+            const uint64_t w0 = uni64(ins[0]), w1 = uni64(ins[1]), w2 = uni64(ins[2]), w3 = uni64(ins[3]);
+            const uint32_t op = (uint32_t)(w0 & 0xFF);
+            const uint32_t reserved = (uint32_t)(w0 >> 8) & 0xFFu;
+            const uint32_t flags_ = (uint32_t)((w0 >> 16) & 0xFF);
+            const uint32_t a1 = (uint32_t)((w0 >> 32) & 0xFFFF);
+            const uint32_t a2 = (uint32_t)(w0 >> 48);
+            const uint32_t i0 = (uint32_t)w1, i1 = (uint32_t)(w1 >> 32);
+            skip = op >= kLaneFrameRun ? a2 : 0u;
+            if (op >= kTreeChoice && op <= kTreeEv) {
+                if (op == kTreeChoice) {
+                    uint32_t c = this->gx(a1);
+                    if (reserved >= 2u) c |= this->gz(a1) << 1;
+                    if (reserved == 4u) c |= (this->gx(a2) << 2) | (this->gz(a2) << 3);
+                    choice_split(c, reserved, i0);
+                    continue;
+                }
+                if (op == kTreeNode) {
+                    if (live) {
+                        cptr<DevProgram> P = opaque(Pg);
+                        const uint32_t s = (this->gz(a1) << 1) | this->gx(a1);
+                        uint32_t o;
+                        if (reserved) {
+                            const clifft_u4_entry* e = &P->u4[i0].entries[(this->gz(a2) << 3) | (this->gx(a2) << 2) | s];
+                            o = e->out_state;
+                            this->set_x(a2, (o >> 2) & 1u);
+                            this->set_z(a2, (o >> 3) & 1u);
+                        } else {
+                            const clifft_u2_node* e = P->u2 + i0;
+                            o = e->out_states[s];
+                        }
+                        this->set_x(a1, o & 1u);
+                        this->set_z(a1, (o >> 1) & 1u);
+                    }
+                    continue;
+                }
+                const uint32_t kind = (uint32_t)w2;
+                uint32_t rank = 0;
+                int32_t ev_sign = 1;
+                if (op != kTreeEv || kind == 0u) pass(Pg, rank, ev_sign);
+                if (op == kTreeMeas) {
+                    measure(rank, a1, i0, flags_ & CLIFFT_FLAG_SIGN, (reserved & 1u) != 0u, (reserved & 2u) != 0u);
+                } else if (op == kTreeEv && live && ev_row) {
+                    cptr<DevProgram> P = opaque(Pg);
+                    const uint64_t mx = cp(P->ev_x)[i0], mz = cp(P->ev_z)[i0];
+                    const uint32_t f = (load_u8(cp(P->ev_sign), i0) ? 1u : 0u) ^
+                                       ((uint32_t)(__popcll(mx & (uint64_t)this->pz) + __popcll(mz & (uint64_t)this->px)) & 1u);
+                    double v = kind == 1u ? 0.0 : 1.0;
+                    if (kind == 0u) {
+                        const double den = psum[2 * node + 1];
+                        v = den > 0.0 ? (double)ev_sign * psum[2 * node] / den : 0.0;
+                    }
+                    if (f) v = -v;
+                    v = v > 1.0 ? 1.0 : v;
+                    ev_row[i1] = v < -1.0 ? -1.0 : v;
+                }
+                continue;
+            }
+            if (!live) continue;
+            switch (op) {
+                case kLaneFrameRun: this->frame_run(a1, w1, w2, w3); break;
+                case kLaneFrameFan: this->frame_fan(reserved, a1, w1); break;
+                case kLaneDetectorRun: this->detector_run(code, pc, a2); break;
+                case kLaneMeasPauli:
+                    if (this->meas_dormant(reserved, a1, i0, flags_)) this->apply_pauli(w2, w3);
+                    break;
+                case CLIFFT_OP_FRAME_CNOT: this->frame_cnot(a1, a2); break;
+                case CLIFFT_OP_FRAME_CZ: this->frame_cz(a1, a2); break;
+                case CLIFFT_OP_FRAME_H: this->frame_h(a1); break;
+                case CLIFFT_OP_FRAME_S:
+                case CLIFFT_OP_FRAME_S_DAG: this->frame_s(a1); break;
+                case CLIFFT_OP_FRAME_SWAP: this->frame_swap(a1, a2); break;
+                case CLIFFT_OP_MEAS_DORMANT_STATIC:
+                case CLIFFT_OP_MEAS_DORMANT_RANDOM: this->meas_dormant(op, a1, i0, flags_); break;
+                case CLIFFT_OP_MEAS_DORMANT_STATIC_FORCED:
+                case CLIFFT_OP_MEAS_DORMANT_RANDOM_FORCED:
+                    if (!this->meas_dormant_forced(op, a1, i0, flags_)) live = 0;
+                    break;
+                case CLIFFT_OP_APPLY_PAULI:
+                    if (L::rget(this->rm, i1)) this->apply_pauli(w2, w3);
+                    break;
+                case CLIFFT_OP_NOISE:
+                    if (i0 == this->next_noise) this->noise(opaque(Pg), i0);
+                    break;
+                case CLIFFT_OP_NOISE_BLOCK: this->noise_block(Pg, i0, i0 + i1); break;
+                case CLIFFT_OP_READOUT_NOISE: this->readout_noise(opaque(Pg), i0); break;
+                case CLIFFT_OP_DETECTOR:
+                case CLIFFT_OP_POSTSELECT:
+                case CLIFFT_OP_OBSERVABLE:
+                    if (!this->record_parity(Pg, op, flags_, i0, i1, w2, w3)) live = 0;
+                    break;
+                default: break;
+            }
+        }
+    }
+};
+
+// The calling workgroup runs the chunks of A->tree_chunk shots from c_first
+// on, c_step apart, of the shots [s_lo, s_hi) of the program.  `buf` (LDS
+// amplitudes: unused) holds 2 x A->amp_elems entries of the team.
+template <class FW, class AmpT>
+__device__ __forceinline__ void tree_range(cptr<DevProgram> Pg, cptr<ShotArgs> Ag, uint64_t c_first, uint64_t c_step,
+                                           uint64_t s_lo, uint64_t s_hi, uint64_t seed, dv2* buf) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    TreeInterp<FW, AmpT> S;
+    typedef typename TreeInterp<FW, AmpT>::lds_u32 lds_u32;
+    S.tid = threadIdx.x;
+    S.lane = threadIdx.x & 63u;
+    S.wave = uni(threadIdx.x >> 6);
+    S.nthreads = blockDim.x;
+    S.nwaves = blockDim.x >> 6;
+    cptr<DevProgram> P = opaque(Pg);
+    cptr<ShotArgs> A = opaque(Ag);
+    const uint32_t chunk = A->tree_chunk, amp = A->amp_elems;
+    const uint32_t wm = lane_words(P->total_meas_slots), wd = lane_words(P->num_det);
+    const uint32_t nwords = wm + wd + lane_words(P->num_obs);
+    unsigned char* p = smem;
+    AmpT *b0, *b1;
+    if (std::is_same<AmpT, lds_d2>::value) {
+        b0 = (AmpT*)((dv2*)p);
+        b1 = b0 + amp;
+        p += 32u * (size_t)amp;
+    } else {
+        b0 = (AmpT*)buf;
+        b1 = b0 + amp;
+    }
+    lds_u32* tables = (lds_u32*)p;
+    p += (16u * chunk + 15u) / 16u * 16u;
+    S.psum = (lds_f64*)p;
+    S.part = S.psum + 2 * chunk;
+    p += 16u * chunk + 16u * kTreeParts;
+    lds_u32* flag0 = (lds_u32*)p;
+    const uint32_t fwords = tree_flag_words(chunk);
+    p += (8u * fwords + 15u) / 16u * 16u;
+    S.stage = (typename TreeInterp<FW, AmpT>::lds_stage*)p;
+    p += sizeof(TreeStage);
+    S.window = (typename TreeInterp<FW, AmpT>::lds_u64*)p;
+    p += 32u * kTreeWindow;
+    lds_col_u32* recs = (lds_col_u32*)(p + (size_t)S.wave * nwords * 256u) + S.lane;
+    S.scale_word = fwords - 1u;
+    S.rm = recs;
+    S.rd = recs + (wm << 6);
+    S.ro = S.rd + (wd << 6);
+    S.amp = nullptr;
+    S.k = 0;
+    for (uint64_t c = c_first;; c += c_step) {
+        const uint64_t s0 = s_lo + c * chunk;
+        if (s0 >= s_hi) break;
+        const uint64_t s = s0 + S.tid;
+        const bool mine = S.tid < chunk && s < s_hi;
+        A = opaque(Ag);
+        P = opaque(Pg);
+        for (uint32_t w = 0; w < nwords; ++w) recs[w << 6] = 0u;
+        S.px = S.pz = 0;
+        S.dust = 0;
+        S.discarded = 0;
+        S.reachable = 1;
+        S.logp = 0.0;
+        S.forced = nullptr;
+        S.next_noise = kNoNoise;
+        S.load_pass(P, 0);
+        S.rng = rng_for_shot(seed, A->shot_begin + s);
+        S.live = mine ? 1u : 0u;
+        S.node = 0;
+        S.N = 1;
+        S.src = b0;
+        S.dst = b1;
+        S.nsrc = tables;
+        S.nsrc2 = tables + chunk;
+        S.nch = tables + 2 * chunk;
+        S.nch2 = tables + 3 * chunk;
+        S.flags = flag0;
+        S.flags2 = flag0 + fwords;
+        double* ev_row = nullptr;
+        if (mine) {
+            S.next_noise = 0;
+            S.draw_next_noise(P, 0.0);
+            if (A->mode == MODE_FORCED) S.forced = A->forced_records + s * P->num_meas;
+            const uint32_t nev = P->num_ev;
+            ev_row = A->out_ev ? A->out_ev + s * nev : nullptr;
+            if (ev_row)
+                for (uint32_t i = 0; i < nev; ++i) ev_row[i] = 0.0;
+        }
+        if (S.tid == 0) {
+            S.nsrc[0] = 0u;
+            S.nch[0] = 0u;
+            S.src[0] = mk(1.0, 0.0);
+        }
+        __syncthreads();
+
+        S.run(Pg, ev_row);
+
+        if (mine) lane_write_rows(opaque(Pg), opaque(Ag), S, s);
+        __syncthreads();  // the tables and the state are rewritten by the next chunk
+    }
+}
+
+}  // namespace csvm
