@@ -131,8 +131,13 @@ struct DevProgram {
     const clifft_instruction* tree_bc;
     const TreePass* tree_passes;
     const TreePhase* tree_phases;
+    const uint32_t* lp_dense;      // whole responses, lp_words each
+    const uint32_t* lp_rows;       // rows, 8 words a unit
+    const TreeSite* lp_sites;
+    const TreeChan* lp_chans;
+    const uint32_t* lp_chan_rows;  // entries of the channels' rows
     uint32_t tree_n;
-    uint32_t pad1;
+    uint32_t lp_words;
 };
 
 // Host-visible state blob for single-shot execution from a preset state.
@@ -159,6 +164,8 @@ constexpr uint32_t kMaxForcedFaults = 64;
 struct KfTables {
     const double* w;   // [n]
     const double* dp;  // [(n + 1) x (k + 1)]
+    // [(n + 2) x (k + 1)]: site i is hit with j faults left if the top 53 bits of its draw are below this
+    const uint64_t* below;
     uint32_t n;        // sites + readout entries
     uint32_t n_q;      // quantum noise sites (indices below n_q)
     uint32_t k;

@@ -315,11 +315,14 @@ struct clifft_svm_program {
     int64_t kf_k = -1;
     // launch planning
     LaunchShape base_shape;
-    // shared-state executor: (bits that may part the shots, rank) of every
-    // writing pass (empty: the program has no plan), and its code length
-    std::vector<std::pair<uint32_t, uint32_t>> tree_sizes;
-    uint32_t tree_n = 0;
+    // shared-state executor: whether the program has a plan, its code length
+    // and response words, and (bits that may part the shots, rank) of every
+    // writing pass
+    bool tree = false;
+    bool tree_force = false;    // ... for forced records too
     bool tree_choices = false;  // frame bits, not outcomes alone, part the shots
+    uint32_t tree_n = 0, tree_words = 0;
+    std::vector<std::pair<uint32_t, uint32_t>> tree_sizes;
     // staging for host outputs (grown on demand)
     void* out_dev = nullptr;
     size_t out_dev_bytes = 0;
@@ -763,43 +766,6 @@ void lane_fuse_meas_pauli(clifft_instruction* code, uint64_t n) {
     }
 }
 
-// Drop the instructions that packed runs, fans and measurement + reset pairs
-// cover (a DETECTOR run reads its covered instructions and keeps them), so
-// the walk reads consecutive memory.
-std::vector<clifft_instruction> compact_covered(const std::vector<clifft_instruction>& code) {
-    std::vector<clifft_instruction> out;
-    for (size_t i = 0; i < code.size(); ++i) {
-        out.push_back(code[i]);
-        const uint32_t op = code[i].opcode;
-        if (op != kLaneFrameRun && op != kLaneFrameFan && op != kLaneMeasPauli) continue;
-        i += out.back().axis_2;
-        out.back().axis_2 = 0;
-    }
-    return out;
-}
-
-uint8_t forced_opcode(uint8_t op) {
-    return op >= CLIFFT_OP_MEAS_DORMANT_STATIC && op <= CLIFFT_OP_SWAP_MEAS_INTERFERE
-               ? (uint8_t)(op + (CLIFFT_OP_MEAS_DORMANT_STATIC_FORCED - CLIFFT_OP_MEAS_DORMANT_STATIC))
-               : op;
-}
-
-// The shared-state executor's bytecode for the sampled and the forced walk.
-void tree_bytecode(const clifft_program_view* v, const TreePlan& plan, std::vector<clifft_instruction>& sample,
-                   std::vector<clifft_instruction>& forced) {
-    std::vector<clifft_instruction> code = plan.code;
-    const std::vector<uint8_t> idle = frame_prune_enabled() ? plan.idle : std::vector<uint8_t>(code.size(), 0);
-    lane_inline_operands(v, code.data(), code.size(), idle);
-    forced = code;
-    for (clifft_instruction& in : forced) {
-        if (in.opcode == kTreeMeas) in.reserved |= 2u;
-        in.opcode = forced_opcode(in.opcode);
-    }
-    lane_fuse_meas_pauli(code.data(), code.size());
-    sample = compact_covered(code);
-    forced = compact_covered(forced);
-}
-
 // CLIFFT_SHARED_STATE: 0 turns the shared-state executor off, 2 uses it
 // wherever it can run; unset, tree_shape decides from its cost estimate.
 int shared_state_mode() {
@@ -1143,31 +1109,33 @@ TreeWork tree_work(const clifft_svm_program* p, uint32_t chunk) {
 }
 
 // A team shape of the shared-state executor for `chunk` shots on `threads`
-// threads; false where its tables do not fit.
-bool tree_team(const clifft_svm_program* p, uint32_t threads, uint32_t chunk, LaunchShape& L) {
+// threads, each with room for `faults` forced faults; false where its tables
+// do not fit.
+bool tree_team(const clifft_svm_program* p, uint32_t threads, uint32_t chunk, uint32_t faults, LaunchShape& L) {
     const TreeWork w = tree_work(p, chunk);
     if (w.elems > (1ull << 31)) return false;
-    const uint32_t rec_words = lane_words(p->total_slots) + lane_words(p->num_det) + lane_words(p->num_obs);
     L = LaunchShape();
     L.tree = true;
     L.tree_chunk = chunk;
     L.tree_elems = (uint32_t)w.elems;
     L.block = threads;
-    L.lane_narrow = p->frame32;
-    L.lds_bytes = tree_team_lds(threads, chunk, rec_words);
+    L.lds_bytes = tree_team_lds(threads, chunk, p->tree_words + 5 * faults);
     L.global_amps = w.elems > kTreeLdsElems;
     if (!L.global_amps) L.lds_bytes += 32u * (size_t)w.elems;
     return L.lds_bytes <= kTreeMaxDynLds;
 }
 
-// Estimated time (us) of one chunk on a team of shape L, alone on its CU:
-// the walk, the passes' fixed part, and the entries visited at what the
-// team's wavefronts reach (fitted to a sweep of team sizes and chunks at
-// peak 6 to 16 on one MI355X).
-double tree_team_us(const clifft_svm_program* p, const LaunchShape& L) {
+// Estimated time (us) of one chunk on a team of shape L that shares its CU
+// with `teams` - 1 others: the walk, the passes' fixed part, and the entries
+// visited at what the wavefronts in flight reach (fitted to a sweep of team
+// sizes and chunks at peak 0 to 16 on one MI355X).
+double tree_team_us(const clifft_svm_program* p, const LaunchShape& L, double teams) {
+    const double waves = L.block / 64.0, per_simd = teams * waves / 4.0;
+    const double passes = p->tree_sizes.size();
+    const double walk = 5.0 + 0.35 * p->tree_n + (2.0 + 0.3 * std::log2(waves)) * passes;
     const double visited = (double)tree_work(p, L.tree_chunk).visited;
-    const double entry = (L.global_amps ? 0.32e-3 : 0.25e-3) * std::max(1.0, 512.0 / L.block);
-    return 15.0 + 0.2 * p->tree_n + 2.2 * p->tree_sizes.size() + 2.0e-3 * L.block + visited * entry;
+    const double entry = (L.global_amps ? 0.32e-3 : 0.25e-3) * std::max(512.0 / L.block, teams);
+    return walk * (1.0 + 0.18 * std::max(0.0, per_simd - 1.0)) + visited * entry;
 }
 // ... and of `shots` shots.
 double tree_cost(const clifft_svm_program* p, const LaunchShape& L, uint64_t shots) {
@@ -1179,39 +1147,37 @@ double tree_cost(const clifft_svm_program* p, const LaunchShape& L, uint64_t sho
     // all teams together move 32 B an entry beyond the caches
     const double bytes = L.global_amps ? std::min(teams, cus * per_cu) * 32.0 * (double)L.tree_elems : 0.0;
     const double memory = bytes > 64e6 ? teams * visited * 32.0 / 4.0e6 : 0.0;
-    return std::max(rounds * tree_team_us(p, L) * (1.0 + 0.25 * (std::min(per_cu, std::ceil(teams / cus)) - 1.0)), memory);
+    return std::max(rounds * tree_team_us(p, L, std::min(per_cu, std::ceil(teams / cus))), memory);
 }
 
 // Whether `shots` shots of a program are better off sharing their states.
-// Measured on one MI355X, per-shot executors against this one (24-qubit
-// Clifford+T, and random programs with noise and frame-dependent phases,
-// where almost no shots share): from peak 11 on it is 1.3 to 48 times
-// faster from 100 shots up; at peak 7 to 10 it wins 2.6 to 66 times from
-// 10000 shots, 1.1 to 1.3 times at 100 to 1000 shots where only outcomes
-// part the shots, and loses up to a quarter at 100 to 1000 shots of a random
-// program; lanes keep peak 6 and below (1.45 and 2.9 times slower at peak 5
-// and 6 with 100000 shots, but faster up to 10000).
+// Measured on one MI355X, per-shot executors against this one (100 to 300000
+// shots): surface-code memories 1.3 to 3 times faster to 49 qubits (25 rounds
+// of distance 3 with 300000 shots: the same), 14 to 470 times beyond 64;
+// 24-qubit Clifford+T at peak 8 to 14 2 to 300 times; random programs, whose
+// frames part almost every shot, 1.1 to 7 times from peak 8 on.  Below that a
+// program with a pass for every few instructions can lose (random, 300
+// instructions, 60 passes: 0.72 to 0.94 times at peak 1 to 7), so it has to
+// beat the lanes' walk, 0.48 us an instruction there.
 bool tree_better(const clifft_svm_program* p, uint64_t shots) {
-    if (p->tree_sizes.empty() || shared_state_mode() == 0) return false;
-    if (shared_state_mode() == 2) return true;
-    const uint32_t k = p->peak_rank;
-    if (k >= 11) return true;
-    if (k >= 7) return shots >= 4096 || (!p->tree_choices && shots >= 100);
-    return k >= 5 && !p->tree_choices && shots >= 65536;
+    if (!p->tree || shared_state_mode() == 0) return false;
+    if (shared_state_mode() == 2 || p->words > 1 || p->peak_rank >= 8) return true;
+    if (p->peak_rank == 7 && shots >= 4096) return true;
+    return 5.0 + 0.35 * p->tree_n + 2.0 * p->tree_sizes.size() <= 0.48 * (double)p->host_bc.size();
 }
 
 // The shared-state shape for a launch of `shots` shots: the team size and
 // the shots per team of the lowest estimate.  False: the program has no
 // plan, or the per-shot executors are faster.
-bool tree_shape(const clifft_svm_program* p, uint64_t shots, LaunchShape& best) {
+bool tree_shape(const clifft_svm_program* p, uint64_t shots, uint32_t faults, LaunchShape& best) {
     if (!tree_better(p, shots)) return false;
     double cost = 0.0;
     bool found = false;
-    for (uint32_t threads : {256u, 512u, 1024u})
+    for (uint32_t threads : {64u, 128u, 256u, 512u, 1024u})
         for (uint32_t chunk = threads; chunk >= 1; chunk /= 2) {
             if (chunk > 2 * shots && chunk > 1) continue;
             LaunchShape L;
-            if (!tree_team(p, threads, chunk, L)) continue;
+            if (!tree_team(p, threads, chunk, faults, L)) continue;
             const double c = tree_cost(p, L, shots);
             if (!found || c < cost) {
                 best = L;
@@ -1223,24 +1189,30 @@ bool tree_shape(const clifft_svm_program* p, uint64_t shots, LaunchShape& best) 
 }
 
 // The shape in a batch, where other programs fill the device: the least
-// time of a compute unit, each team taking its part of one.
+// time of a compute unit, each team taking its part of one.  Two team sizes,
+// the larger alone for states in memory: each more is one more launch with
+// an end of its own (512 Clifford+T programs of peak 4 to 16, 1000 shots
+// each, all of 64 to 1024 threads: 766 us, 256 and 1024: 572, 1024 alone:
+// 552, 512 alone: 735); smaller ones where the records leave no room.
 bool tree_batch_shape(const clifft_svm_program* p, uint64_t shots, LaunchShape& best) {
-    if (p->peak_rank < 7 || !tree_better(p, std::max<uint64_t>(shots, 4096))) return false;
+    if (!tree_better(p, std::max<uint64_t>(shots, 4096))) return false;
     double cost = 0.0;
     bool found = false;
-    for (uint32_t threads : {256u, 512u, 1024u})
+    for (uint32_t threads : {1024u, 256u, 64u}) {
+        if (found && threads == 64u) break;
         for (uint32_t chunk = threads; chunk >= 64; chunk /= 2) {
             if (chunk > 64 && chunk >= 2 * shots) continue;
             LaunchShape L;
-            if (!tree_team(p, threads, chunk, L)) continue;
+            if (!tree_team(p, threads, chunk, 0, L) || (found && L.global_amps && threads < best.block)) continue;
             const double part = std::max((double)threads / 1024.0, (double)L.lds_bytes / (double)kLdsBytes);
-            const double c = std::ceil((double)shots / chunk) * part * tree_team_us(p, L);
+            const double c = std::ceil((double)shots / chunk) * part * tree_team_us(p, L, 1.0 / part);
             if (!found || c < cost) {
                 best = L;
                 cost = c;
                 found = true;
             }
         }
+    }
     return found;
 }
 
@@ -1435,19 +1407,22 @@ int clifft_svm_program_create(const clifft_program_view* view, clifft_svm_progra
     size_t o_eo = add(view->expected_observables, view->num_expected_observables);
     // the shared-state executor's tables
     TreePlan plan;
-    std::vector<clifft_instruction> tree_code, tree_forced;
     if (!has_forced && shared_state_mode() != 0) {
-        TreePlanner planner(view, khist);
-        plan = planner.run();
-        if (plan.ok && !plan.passes.empty()) {
-            tree_bytecode(view, plan, tree_code, tree_forced);
-            p->tree_sizes = plan.sizes;
-            p->tree_n = (uint32_t)tree_code.size();
-            for (const clifft_instruction& in : tree_code) p->tree_choices |= in.opcode == kTreeChoice;
-        }
+        plan = TreePlanner(view, khist).run();
+        p->tree = plan.ok;
+        p->tree_force = plan.can_force;
+        p->tree_choices = plan.choices;
+        p->tree_n = (uint32_t)plan.code.size();
+        p->tree_words = plan.words;
+        p->tree_sizes = plan.sizes;
     }
-    size_t o_trb = add(tree_code.data(), tree_code.size() * sizeof(clifft_instruction));
-    size_t o_trf = add(tree_forced.data(), tree_forced.size() * sizeof(clifft_instruction));
+    size_t o_trb = add(plan.code.data(), plan.code.size() * sizeof(clifft_instruction));
+    size_t o_trf = add(plan.forced.data(), plan.forced.size() * sizeof(clifft_instruction));
+    size_t o_lpd = add(plan.dense.data(), plan.dense.size() * 4);
+    size_t o_lpr = add(plan.rows.data(), plan.rows.size() * 4);
+    size_t o_lps = add(plan.sites.data(), plan.sites.size() * sizeof(TreeSite));
+    size_t o_lpc = add(plan.chans.data(), plan.chans.size() * sizeof(TreeChan));
+    size_t o_lpe = add(plan.chan_rows.data(), plan.chan_rows.size() * 4);
     plan.passes.resize(plan.passes.size() + 1);  // the executor reads one ahead
     size_t o_trp = add(plan.passes.data(), plan.passes.size() * sizeof(TreePass));
     size_t o_trh = add(plan.phases.data(), plan.phases.size() * sizeof(TreePhase));
@@ -1546,14 +1521,20 @@ int clifft_svm_program_create(const clifft_program_view* view, clifft_svm_progra
     d.tree_bc = reinterpret_cast<const clifft_instruction*>(base + o_trb);
     d.tree_passes = reinterpret_cast<const TreePass*>(base + o_trp);
     d.tree_phases = reinterpret_cast<const TreePhase*>(base + o_trh);
-    d.tree_n = (uint32_t)tree_code.size();
+    d.lp_dense = reinterpret_cast<const uint32_t*>(base + o_lpd);
+    d.lp_rows = reinterpret_cast<const uint32_t*>(base + o_lpr);
+    d.lp_sites = reinterpret_cast<const TreeSite*>(base + o_lps);
+    d.lp_chans = reinterpret_cast<const TreeChan*>(base + o_lpc);
+    d.lp_chan_rows = reinterpret_cast<const uint32_t*>(base + o_lpe);
+    d.tree_n = plan.ok ? (uint32_t)plan.code.size() - 1 : 0;
+    d.lp_words = plan.words;
     {
         DevProgram both[2] = {d, d};
         both[1].bc = p->forced_bc;
         both[1].lane_bc = reinterpret_cast<const clifft_instruction*>(base + o_lfbc);
         both[1].team_bc = reinterpret_cast<const clifft_instruction*>(base + o_tfbc);
         both[1].tree_bc = reinterpret_cast<const clifft_instruction*>(base + o_trf);
-        both[1].tree_n = (uint32_t)tree_forced.size();
+        both[1].tree_n = plan.ok ? (uint32_t)plan.forced.size() - 1 : 0;
         e = hipMemcpy(base + o_dp, both, sizeof(both), hipMemcpyHostToDevice);
         if (e != hipSuccess) {
             std::string msg = std::string("program upload: ") + hipGetErrorString(e);
@@ -1617,7 +1598,7 @@ static int run_shots(clifft_svm_program* p, uint64_t shots, uint64_t seed, uint3
         LaunchShape L;
         void* gs = nullptr;
         int rc;
-        const bool tree = !kfault && tree_shape(p, n, L);
+        const bool tree = (mode != MODE_FORCED || p->tree_force) && tree_shape(p, n, kfault ? (uint32_t)p->kf_k : 0u, L);
         if (tree) {
             rc = tree_finalize(L, n, st, &gs);
         } else {
@@ -1669,7 +1650,8 @@ static int run_shots(clifft_svm_program* p, uint64_t shots, uint64_t seed, uint3
                 A.forced_records = fdev;
             }
         }
-        HIP_TRY(launch_with_args(p, L, mode == MODE_FORCED ? p->dp_forced_dev : p->dp_dev, A, st));
+        const DevProgram* dp = mode == MODE_FORCED ? p->dp_forced_dev : p->dp_dev;
+        HIP_TRY(tree ? launch_tree(L, dp, A, st) : launch_with_args(p, L, dp, A, st));
         if (!dev_out) {
             if (out && out->measurements && n * bm)
                 HIP_TRY(hipMemcpyAsync(out->measurements + base * bm, A.out_meas, n * bm, hipMemcpyDeviceToHost, st));
@@ -1894,7 +1876,8 @@ static int kfault_tables(clifft_svm_program* p, uint32_t k, hipStream_t st, cons
     for (uint32_t i = 1; i < n; ++i)
         if (probs[i] != probs[0]) uniform = false;
     const size_t o_w = align_up(sizeof(KfTables), 256), o_dp = o_w + align_up((size_t)(n + 1) * 8, 256);
-    const size_t total = o_dp + (size_t)(n + 1) * (k + 1) * 8;
+    const size_t o_below = o_dp + align_up((size_t)(n + 1) * (k + 1) * 8, 256);
+    const size_t total = o_below + (size_t)(n + 2) * (k + 1) * 8;
     if ((int64_t)k != p->kf_k || total > p->kf_dev_bytes) {
         if (total > p->kf_dev_bytes) {
             if (p->kf_dev) {
@@ -1909,6 +1892,7 @@ static int kfault_tables(clifft_svm_program* p, uint32_t k, hipStream_t st, cons
         std::vector<uint8_t> staging(total, 0);
         auto* w = reinterpret_cast<double*>(staging.data() + o_w);
         auto* dp = reinterpret_cast<double*>(staging.data() + o_dp);
+        auto* below = reinterpret_cast<uint64_t*>(staging.data() + o_below);
         if (!uniform) {
             double sum = 0.0;  // odds ratios rescaled to mean 1
             for (uint32_t i = 0; i < n; ++i) {
@@ -1926,11 +1910,20 @@ static int kfault_tables(clifft_svm_program* p, uint32_t k, hipStream_t st, cons
                     dp[(size_t)i * stride + j] =
                         dp[(size_t)(i + 1) * stride + j] + w[i] * dp[(size_t)(i + 1) * stride + j - 1];
             }
+            for (uint32_t i = 0; i < n; ++i)
+                for (uint32_t j = 1; j <= k; ++j) {
+                    const double denom = dp[(size_t)i * stride + j];
+                    const double hit =
+                        j == n - i ? 1.0 : denom > 0.0 ? (w[i] * dp[(size_t)(i + 1) * stride + j - 1]) / denom : 0.0;
+                    // x 2^-53 < hit for the draw's top 53 bits x (scaling by 2^53 is exact)
+                    below[(size_t)i * stride + j] = (uint64_t)std::ceil(std::min(hit, 1.0) * 0x1.0p53);
+                }
         }
         auto* base = static_cast<uint8_t*>(p->kf_dev);
         KfTables T{};
         T.w = reinterpret_cast<const double*>(base + o_w);
         T.dp = reinterpret_cast<const double*>(base + o_dp);
+        T.below = reinterpret_cast<const uint64_t*>(base + o_below);
         T.n = n;
         T.n_q = p->num_sites;
         T.k = k;
@@ -2359,7 +2352,7 @@ int batch_group(clifft_svm_batch* b, uint64_t cap) {
             group_of[i] = (uint32_t)gi;
             const uint64_t n = std::min<uint64_t>(b->shots[i], cap);
             const uint32_t step = g.L.tree ? shape[i].tree_chunk : chunk;
-            const double c = g.L.tree ? tree_team_us(b->progs[i], shape[i]) / step : shot_cost(b->progs[i], g.L);
+            const double c = g.L.tree ? tree_team_us(b->progs[i], shape[i], 1.0) / step : shot_cost(b->progs[i], g.L);
             if (g.L.tree) {
                 b->args[i].tree_chunk = shape[i].tree_chunk;
                 b->args[i].amp_elems = shape[i].tree_elems;
@@ -2408,7 +2401,7 @@ int batch_audit(const clifft_svm_batch* b) {
                 LaunchShape one;
                 if (it.shot_hi - it.shot_lo > A.tree_chunk || A.tree_chunk > L.block || A.tree_chunk == 0)
                     return fail(CLIFFT_E_INVALID, where + "item over the team's shots");
-                if (!tree_team(p, L.block, A.tree_chunk, one) || one.lds_bytes > L.lds_bytes || one.global_amps != L.global_amps)
+                if (!tree_team(p, L.block, A.tree_chunk, 0, one) || one.lds_bytes > L.lds_bytes || one.global_amps != L.global_amps)
                     return fail(CLIFFT_E_INVALID, where + "team tables exceed the launch's LDS");
                 if (A.amp_elems != one.tree_elems || one.tree_elems > g.amp_elems)
                     return fail(CLIFFT_E_INVALID, where + "amplitude buffers exceed the team's");

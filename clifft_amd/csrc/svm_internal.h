@@ -24,7 +24,7 @@ struct LaunchShape {
     bool lane_narrow = false;  // lane kernel with 32-bit frame words (at most 32 qubits)
     uint32_t amp_slices = 1;   // global-amplitude slices per team (2: fused permutation/phase runs, 3: and candidate folds)
     uint32_t rec_stride = 0;   // LDS bytes of one wavefront's record block (team tiers)
-    bool tree = false;         // shared-state executor (svm_tree.h); global_amps, lane_narrow, block and lds_bytes apply
+    bool tree = false;         // shared-state executor (svm_tree.h); global_amps, block and lds_bytes apply
     uint32_t tree_chunk = 0;   // its shots per team
     uint32_t tree_elems = 0;   // entries of each of a team's two amplitude buffers
     uint32_t block = 256;      // threads per workgroup
@@ -63,7 +63,9 @@ constexpr size_t kTreeMaxDynLds = 158 * 1024;
 // Shared-state executor (svm_tree.hip): a shape's kernel, plain or batched,
 // and the LDS of a team apart from LDS amplitudes.
 const void* tree_kernel_fn(const LaunchShape& L, bool batch);
-uint32_t tree_team_lds(uint32_t threads, uint32_t chunk, uint32_t rec_words);
+uint32_t tree_team_lds(uint32_t threads, uint32_t chunk, uint32_t lane_words);
+// The launch arguments travel with the kernel's.
+hipError_t launch_tree(const LaunchShape& L, const DevProgram* P, const ShotArgs& A, hipStream_t st);
 
 // Adjoint-gradient executor (P and A are device memory).
 hipError_t adjoint_occupancy(bool global_amps, uint32_t block, size_t lds_bytes, int* blocks_per_cu);

@@ -521,13 +521,7 @@ hipError_t shot_occupancy(const LaunchShape& L, int* blocks_per_cu) {
     return hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, fn, (int)L.block, L.lds_bytes);
 }
 
-// (a tree shape's dynamic-LDS attribute is set by shot_occupancy, which
-// sizes its grid)
 hipError_t launch_shots(const LaunchShape& L, const DevProgram* P, const ShotArgs* A, hipStream_t st) {
-    if (L.tree) {
-        void* args[] = {&P, &A};
-        return hipLaunchKernel(tree_kernel_fn(L, false), dim3(L.grid), dim3(L.block), args, L.lds_bytes, st);
-    }
     if (L.lane) return launch_lane(L, P, A, st);
     switch (L.nw) {
         case 1: return launch_fk<FRAME_W1>(L, P, A, st);

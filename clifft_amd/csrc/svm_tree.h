@@ -2,9 +2,10 @@
 // workgroup, one copy of the amplitudes per group of shots that agree on
 // everything the amplitudes depend on.
 //
-// One shot per thread holds the Pauli frame, the xoshiro256++ state and its
-// record bits exactly as the lane interpreter does (svm_lane.h); every
-// thread walks the same bytecode.  Shots whose random
+// One shot per thread holds its xoshiro256++ state and its response
+// (svm_tree_args.h): the record bits and the few other bits the walk reads,
+// to which every random bit that comes up 1 adds a precomputed row.  There
+// is no Pauli frame, and no opcode that only moves one.  Shots whose random
 // outcomes (and frame bits at phase opcodes) agreed so far have the same
 // amplitudes, bit for bit, so the team keeps one state per such group
 // ("node") and sweeps all nodes as one flat array: entry i of node n at
@@ -22,12 +23,18 @@
 // 16 moves about 12 x 2^16 entries instead of 1000 x 2 x 2^16, and every
 // opcode is dispatched once per 64 shots.
 //
-// Measured on one MI355X (per launch, before -> after; before: the per-shot
-// tiers): 24-qubit Clifford+T, peak 10 x 20000 shots 2307 -> 82 us, peak 13
-// x 20000 2250 -> 147 us, peak 16 x 2000 1808 -> 291 us; 34 qubits, peak 25
-// x 64 shots 750 -> 67 ms; 512 programs x 1000 shots 54.3 -> 1.4 ms.  What
-// bounds it: up to peak 12 the bytecode walk (about 0.35 us a dispatch), from
-// peak 14 the passes (16 instructions and 32 bytes an entry).
+// Measured on one MI355X (per call, before -> after; before: the per-shot
+// tiers): 24-qubit Clifford+T, peak 10 x 20000 shots 2304 -> 58 us, peak 16 x
+// 2000 1805 -> 276 us; 34 qubits, peak 25 x 64 shots 752 -> 67 ms; 512
+// programs x 1000 shots 54.4 -> 0.67 ms; surface-code memories, distance 3 x
+// 10^6 shots 162 -> 128 us, distance 7 (97 qubits) x 20000 7770 -> 92 us,
+// distance 5 with 4 forced faults x 20000 3940 -> 530 us (360 of them copies
+// to the host).  With a frame per shot and every opcode walked (the same
+// executor before the response) peak 10 took 82 us, its walk 35 of them.
+// What bounds it: memories, the dependent loads of a noise event (about 1.3
+// us for the slowest of 64 shots) and the draws; up to peak 12 the passes'
+// fixed part, about 2 us a measurement; from peak 14 their entries (16
+// instructions and 32 bytes each).
 //
 // The array work itself is planned on the host (svm_tree_plan.h): each pass
 // gathers through a linear map over GF(2), so a lane's source index is the
@@ -35,7 +42,7 @@
 // changes by one column between its entries.
 #pragma once
 
-#include "svm_lane.h"
+#include "svm_device.h"
 #include "svm_tree_args.h"
 #include "svm_sweeps.h"
 
@@ -45,25 +52,39 @@ struct TreeStage {  // the running pass's expansion products
     double tab[1u << kTreeMaxExpand][2];
 };
 constexpr uint32_t kTreeParts = 128;  // partial sums of a pass with several per node
-constexpr uint32_t kTreeWindow = 256;  // bytecode instructions held in LDS
 
 // LDS of one team of `threads` threads and at most `chunk` shots: per-wave
-// record columns, two node tables (source node, choice word), per-node
-// sums, partial sums, two key bitmaps (and the rescale flag), the stage, the
-// bytecode window.
+// response columns (64 x 4 B a word; with k-fault sampling also the fault
+// lists), two node tables (source node, choice word), per-node
+// sums, partial sums, two key bitmaps (and the rescale flag), the stage.
 __host__ __device__ inline uint32_t tree_flag_words(uint32_t chunk) { return (chunk + 1u) / 2u + 2u; }
-__host__ __device__ inline uint32_t tree_lds_bytes(uint32_t threads, uint32_t chunk, uint32_t rec_words) {
-    uint32_t b = (threads >> 6) * rec_words * 256u;
+__host__ __device__ inline uint32_t tree_lds_bytes(uint32_t threads, uint32_t chunk, uint32_t lane_words_) {
+    uint32_t b = (threads >> 6) * lane_words_ * 256u;
     b += (16u * chunk + 15u) / 16u * 16u;  // 4 x u32 tables
     b += 16u * chunk + 16u * kTreeParts;
     b += (8u * tree_flag_words(chunk) + 15u) / 16u * 16u;
-    return b + (uint32_t)sizeof(TreeStage) + 32u * kTreeWindow;
+    return b + (uint32_t)sizeof(TreeStage);
 }
 
-template <class FW, class AmpT>
-struct TreeInterp : LaneInterp<FW> {
-    typedef LaneInterp<FW> L;
-    typedef __attribute__((address_space(3))) uint32_t lds_u32;
+typedef __attribute__((address_space(3))) uint32_t tree_lds_u32;
+typedef uint32_t TreeQuad __attribute__((ext_vector_type(4)));  // a group of a row
+
+// orders one lane's LDS accesses with another's of its wavefront
+CSVM_INLINE void tree_wave_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// (tables that lanes index for themselves)
+typedef const __attribute__((address_space(1))) TreeQuad* glb_quad;
+typedef const __attribute__((address_space(1))) double* glb_f64;
+typedef const __attribute__((address_space(1))) uint32_t* glb_u32;
+typedef const __attribute__((address_space(1))) uint64_t* glb_u64;
+
+template <class AmpT>
+struct TreeInterp {
+    typedef tree_lds_u32 lds_u32;
     typedef __attribute__((address_space(3))) TreeStage lds_stage;
     typedef __attribute__((address_space(3))) uint64_t lds_u64;
     static constexpr uint32_t G = 4;  // pairs in flight per lane: eight 16-byte loads
@@ -76,13 +97,252 @@ struct TreeInterp : LaneInterp<FW> {
     uint32_t scale_word;    // index of the rescale flag behind the bitmaps' words
     lds_f64 *psum, *part;
     lds_stage* stage;
-    lds_u64* window;        // bytecode instructions [.., ..) of the walk
     uint32_t N;             // nodes
     // the next pass's words (svm_tree_args.h), loaded while the one before
     // it runs: lane b of `wa` the header, of the halves of `wa`, `wb`, `wc`
     // the columns
     uint32_t next, wa, wb, wc;
-    uint32_t node, live;    // this thread's shot
+    // this thread's shot
+    uint32_t node, live;
+    Rng rng;
+    uint32_t next_noise, discarded, reachable, dust;
+    double logp;
+    const uint8_t* forced;  // its forced record row (MODE_FORCED)
+    lds_u32* R;             // its response: word w at R[w << 6]
+    // MODE_KFAULT: its forced noise sites, then readout entries, each ascending
+    lds_u32* kf;
+    uint32_t kf_nn, kf_pos, kf_n, kf_rpos;  // kf null: gap sampling
+
+    // -------------------------------------------------------------- response
+    CSVM_INLINE static void add_word(lds_u32* p, uint32_t x) {
+        (void)__hip_atomic_fetch_xor(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);  // one LDS instruction
+    }
+    // Add a row of `units` units where `on`: a few entries, against some dozen
+    // words of a response.
+    CSVM_INLINE void add_entries(TreeQuad e) {
+        if (e.y) add_word(R + e.x, e.y);
+        if (e.w) add_word(R + e.z, e.w);
+    }
+    CSVM_INLINE void add_row(cptr<TreeQuad> row, uint32_t units, bool on) {
+        const TreeQuad e0 = row[0], e1 = row[1];
+        if (!on) return;
+        add_entries(e0);
+        add_entries(e1);
+        for (uint32_t g = 2; g < 2u * units; ++g) add_entries(row[g]);
+    }
+    // The same for `count` rows in turn, bit j's being fires().  A row's first
+    // unit arrives while the one before it is added (its load is issued after
+    // that one's wait: scalar loads are only waited for all together), and
+    // entries are masked, not branched over: at a wavefront or two per SIMD a
+    // taken branch costs as much as several instructions.
+    template <class F>
+    CSVM_INLINE void add_rows(cptr<TreeQuad> row, uint32_t units, uint32_t count, F fires) {
+        TreeQuad e0 = row[0], e1 = row[1];
+        for (uint32_t j = 0; j < count; ++j) {
+            cptr<TreeQuad> next = row + (j + 1u < count ? 2u * units : 0u);
+            asm volatile("" ::"s"(e0.x), "s"(e1.x));
+            const TreeQuad n0 = next[0], n1 = next[1];
+            const uint32_t m = fires() ? 0xFFFFFFFFu : 0u;
+            add_word(R + e0.x, e0.y & m);
+            if (e0.w) {
+                add_word(R + e0.z, e0.w & m);
+                add_word(R + e1.x, e1.y & m);
+                add_word(R + e1.z, e1.w & m);
+            }
+            for (uint32_t g = 2; g < 2u * units; ++g) {
+                const TreeQuad e = row[g];
+                if (!e.y) break;
+                add_word(R + e.x, e.y & m);
+                add_word(R + e.z, e.w & m);
+            }
+            row = next;
+            e0 = n0;
+            e1 = n1;
+        }
+    }
+    CSVM_INLINE static cptr<TreeQuad> row_at(cptr<DevProgram> P, uint32_t unit) {
+        return (cptr<TreeQuad>)cp(P->lp_rows) + 2 * (size_t)unit;
+    }
+    CSVM_INLINE uint32_t bits(uint32_t at, uint32_t n) const { return (R[(at >> 5) << 6] >> (at & 31u)) & ((1u << n) - 1u); }
+
+    // ----------------------------------------------------------------- noise
+    // Gap sampler (svm.h:229-243)
+    CSVM_INLINE void draw_next_noise(cptr<DevProgram> P, double cur) {
+        const uint32_t n = P->num_sites;
+        if (n == 0 || next_noise >= n) {
+            next_noise = kNoNoise;
+            return;
+        }
+        const double gap = -log(1.0 - rng_double(rng));
+        next_noise = hazard_upper_bound((glb_f64)P->hazards, n, (glb_u32)P->hz_guide, P->hz_buckets, P->hz_scale, cur + gap);
+    }
+    // The first channel whose running sum exceeds r (pick_channel's rule and
+    // first try, on TreeChan records): its row's first entry and their number.
+    CSVM_INLINE static double chan_cum(TreeQuad c) { return __hiloint2double((int)c.y, (int)c.x); }
+    CSVM_INLINE void pick(glb_quad ch, uint32_t n, double u, uint32_t& first, uint32_t& count) {
+        const uint32_t q = (uint32_t)(u * (double)n), g = q < n ? q : n - 1u;
+        const TreeQuad last = ch[n - 1u], before = ch[g > 0 ? g - 1u : 0u];
+        TreeQuad c = ch[g];
+        const double r = u * chan_cum(last);
+        count = 0;
+        if (!((g == 0 || chan_cum(before) <= r) && r < chan_cum(c))) {
+            uint32_t lo = 0, hi = n;
+            while (lo < hi) {
+                const uint32_t mid = lo + (hi - lo) / 2;
+                if (r < chan_cum(ch[mid]))
+                    hi = mid;
+                else
+                    lo = mid + 1;
+            }
+            if (lo == n) return;
+            c = ch[lo];
+        }
+        first = c.z;
+        count = c.w;
+    }
+    // Fire the site next_noise and find the next one (svm_kernels.inl:1886-1920).
+    // A chain of dependent loads bounds it, so the tables are laid out for
+    // few of them, and the row's first entries are under way while the next
+    // site is looked up.
+    CSVM_INLINE void noise(cptr<DevProgram> P) {
+        const TreeQuad t = ((glb_quad)P->lp_sites)[next_noise];
+        const double u = rng_double(rng);
+        uint32_t first = 0, count = 0;
+        if (t.y) pick((glb_quad)P->lp_chans + t.x, t.y, u, first, count);
+        glb_quad row = (glb_quad)P->lp_chan_rows + (first >> 1);
+        TreeQuad e0{0, 0, 0, 0}, e1{0, 0, 0, 0};
+        if (count > 0) e0 = row[0];
+        if (count > 2) e1 = row[1];
+        if (kf) {  // svm.h:218-225
+            next_noise = kf_pos < kf_nn ? kf[kf_pos << 6] : kNoNoise;
+            kf_pos++;
+        } else {
+            next_noise++;
+            draw_next_noise(P, chan_cum(TreeQuad{t.z, t.w, 0, 0}));
+        }
+        for (uint32_t i = 0;;) {  // (adding zero does nothing)
+            add_word(R + e0.x, e0.y);
+            add_word(R + e0.z, e0.w);
+            add_word(R + e1.x, e1.y);
+            add_word(R + e1.z, e1.w);
+            i += 4;
+            if (i >= count) break;
+            e0 = row[i >> 1];
+            e1 = TreeQuad{0, 0, 0, 0};
+            if (i + 2u < count) e1 = row[(i >> 1) + 1u];
+        }
+    }
+
+    // Choose this shot's (`on`) fault set (svm.cc:435-520; with unequal
+    // probabilities about 45 instructions a site, 85 us for 670 sites, where
+    // looking the limits up as they are needed took 134) into its list -- room
+    // for 5 k words a lane: picks, then the sparse Fisher-Yates map of at
+    // most 2 k positions -- and arm the noise cursor.
+    CSVM_INLINE void kfault_prepare(cptr<KfTables> T, lds_u32* list, bool on) {
+        const uint32_t n = T->n, k = T->k, n_q = T->n_q;
+        uint32_t m = 0;
+        if (k == 0) {
+        } else if (T->uniform) {
+            lds_u32 *keys = list + (k << 6), *vals = list + (3u * k << 6);
+            uint32_t nk = 0;
+            auto find = [&](uint32_t pos) -> uint32_t {  // index in the map, or nk
+                uint32_t e = 0;
+                while (e < nk && keys[e << 6] != pos) ++e;
+                return e;
+            };
+            for (uint32_t j = 0; j < k; ++j) {
+                const uint32_t pick = j + (uint32_t)(rng_double(rng) * (double)(n - j));
+                if (pick == j) continue;  // swap with itself
+                const uint32_t nk0 = nk, ej = find(j), ep = find(pick);
+                const uint32_t vj = ej < nk0 ? vals[ej << 6] : j, vp = ep < nk0 ? vals[ep << 6] : pick;
+                const uint32_t sj = ej < nk0 ? ej : nk++, sp = ep < nk0 ? ep : nk++;
+                keys[sj << 6] = j;  // pool[j] <- pool[pick], pool[pick] <- pool[j]
+                vals[sj << 6] = vp;
+                keys[sp << 6] = pick;
+                vals[sp << 6] = vj;
+            }
+            for (uint32_t j = 0; j < k; ++j) {  // prefix pool[0..k), sorted as it is taken
+                const uint32_t e = find(j), v = e < nk ? vals[e << 6] : j;
+                uint32_t b = j;
+                for (; b > 0 && list[(b - 1u) << 6] > v; --b) list[b << 6] = list[(b - 1u) << 6];
+                list[b << 6] = v;
+            }
+            m = k;
+        } else {
+            // One draw a site until every fault is placed, against a limit that
+            // depends on the faults still to place.  The limits of some sites
+            // at a time are laid out for the wavefront in the rest of its
+            // lists' room (128 k of them).  No branch on a hit: the site is
+            // stored where the next hit's will overwrite it, and both limits
+            // that the next site can have are loaded under this one's draw.
+            const glb_u64 lim = (glb_u64)T->below;
+            lds_u64* held = (lds_u64*)(list - lane + (k << 6));
+            const uint32_t stride = k + 1u, per = (k << 7) / stride;
+            uint32_t needed = on ? k : 0u;
+            lds_u32* slot = list;
+            for (uint32_t base = 0; base < n && __any(needed != 0u); base += per - 1u) {
+                tree_wave_fence();
+                for (uint32_t e = lane; e < per * stride; e += 64u)
+                    if (base * stride + e < (n + 1u) * stride) held[e] = lim[base * stride + e];
+                tree_wave_fence();
+                const uint32_t end = n - base < per - 1u ? n : base + per - 1u;
+                const lds_u64* q = held + needed;
+                uint64_t p = *q;
+                for (uint32_t i = base; i < end && needed; ++i) {
+                    q += stride;
+                    const uint64_t miss = q[0], next = q[-1];
+                    const uint64_t x = rng_next(rng) >> 11;
+                    *slot = i;
+                    const bool hit = x < p;
+                    slot += hit ? 64 : 0;
+                    q -= hit ? 1 : 0;
+                    needed -= hit ? 1u : 0u;
+                    p = hit ? next : miss;
+                }
+            }
+            m = k - needed;
+            tree_wave_fence();
+        }
+        // picks are ascending: quantum sites first, then readout entries
+        uint32_t nn = 0;
+        while (nn < m && list[nn << 6] < n_q) ++nn;
+        for (uint32_t j = nn; j < m; ++j) list[j << 6] -= n_q;
+        kf = list;
+        kf_nn = nn;
+        kf_n = m;
+        kf_rpos = nn;
+        next_noise = on && nn ? list[0] : kNoNoise;
+        kf_pos = 1;
+    }
+
+    // svm_internal.h:65-79
+    CSVM_INLINE uint32_t sample_branch(double p0, double p1, double total) {
+        const double eps = kDustEpsilon * total;
+        if (p1 <= eps) {
+            if (p1 > 0.0) dust++;
+            return 0;
+        }
+        if (p0 <= eps) {
+            if (p0 > 0.0) dust++;
+            return 1;
+        }
+        const double r = rng_double(rng);
+        return (r * total < p0) ? 0u : 1u;
+    }
+    // svm_forced_kernels.cc:43-61; false: outcome b is unreachable
+    CSVM_INLINE bool forced_branch(double p0, double p1, double total, uint32_t b) {
+        const double eps = kDustEpsilon * total;
+        if (p1 <= eps) {
+            if (p1 > 0.0) dust++;
+            return b == 0;
+        }
+        if (p0 <= eps) {
+            if (p0 > 0.0) dust++;
+            return b == 1;
+        }
+        logp += log((b ? p1 : p0) / total);
+        return true;
+    }
 
     // ------------------------------------------------------------- splitting
     // The live shots' keys (below nkeys) become the new node numbers, in key
@@ -521,24 +781,27 @@ struct TreeInterp : LaneInterp<FW> {
     }
 
     // The measurement's shots draw (or are told) their outcomes and part.
-    CSVM_INLINE void measure(uint32_t rank, uint32_t axis, uint32_t idx, uint32_t sign, bool interfere, bool forced_op) {
+    CSVM_INLINE void measure(cptr<TreeQuad> row, uint32_t units, uint32_t rank, uint32_t idx, bool forced_op) {
         uint32_t b = 0, need = 0;
         double pb = 0.0;
         if (live) {
             const double p0 = psum[2 * node], p1 = psum[2 * node + 1], total = p0 + p1;
-            uint32_t m_abs, rec;
-            if (this->choose(p0, p1, total, interfere ? this->gz(axis) : this->gx(axis), sign, idx, forced_op, b, m_abs, rec)) {
-                pb = b ? p1 : p0;
-                this->set_x(axis, m_abs);
-                this->set_z(axis, 0u);
-                L::rset(this->rm, idx, rec);
-                // svm.h:177-186 rescales the array once |gamma|, the inverse of
-                // its norm, leaves [1e-100, 1e100]
-                need = (pb < 1e-200 && pb > 0.0) || pb > 1e200;
+            if (forced_op) {
+                // the response still holds the record of outcome 0
+                b = (forced[idx] ? 1u : 0u) ^ bits(idx, 1u);
+                if (!forced_branch(p0, p1, total, b)) {
+                    reachable = 0;
+                    live = 0;
+                }
             } else {
-                live = 0;
+                b = sample_branch(p0, p1, total);
             }
+            // svm.h:177-186 rescales the array once |gamma|, the inverse of
+            // its norm, leaves [1e-100, 1e100]
+            pb = b ? p1 : p0;
+            need = (pb < 1e-200 && pb > 0.0) || pb > 1e200;
         }
+        add_row(row, units, live && b);
         const uint32_t key = 2u * node + b, id = renumber(key, 2u * N, need);
         if (live) {
             nsrc2[id] = key;
@@ -562,128 +825,170 @@ struct TreeInterp : LaneInterp<FW> {
     }
 
     // ---------------------------------------------------------------- dispatch
-    // Walks the tree copy of the bytecode.  Tree opcodes are run by every
-    // thread (they hold barriers); the others by the live shots.
+    // Walks the bytecode.  Opcodes that hold barriers are run by every
+    // thread, the others by the live shots.
     CSVM_INLINE void run(cptr<DevProgram> Pg, double* ev_row) {
-        cptr<DevProgram> P0 = opaque(Pg);
-        cptr<uint64_t> code = cp(reinterpret_cast<const uint64_t*>(P0->tree_bc));
-        const uint32_t n_instr = P0->tree_n;
-        uint32_t skip = 0, wbegin = 0, wend = 0;
-        for (uint32_t pc = 0; pc < n_instr; pc += 1 + skip) {
-            if (pc >= wend) {  // the next instructions into LDS: a scalar load from L2 each would cost more
-                wbegin = pc;
-                wend = pc + kTreeWindow < n_instr ? pc + kTreeWindow : n_instr;
-                const uint64_t* from = reinterpret_cast<const uint64_t*>(opaque(Pg)->tree_bc) + 4 * (size_t)pc;
-                __syncthreads();
-                for (uint32_t e = tid; e < 4u * (wend - wbegin); e += nthreads) window[e] = from[e];
-                __syncthreads();
-            }
-            const lds_u64* ins = window + 4u * (pc - wbegin);
-            const uint64_t w0 = uni64(ins[0]), w1 = uni64(ins[1]), w2 = uni64(ins[2]), w3 = uni64(ins[3]);
-            const uint32_t op = (uint32_t)(w0 & 0xFF);
-            const uint32_t reserved = (uint32_t)(w0 >> 8) & 0xFFu;
-            const uint32_t flags_ = (uint32_t)((w0 >> 16) & 0xFF);
-            const uint32_t a1 = (uint32_t)((w0 >> 32) & 0xFFFF);
-            const uint32_t a2 = (uint32_t)(w0 >> 48);
-            const uint32_t i0 = (uint32_t)w1, i1 = (uint32_t)(w1 >> 32);
-            skip = op >= kLaneFrameRun ? a2 : 0u;
-            if (op >= kTreeChoice && op <= kTreeEv) {
-                if (op == kTreeChoice) {
-                    uint32_t c = this->gx(a1);
-                    if (reserved >= 2u) c |= this->gz(a1) << 1;
-                    if (reserved == 4u) c |= (this->gx(a2) << 2) | (this->gz(a2) << 3);
-                    choice_split(c, reserved, i0);
-                    continue;
-                }
-                if (op == kTreeNode) {
-                    if (live) {
-                        cptr<DevProgram> P = opaque(Pg);
-                        const uint32_t s = (this->gz(a1) << 1) | this->gx(a1);
-                        uint32_t o;
-                        if (reserved) {
-                            const clifft_u4_entry* e = &P->u4[i0].entries[(this->gz(a2) << 3) | (this->gx(a2) << 2) | s];
-                            o = e->out_state;
-                            this->set_x(a2, (o >> 2) & 1u);
-                            this->set_z(a2, (o >> 3) & 1u);
-                        } else {
-                            const clifft_u2_node* e = P->u2 + i0;
-                            o = e->out_states[s];
-                        }
-                        this->set_x(a1, o & 1u);
-                        this->set_z(a1, (o >> 1) & 1u);
-                    }
-                    continue;
-                }
-                const uint32_t kind = (uint32_t)w2;
+        const uint32_t n_instr = opaque(Pg)->tree_n;
+        cptr<uint64_t> code = (cptr<uint64_t>)cp(opaque(Pg)->tree_bc);
+        uint64_t n0 = code[0], n1 = code[1], n2 = code[2];
+        for (uint32_t pc = 0; pc < n_instr; ++pc) {
+            const uint64_t w0 = n0, w1 = n1, w2 = n2;
+            code = opaque(code + 4);  // (the next instruction arrives while this one runs)
+            n0 = code[0];
+            n1 = code[1];
+            n2 = code[2];
+            const uint32_t op = (uint32_t)(w0 & 0xFF), reserved = (uint32_t)(w0 >> 8) & 0xFFu;
+            const uint32_t count = (uint32_t)((w0 >> 32) & 0xFFFF), i0 = (uint32_t)w1, i1 = (uint32_t)(w1 >> 32);
+            const uint32_t units = (uint32_t)(w0 >> 48);
+            cptr<DevProgram> P = opaque(Pg);
+            if (op == kLpNoise) {
+                while (next_noise >= i0 && next_noise < i1) noise(P);  // (a dead shot's index is kNoNoise)
+            } else if (op == kTreeMeas || op == kTreePass || op == kTreeEv) {
                 uint32_t rank = 0;
                 int32_t ev_sign = 1;
-                if (op != kTreeEv || kind == 0u) pass(Pg, rank, ev_sign);
+                if (op != kTreeEv || w2 == 0u) pass(Pg, rank, ev_sign);
                 if (op == kTreeMeas) {
-                    measure(rank, a1, i0, flags_ & CLIFFT_FLAG_SIGN, (reserved & 1u) != 0u, (reserved & 2u) != 0u);
+                    measure(row_at(opaque(Pg), i1), units, rank, i0, reserved != 0u);
+                    if (!live) next_noise = kNoNoise;
                 } else if (op == kTreeEv && live && ev_row) {
-                    cptr<DevProgram> P = opaque(Pg);
-                    const uint64_t mx = cp(P->ev_x)[i0], mz = cp(P->ev_z)[i0];
-                    const uint32_t f = (load_u8(cp(P->ev_sign), i0) ? 1u : 0u) ^
-                                       ((uint32_t)(__popcll(mx & (uint64_t)this->pz) + __popcll(mz & (uint64_t)this->px)) & 1u);
-                    double v = kind == 1u ? 0.0 : 1.0;
-                    if (kind == 0u) {
+                    double v = w2 == 1u ? 0.0 : 1.0;
+                    if (w2 == 0u) {
                         const double den = psum[2 * node + 1];
                         v = den > 0.0 ? (double)ev_sign * psum[2 * node] / den : 0.0;
                     }
-                    if (f) v = -v;
+                    if (bits(i1, 1u)) v = -v;
                     v = v > 1.0 ? 1.0 : v;
-                    ev_row[i1] = v < -1.0 ? -1.0 : v;
+                    ev_row[i0] = v < -1.0 ? -1.0 : v;
                 }
-                continue;
-            }
-            if (!live) continue;
-            switch (op) {
-                case kLaneFrameRun: this->frame_run(a1, w1, w2, w3); break;
-                case kLaneFrameFan: this->frame_fan(reserved, a1, w1); break;
-                case kLaneDetectorRun: this->detector_run(code, pc, a2); break;
-                case kLaneMeasPauli:
-                    if (this->meas_dormant(reserved, a1, i0, flags_)) this->apply_pauli(w2, w3);
-                    break;
-                case CLIFFT_OP_FRAME_CNOT: this->frame_cnot(a1, a2); break;
-                case CLIFFT_OP_FRAME_CZ: this->frame_cz(a1, a2); break;
-                case CLIFFT_OP_FRAME_H: this->frame_h(a1); break;
-                case CLIFFT_OP_FRAME_S:
-                case CLIFFT_OP_FRAME_S_DAG: this->frame_s(a1); break;
-                case CLIFFT_OP_FRAME_SWAP: this->frame_swap(a1, a2); break;
-                case CLIFFT_OP_MEAS_DORMANT_STATIC:
-                case CLIFFT_OP_MEAS_DORMANT_RANDOM: this->meas_dormant(op, a1, i0, flags_); break;
-                case CLIFFT_OP_MEAS_DORMANT_STATIC_FORCED:
-                case CLIFFT_OP_MEAS_DORMANT_RANDOM_FORCED:
-                    if (!this->meas_dormant_forced(op, a1, i0, flags_)) live = 0;
-                    break;
-                case CLIFFT_OP_APPLY_PAULI:
-                    if (L::rget(this->rm, i1)) this->apply_pauli(w2, w3);
-                    break;
-                case CLIFFT_OP_NOISE:
-                    if (i0 == this->next_noise) this->noise(opaque(Pg), i0);
-                    break;
-                case CLIFFT_OP_NOISE_BLOCK: this->noise_block(Pg, i0, i0 + i1); break;
-                case CLIFFT_OP_READOUT_NOISE: this->readout_noise(opaque(Pg), i0); break;
-                case CLIFFT_OP_DETECTOR:
-                case CLIFFT_OP_POSTSELECT:
-                case CLIFFT_OP_OBSERVABLE:
-                    if (!this->record_parity(Pg, op, flags_, i0, i1, w2, w3)) live = 0;
-                    break;
-                default: break;
+            } else if (op == kLpRandom) {
+                add_rows(row_at(P, i1), units, count, [&] { return live && (rng_next(rng) >> 63); });  // the draw is not below 1/2
+            } else if (op == kLpReadout) {
+                uint32_t r = i0;
+                add_rows(row_at(P, i1), units, count, [&] {
+                    bool fire = false;
+                    if (live) {
+                        if (kf) {
+                            fire = kf_rpos < kf_n && kf[kf_rpos << 6] == r;
+                            if (fire) kf_rpos++;
+                        } else {
+                            fire = rng_double(rng) < cp(P->ro_prob)[r];
+                        }
+                    }
+                    ++r;
+                    return fire;
+                });
+            } else if (op == kTreeChoice) {
+                choice_split(bits(i0, reserved), reserved, (uint32_t)w2);
+            } else if (op == kTreeNode) {
+                const uint32_t st = bits(i1, reserved);
+                const uint32_t o = reserved == 4u ? P->u4[i0].entries[st].out_state : P->u2[i0].out_states[st];
+                for (uint32_t j = 0; j < reserved; ++j) add_row(row_at(P, (uint32_t)w2 + j * units), units, live && ((o >> j) & 1u));
+            } else if (op == kLpPostselect) {
+                if (live && bits(i0, 1u)) {
+                    cptr<uint32_t> row = cp(P->lp_dense) + (size_t)i1 * P->lp_words;
+                    for (uint32_t w = 0; w < P->lp_words; ++w) R[w << 6] &= row[w];
+                    discarded = 1;
+                    live = 0;
+                    next_noise = kNoNoise;
+                }
+            } else if (op == kLpCoin) {
+                bool one = false;
+                if (live) {
+                    logp += log(0.5);
+                    one = (forced[i0] ? 1u : 0u) != bits(i0, 1u);
+                }
+                add_row(row_at(P, i1), units, one);
+            } else {  // kLpStatic
+                if (live && (forced[i0] ? 1u : 0u) != bits(i0, 1u)) {
+                    reachable = 0;
+                    live = 0;
+                    next_noise = kNoNoise;
+                }
             }
         }
     }
 };
 
-// The calling workgroup runs the chunks of A->tree_chunk shots from c_first
-// on, c_step apart, of the shots [s_lo, s_hi) of the program.  `buf` (LDS
-// amplitudes: unused) holds 2 x A->amp_elems entries of the team.
-template <class FW, class AmpT>
+// Rows of n bits of a wavefront's first `shots` shots, shot f of the launch
+// on, from response word w0 on: one byte a bit, or 8 bits a byte.  The rows
+// are consecutive bytes, so the lanes write them 16 bytes (packed: 4 bytes)
+// a step, wherever shots begin, and not each its own shot byte by byte.
+CSVM_INLINE void tree_write_section(uint8_t* out, uint64_t f, uint32_t shots, uint32_t n, bool packed,
+                                    const tree_lds_u32* wave_R, uint32_t w0, uint32_t lane) {
+    if (!out || n == 0 || shots == 0) return;
+    const tree_lds_u32* R = wave_R + (w0 << 6);
+    const uint32_t row = packed ? (n + 7u) / 8u : n, total = shots * row, unit = packed ? 4u : 16u;
+    uint8_t* to = out + f * row;
+    const uint32_t head = (uint32_t)(reinterpret_cast<uintptr_t>(to) & (unit - 1u));
+    for (uint32_t b = unit * lane; b < total + head; b += 64u * unit) {
+        // bytes [lo, hi) of the section; lo is unit-aligned except at its start
+        const uint32_t lo = b < head ? 0u : b - head, hi = b + unit - head < total ? b + unit - head : total;
+        uint32_t s = lo / row, i = lo - s * row, acc = 0;
+        for (uint32_t t = lo; t < hi;) {
+            const uint32_t take = hi - t < row - i ? hi - t : row - i;
+            const tree_lds_u32* col = R + s;
+            if (packed) {
+                const uint32_t w = i >> 2, sh = (i & 3u) * 8u;
+                uint64_t x = col[w << 6];
+                if (sh && (w + 1u) * 4u < row) x |= (uint64_t)col[(w + 1u) << 6] << 32;
+                const uint32_t m = take < 4u ? (1u << (8u * take)) - 1u : 0xFFFFFFFFu;
+                acc |= ((uint32_t)(x >> sh) & m) << (8u * (t - lo));
+            } else {
+                const uint32_t w = i >> 5, sh = i & 31u;
+                uint64_t x = col[w << 6];
+                if (sh + take > 32u) x |= (uint64_t)col[(w + 1u) << 6] << 32;
+                acc |= ((uint32_t)(x >> sh) & ((1u << take) - 1u)) << (t - lo);
+            }
+            t += take;
+            i = 0;
+            ++s;
+        }
+        if (packed) {
+            if (hi - lo == 4u)
+                *reinterpret_cast<uint32_t*>(to + lo) = acc;
+            else
+                for (uint32_t t = lo; t < hi; ++t) to[t] = (uint8_t)(acc >> (8u * (t - lo)));
+        } else if (hi - lo == 16u) {
+            // bits 4j .. 4j + 3 to the bytes of word j
+            TreeQuad q;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) q[j] = (((acc >> (4u * j)) & 15u) * 0x00204081u) & 0x01010101u;
+            *reinterpret_cast<TreeQuad*>(to + lo) = q;
+        } else {
+            for (uint32_t t = lo; t < hi; ++t) to[t] = (uint8_t)((acc >> (t - lo)) & 1u);
+        }
+    }
+}
+
+// What the wavefront's shots leave; s: this lane's shot within the launch,
+// if `mine`, f the first lane's.
+template <class S>
+CSVM_INLINE void tree_write_rows(cptr<DevProgram> P, cptr<ShotArgs> A, const S& shot, uint64_t s, uint64_t f, bool mine) {
+    const bool packed = (A->flags & CLIFFT_REC_PACKED) != 0;
+    const uint32_t shots = (uint32_t)__builtin_popcountll(__ballot(mine));
+    const uint32_t wm = lane_words(P->num_meas), wd = lane_words(P->num_det);
+    cptr<uint8_t> expo = cp(P->expected_obs);
+    for (uint32_t i = 0; i < P->n_expected_obs && i < P->num_obs; ++i)
+        if (load_u8(expo, i)) shot.R[(wm + wd + (i >> 5)) << 6] ^= 1u << (i & 31u);
+    tree_wave_fence();
+    const tree_lds_u32* R = shot.R - shot.lane;
+    tree_write_section(A->out_meas, f, shots, P->num_meas, packed, R, 0, shot.lane);
+    tree_write_section(A->out_det, f, shots, P->num_det, packed, R, wm, shot.lane);
+    tree_write_section(A->out_obs, f, shots, P->num_obs, packed, R, wm + wd, shot.lane);
+    tree_wave_fence();  // (the next chunk's shots overwrite the columns)
+    if (!mine) return;
+    if (A->out_disc) A->out_disc[s] = (uint8_t)shot.discarded;
+    if (A->mode == MODE_FORCED && A->out_logp) A->out_logp[s] = shot.reachable ? shot.logp : kUnreachable;
+    if (shot.dust && A->dust_counter) atomicAdd(A->dust_counter, (unsigned long long)shot.dust);
+}
+
+template <class AmpT>
 __device__ __forceinline__ void tree_range(cptr<DevProgram> Pg, cptr<ShotArgs> Ag, uint64_t c_first, uint64_t c_step,
                                            uint64_t s_lo, uint64_t s_hi, uint64_t seed, dv2* buf) {
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-    TreeInterp<FW, AmpT> S;
-    typedef typename TreeInterp<FW, AmpT>::lds_u32 lds_u32;
+    typedef TreeInterp<AmpT> Interp;
+    typedef tree_lds_u32 lds_u32;
+    Interp S;
     S.tid = threadIdx.x;
     S.lane = threadIdx.x & 63u;
     S.wave = uni(threadIdx.x >> 6);
@@ -692,8 +997,7 @@ __device__ __forceinline__ void tree_range(cptr<DevProgram> Pg, cptr<ShotArgs> A
     cptr<DevProgram> P = opaque(Pg);
     cptr<ShotArgs> A = opaque(Ag);
     const uint32_t chunk = A->tree_chunk, amp = A->amp_elems;
-    const uint32_t wm = lane_words(P->total_meas_slots), wd = lane_words(P->num_det);
-    const uint32_t nwords = wm + wd + lane_words(P->num_obs);
+    const uint32_t words = P->lp_words, kf_words = A->mode == MODE_KFAULT ? 5u * cp(A->kf)->k : 0u;
     unsigned char* p = smem;
     AmpT *b0, *b1;
     if (std::is_same<AmpT, lds_d2>::value) {
@@ -712,17 +1016,10 @@ __device__ __forceinline__ void tree_range(cptr<DevProgram> Pg, cptr<ShotArgs> A
     lds_u32* flag0 = (lds_u32*)p;
     const uint32_t fwords = tree_flag_words(chunk);
     p += (8u * fwords + 15u) / 16u * 16u;
-    S.stage = (typename TreeInterp<FW, AmpT>::lds_stage*)p;
+    S.stage = (typename Interp::lds_stage*)p;
     p += sizeof(TreeStage);
-    S.window = (typename TreeInterp<FW, AmpT>::lds_u64*)p;
-    p += 32u * kTreeWindow;
-    lds_col_u32* recs = (lds_col_u32*)(p + (size_t)S.wave * nwords * 256u) + S.lane;
+    S.R = (lds_u32*)(p + (size_t)S.wave * (words + kf_words) * 256u) + S.lane;
     S.scale_word = fwords - 1u;
-    S.rm = recs;
-    S.rd = recs + (wm << 6);
-    S.ro = S.rd + (wd << 6);
-    S.amp = nullptr;
-    S.k = 0;
     for (uint64_t c = c_first;; c += c_step) {
         const uint64_t s0 = s_lo + c * chunk;
         if (s0 >= s_hi) break;
@@ -730,13 +1027,17 @@ __device__ __forceinline__ void tree_range(cptr<DevProgram> Pg, cptr<ShotArgs> A
         const bool mine = S.tid < chunk && s < s_hi;
         A = opaque(Ag);
         P = opaque(Pg);
-        for (uint32_t w = 0; w < nwords; ++w) recs[w << 6] = 0u;
-        S.px = S.pz = 0;
+        {
+            cptr<uint32_t> first = cp(P->lp_dense);  // the constants
+            for (uint32_t w = 0; w < words; ++w) S.R[w << 6] = first[w];
+        }
         S.dust = 0;
         S.discarded = 0;
         S.reachable = 1;
         S.logp = 0.0;
         S.forced = nullptr;
+        S.kf = nullptr;
+        S.kf_nn = S.kf_pos = S.kf_n = S.kf_rpos = 0;
         S.next_noise = kNoNoise;
         S.load_pass(P, 0);
         S.rng = rng_for_shot(seed, A->shot_begin + s);
@@ -752,9 +1053,13 @@ __device__ __forceinline__ void tree_range(cptr<DevProgram> Pg, cptr<ShotArgs> A
         S.flags = flag0;
         S.flags2 = flag0 + fwords;
         double* ev_row = nullptr;
+        // svm.cc:602-606: no gap draw, fault set first
+        if (A->mode == MODE_KFAULT) S.kfault_prepare(cp(A->kf), S.R + (words << 6), mine);
         if (mine) {
-            S.next_noise = 0;
-            S.draw_next_noise(P, 0.0);
+            if (A->mode != MODE_KFAULT) {
+                S.next_noise = 0;
+                S.draw_next_noise(P, 0.0);
+            }
             if (A->mode == MODE_FORCED) S.forced = A->forced_records + s * P->num_meas;
             const uint32_t nev = P->num_ev;
             ev_row = A->out_ev ? A->out_ev + s * nev : nullptr;
@@ -764,13 +1069,13 @@ __device__ __forceinline__ void tree_range(cptr<DevProgram> Pg, cptr<ShotArgs> A
         if (S.tid == 0) {
             S.nsrc[0] = 0u;
             S.nch[0] = 0u;
-            S.src[0] = mk(1.0, 0.0);
+            if (amp) S.src[0] = mk(1.0, 0.0);
         }
         __syncthreads();
 
         S.run(Pg, ev_row);
 
-        if (mine) lane_write_rows(opaque(Pg), opaque(Ag), S, s);
+        tree_write_rows(opaque(Pg), opaque(Ag), S, s, s0 + 64u * S.wave, mine);
         __syncthreads();  // the tables and the state are rewritten by the next chunk
     }
 }

@@ -6,23 +6,50 @@
 
 namespace csvm {
 
-// Tree-bytecode opcodes (below the lane superinstructions, above the
-// reference's range).
-//   kTreeChoice  the shots of a node part by frame bits that the amplitudes
-//                depend on: reserved = how many bits (1: p_x of axis_1; 2:
-//                p_x, p_z of axis_1; 4: those of axis_1, then of axis_2),
-//                payload word 1 = their place in the node's choice word
-//   kTreeMeas    active measurement of axis_1 (reserved bit 0: interfere,
-//                else diagonal; bit 1: forced); payload word 1 = record
-//                index
-//   kTreePass    a pass with no per-shot part
-//   kTreeNode    the frame of a U2 (reserved 0) or U4 (reserved 1)
-//                node, payload word 1 = node index
-//   kTreeEv      EXP_VAL: payload word 1 = mask index | output index << 32,
-//                word 2 = kind (0: computed, 1: the value is 0, 2: it is +-1
-//                by the sign alone)
+// The shots' classical part is linear over GF(2): every record, detector and
+// observable bit, and every bit the walk has to read (whether a shot parts
+// from its node, a post-selection parity, the sign of an expectation value),
+// is a constant plus the sum of some of the shot's random bits.  A shot
+// therefore keeps these bits themselves (its "response"), starting from the
+// constants, and each random bit that comes up 1 adds the row of bits it
+// flips.  The Pauli frame and all opcodes that only move it are gone.
+//
+// Response: words of 32 bits -- measurement records, detectors, observables,
+// then the bits that are read -- each section starting on a word.
+// `dense` holds whole responses: number 0 the constants, the others sets of
+// bits to keep.  A row is what one random bit flips, few of the words: a list
+// of (word << 6, mask), the masks nonzero.  `rows` is made of units of four
+// such entries; the rows that an opcode names lie one after another, all of
+// axis_2 units, filled up with zeros.
+//
+// Opcodes (payload word 1 unless stated; a bit is word * 32 + position; a
+// row is named by its first unit):
+//   kLpRandom      axis_1 coin flips, rows from i1 on
+//   kLpNoise       the noise sites [i0, i1)
+//   kLpReadout     axis_1 readout-noise entries from i0 on, rows from i1 on
+//   kLpPostselect  the shot is discarded if bit i0 is set, keeping the bits
+//                  of response i1 of `dense`
+//   kLpCoin        forced coin flip of record i0, row i1
+//   kLpStatic      forced: record i0 has to equal its response bit
+//   kTreeChoice    the shots of a node part by the `reserved` bits from i0 on
+//                  (one word); payload word 2 = their place in the choice word
+//   kTreeMeas      active measurement into record i0, row i1 flipped by
+//                  outcome 1 (reserved bit 0: forced)
+//   kTreePass      a pass with no per-shot part
+//   kTreeNode      U2 (reserved 2) or U4 (reserved 4) node i0: its frame
+//                  state from the `reserved` bits at bit i1; payload word 2 =
+//                  first of as many rows, one per bit of the state it leaves
+//   kTreeEv        EXP_VAL: output i0, sign bit i1, payload word 2 = kind (0:
+//                  computed, 1: the value is 0, 2: it is +-1 by the sign)
 // kTreeMeas, kTreePass and the computed kTreeEv each run the next pass of
 // the plan: the program is straight-line, so passes run in table order.
+// The walk reads one instruction ahead: a spare one follows the last.
+constexpr uint32_t kLpRandom = 0xD0;
+constexpr uint32_t kLpNoise = 0xD1;
+constexpr uint32_t kLpReadout = 0xD2;
+constexpr uint32_t kLpPostselect = 0xD3;
+constexpr uint32_t kLpCoin = 0xD4;
+constexpr uint32_t kLpStatic = 0xD5;
 constexpr uint32_t kTreeChoice = 0xE0;
 constexpr uint32_t kTreeMeas = 0xE1;
 constexpr uint32_t kTreePass = 0xE2;
@@ -47,6 +74,19 @@ constexpr uint32_t kTreeMaxExpand = 5;   // pending expansions a pass reads thro
 constexpr uint32_t kTreeMaxGen = 31;     // general phases of a pass
 constexpr uint32_t kTreeMaxChoice = 32;  // bits of a node's choice word
 constexpr uint32_t kTreeMaxRank = 26;
+constexpr uint32_t kTreeMaxWords = 512;  // of a shot's response
+
+// A noise site: its channels [first, first + n) and its cumulative hazard.
+struct TreeSite {
+    uint32_t first, n;
+    double hazard;
+};
+// A channel: the running sum of its site's channel probabilities, and the
+// row it adds: entries [first, first + n), first even.
+struct TreeChan {
+    double cum;
+    uint32_t first, n;
+};
 
 // General phase of a pass: the entry is multiplied by (pr, pi), by its
 // conjugate where the node's choice bit is set (choice < 0: never).

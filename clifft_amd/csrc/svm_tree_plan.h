@@ -14,10 +14,11 @@
 //     quarter turn that all pairs share.  What the entries have in common
 //     goes on to the next pass: it never interferes, and at the end nothing
 //     reads it;
-//   * their effect on the Pauli frame becomes frame opcodes, which the
-//     caller packs into the lane superinstructions;
 //   * where the amplitudes depend on a frame bit that may be set (T, ROT,
-//     expansions: p_x; U2, U4: both bits), a kTreeChoice parts the shots.
+//     expansions: p_x; U2, U4: both bits), a kTreeChoice parts the shots;
+//   * the Pauli frame itself, with every opcode that only moves it, becomes
+//     the rows by which a shot's random bits flip its response
+//     (svm_tree_args.h), found by one backward pass over the program.
 // Expansions commute with the permutations and phases recorded before them
 // (they add the top axis), so a pass always applies expansions first.
 // Clifford phases are exact (signs and swaps of parts), so where they are
@@ -39,12 +40,388 @@ namespace csvm {
 
 struct TreePlan {
     bool ok = false;
-    std::vector<clifft_instruction> code;  // sampling opcodes; frame opcodes not packed yet
-    std::vector<uint8_t> idle;             // frame opcodes that are the identity from the zero frame
+    std::vector<clifft_instruction> code, forced;  // the sampled and the forced walk
     std::vector<TreePass> passes;
     std::vector<TreePhase> phases;
+    uint32_t words = 0;               // of a shot's response
+    std::vector<uint32_t> dense;      // `words` each
+    std::vector<uint32_t> rows;       // 8 words a unit
+    std::vector<TreeSite> sites;
+    std::vector<TreeChan> chans;
+    std::vector<uint32_t> chan_rows;  // two words an entry
+    bool can_force = false;           // every record slot is visible and written once
+    bool choices = false;             // some kTreeChoice parts the shots
     // per writing pass: bits that may part the shots before it, and its rank
     std::vector<std::pair<uint32_t, uint32_t>> sizes;
+};
+
+// The response rows: the program (frame opcodes, measurements, noise, and
+// the planner's opcodes) taken backward, with the response that an X or a Z
+// on each qubit, and each record bit, has from there on.
+class ResponsePlanner {
+  public:
+    ResponsePlanner(const clifft_program_view* view, const std::vector<clifft_instruction>& code, TreePlan& plan)
+        : v(view), in(code), out(plan) {}
+
+    bool run() {
+        wm = (v->num_measurements + 31) / 32;
+        wd = (v->num_detectors + 31) / 32;
+        wo = (v->num_observables + 31) / 32;
+        if (!single_writers()) return false;
+        // bits that are read, each opcode's within one word
+        read_at.assign(in.size(), 0);
+        uint32_t next = 32 * (wm + wd + wo);
+        for (size_t i = 0; i < in.size(); ++i) {
+            const uint32_t op = in[i].opcode;
+            const uint32_t n = op == kTreeChoice || op == kTreeNode ? in[i].reserved
+                               : op == kTreeEv || op == CLIFFT_OP_POSTSELECT ? 1u : 0u;
+            if (n == 0) continue;
+            if (next % 32 + n > 32) next = (next + 31) / 32 * 32;
+            read_at[i] = next;
+            next += n;
+        }
+        W = std::max<uint32_t>((next + 31) / 32, 1);
+        if (W > kTreeMaxWords) return false;
+        out.words = W;
+        const uint32_t nq = 64 * v->words;
+        rx.assign(nq, Row(W, 0));
+        rz.assign(nq, Row(W, 0));
+        rec.assign(v->total_meas_slots, Row(W, 0));
+        for (uint32_t i = 0; i < v->num_measurements; ++i) flip(rec[i], i);
+        constant.assign(W, 0);
+        out.sites.resize(v->num_sites);
+        out.chans.resize(v->num_channels);
+        for (uint32_t t = 0; t < v->num_sites; ++t) {
+            const uint32_t c0 = v->site_chan_off[t], c1 = v->site_chan_off[t + 1];
+            out.sites[t] = {c0, c1 - c0, v->hazards[t]};
+            double acc = 0.0;  // in the reference's summation order (svm_kernels.inl:1894-1909)
+            for (uint32_t c = c0; c < c1; ++c) out.chans[c] = {acc += v->chan_prob[c], 0, 0};
+        }
+        std::vector<clifft_instruction> code, forced;
+        for (size_t i = in.size(); i-- > 0;) back(i, code, forced);
+        std::reverse(code.begin(), code.end());
+        std::reverse(forced.begin(), forced.end());
+        out.code = merged(code);
+        out.forced = forced;
+        out.dense = constant;
+        for (std::vector<clifft_instruction>* c : {&out.code, &out.forced}) {
+            for (clifft_instruction& x : *c) place_rows(x);
+            c->push_back(make(kTreePass, 0, 0, 0));  // read ahead, never run
+        }
+        return true;
+    }
+
+  private:
+    typedef std::vector<uint32_t> Row;
+    const clifft_program_view* v;
+    const std::vector<clifft_instruction>& in;
+    TreePlan& out;
+    uint32_t W = 1, wm = 0, wd = 0, wo = 0;
+    std::vector<uint32_t> read_at;
+    std::vector<Row> rx, rz, rec;
+    Row constant;
+    std::vector<Row> all;  // rows by number, until they are laid down
+
+    static void add(Row& a, const Row& b) {
+        for (size_t w = 0; w < a.size(); ++w) a[w] ^= b[w];
+    }
+    static void flip(Row& a, uint32_t bit) { a[bit / 32] ^= 1u << (bit % 32); }
+    static void word(clifft_instruction& x, int w, uint64_t y) { memcpy(x.p.raw + 8 * w, &y, 8); }
+    uint32_t det_bit(uint32_t i) const { return 32 * wm + i; }
+    uint32_t obs_bit(uint32_t i) const { return 32 * (wm + wd) + i; }
+    uint32_t add_row(const Row& a) {
+        all.push_back(a);
+        return (uint32_t)all.size() - 1;
+    }
+    // Lay down the rows that an instruction names.
+    void place_rows(clifft_instruction& x) {
+        uint64_t w2;
+        memcpy(&w2, x.p.raw + 8, 8);
+        uint32_t first = x.p.classical.expected_val, n = 1;
+        if (x.opcode == kLpPostselect) {
+            x.p.classical.expected_val = (uint32_t)(out.dense.size() / W);
+            out.dense.insert(out.dense.end(), all[first].begin(), all[first].end());
+            return;
+        }
+        if (x.opcode == kTreeNode) {
+            first = (uint32_t)w2;
+            n = x.reserved;
+        } else if (x.opcode == kLpRandom || x.opcode == kLpReadout) {
+            n = x.axis_1;
+        } else if (x.opcode != kLpCoin && x.opcode != kTreeMeas) {
+            return;
+        }
+        size_t most = 1;
+        for (uint32_t r = first; r < first + n; ++r) {
+            size_t k = 0;
+            for (uint32_t m : all[r]) k += m != 0;
+            most = std::max(most, k);
+        }
+        const size_t units = (most + 3) / 4, base = out.rows.size() / 8;
+        for (uint32_t r = first; r < first + n; ++r) {
+            const size_t end = out.rows.size() + 8 * units;
+            entries(all[r], out.rows);
+            out.rows.resize(end, 0);
+        }
+        x.axis_2 = (uint16_t)units;
+        if (x.opcode == kTreeNode)
+            word(x, 1, base);
+        else
+            x.p.classical.expected_val = (uint32_t)base;
+    }
+    static void entries(const Row& a, std::vector<uint32_t>& to) {
+        for (uint32_t w = 0; w < a.size(); ++w)
+            if (a[w]) {
+                to.push_back(w << 6);
+                to.push_back(a[w]);
+            }
+    }
+    clifft_instruction make(uint32_t op, uint32_t count, uint64_t i0, uint64_t i1) {
+        clifft_instruction x;
+        memset(&x, 0, sizeof(x));
+        x.opcode = (uint8_t)op;
+        x.axis_1 = (uint16_t)count;
+        word(x, 0, (i0 & 0xFFFFFFFFu) | (i1 << 32));
+        return x;
+    }
+    // Every record and detector slot has one writer, and no post-selection
+    // stands between two terms of an observable: the response then holds each
+    // bit's final value, and what a discarded shot leaves is a set of bits.
+    bool single_writers() {
+        std::vector<uint8_t> m(v->total_meas_slots, 0), d(v->num_detectors, 0), o(v->num_observables, 0);
+        bool post = false;
+        std::vector<uint8_t> o_post(v->num_observables, 0);
+        for (const clifft_instruction& x : in) {
+            switch (x.opcode) {
+                case CLIFFT_OP_MEAS_DORMANT_STATIC: case CLIFFT_OP_MEAS_DORMANT_RANDOM: case kTreeMeas:
+                    if (m[x.p.classical.classical_idx]++) return false;
+                    break;
+                case CLIFFT_OP_POSTSELECT:
+                    for (size_t i = 0; i < o.size(); ++i) o_post[i] = o[i];
+                    post = true;
+                    if (d[x.p.pauli.condition_idx]++) return false;
+                    break;
+                case CLIFFT_OP_DETECTOR:
+                    if (d[x.p.pauli.condition_idx]++) return false;
+                    break;
+                case CLIFFT_OP_OBSERVABLE:
+                    if (post && o_post[x.p.pauli.condition_idx]) return false;
+                    o[x.p.pauli.condition_idx] = 1;
+                    break;
+            }
+        }
+        out.can_force = v->total_meas_slots == v->num_measurements;
+        for (uint8_t n : m) out.can_force = out.can_force && n == 1;
+        return true;
+    }
+    // the bits that stand when the walk has come to instruction i
+    Row written(size_t i) const {
+        Row a(W, 0);
+        for (size_t j = 0; j < i; ++j) {
+            const clifft_instruction& x = in[j];
+            uint32_t bit = ~0u;
+            if (x.opcode == CLIFFT_OP_MEAS_DORMANT_STATIC || x.opcode == CLIFFT_OP_MEAS_DORMANT_RANDOM || x.opcode == kTreeMeas) {
+                if (x.p.classical.classical_idx < v->num_measurements) bit = x.p.classical.classical_idx;
+            } else if (x.opcode == CLIFFT_OP_DETECTOR) {
+                bit = det_bit(x.p.pauli.condition_idx);
+            } else if (x.opcode == CLIFFT_OP_OBSERVABLE) {
+                bit = obs_bit(x.p.pauli.condition_idx);
+            }
+            if (bit != ~0u) a[bit / 32] |= 1u << (bit % 32);
+        }
+        return a;
+    }
+    template <class F>
+    void each_bit(const uint64_t* mask, F f) const {
+        for (uint32_t w = 0; w < v->words; ++w)
+            for (uint64_t r = mask[w]; r; r &= r - 1) f(64 * w + (uint32_t)__builtin_ctzll(r));
+    }
+    void parity_into(uint32_t list, bool obs, uint32_t bit) {
+        const uint32_t* off = obs ? v->obs_off : v->det_off;
+        const uint32_t* tgt = obs ? v->obs_tgt : v->det_tgt;
+        for (uint32_t j = off[list]; j < off[list + 1]; ++j) flip(rec[tgt[j]], bit);
+    }
+
+    void back(size_t i, std::vector<clifft_instruction>& code, std::vector<clifft_instruction>& forced) {
+        const clifft_instruction& x = in[i];
+        const uint32_t op = x.opcode, a = x.axis_1, b = x.axis_2;
+        const uint32_t sign = x.flags & CLIFFT_FLAG_SIGN, idx = x.p.classical.classical_idx;
+        auto both = [&](const clifft_instruction& y) {
+            code.push_back(y);
+            forced.push_back(y);
+        };
+        switch (op) {
+            case CLIFFT_OP_FRAME_CNOT:  // x_b ^= x_a, z_a ^= z_b
+                add(rx[a], rx[b]);
+                add(rz[b], rz[a]);
+                break;
+            case CLIFFT_OP_FRAME_CZ:  // z_b ^= x_a, z_a ^= x_b
+                add(rx[a], rz[b]);
+                add(rx[b], rz[a]);
+                break;
+            case CLIFFT_OP_FRAME_H:
+                rx[a].swap(rz[a]);
+                break;
+            case CLIFFT_OP_FRAME_S:
+            case CLIFFT_OP_FRAME_S_DAG:  // z_a ^= x_a
+                add(rx[a], rz[a]);
+                break;
+            case CLIFFT_OP_FRAME_SWAP:
+                if (a != b) {
+                    rx[a].swap(rx[b]);
+                    rz[a].swap(rz[b]);
+                }
+                break;
+            case CLIFFT_OP_MEAS_DORMANT_STATIC:  // record = x_a ^ sign
+                if (!(x.flags & CLIFFT_FLAG_IDENTITY)) add(rx[a], rec[idx]);
+                if (sign) add(constant, rec[idx]);
+                rec[idx].assign(W, 0);
+                forced.push_back(make(kLpStatic, 0, idx, 0));
+                break;
+            case CLIFFT_OP_MEAS_DORMANT_RANDOM: {  // x_a = m, z_a = 0, record = m ^ sign
+                Row m = rx[a];
+                add(m, rec[idx]);
+                if (sign) add(constant, rec[idx]);
+                const uint32_t r = add_row(m);
+                code.push_back(make(kLpRandom, 1, 0, r));
+                forced.push_back(make(kLpCoin, 1, idx, r));
+                rx[a].assign(W, 0);
+                rz[a].assign(W, 0);
+                rec[idx].assign(W, 0);
+                break;
+            }
+            case kTreeMeas: {  // x_a = m = outcome ^ (x_a or z_a), z_a = 0, record = m ^ sign
+                Row m = rx[a];
+                add(m, rec[idx]);
+                if (sign) add(constant, rec[idx]);
+                clifft_instruction y = make(kTreeMeas, 0, idx, add_row(m));
+                code.push_back(y);
+                y.reserved = 1;
+                forced.push_back(y);
+                (x.reserved & 1 ? rz : rx)[a] = m;
+                (x.reserved & 1 ? rx : rz)[a].assign(W, 0);
+                rec[idx].assign(W, 0);
+                break;
+            }
+            case kTreeChoice: {
+                clifft_instruction y = make(kTreeChoice, 0, read_at[i], 0);
+                y.reserved = x.reserved;
+                word(y, 1, x.p.classical.classical_idx);  // place in the choice word
+                read_frame(x, read_at[i]);
+                both(y);
+                out.choices = true;
+                break;
+            }
+            case kTreeNode: {  // the axes' bits become those of the state the node leaves
+                clifft_instruction y = make(kTreeNode, 0, idx, read_at[i]);
+                y.reserved = x.reserved;
+                const uint32_t r = add_row(rx[a]);
+                add_row(rz[a]);
+                if (x.reserved == 4) {
+                    add_row(rx[b]);
+                    add_row(rz[b]);
+                }
+                word(y, 1, r);
+                for (uint32_t q : {a, x.reserved == 4 ? b : a}) {
+                    rx[q].assign(W, 0);
+                    rz[q].assign(W, 0);
+                }
+                read_frame(x, read_at[i]);
+                both(y);
+                break;
+            }
+            case kTreePass:
+                both(x);
+                break;
+            case kTreeEv: {
+                const uint32_t ci = x.p.exp_val.cp_exp_val_idx;
+                clifft_instruction y = make(kTreeEv, 0, x.p.exp_val.exp_val_idx, read_at[i]);
+                memcpy(y.p.raw + 8, x.p.raw + 8, 8);  // kind
+                each_bit(v->ev_x + (size_t)ci * v->words, [&](uint32_t q) { flip(rz[q], read_at[i]); });
+                each_bit(v->ev_z + (size_t)ci * v->words, [&](uint32_t q) { flip(rx[q], read_at[i]); });
+                if (v->ev_sign[ci]) flip(constant, read_at[i]);
+                both(y);
+                break;
+            }
+            case CLIFFT_OP_APPLY_PAULI: {
+                const size_t m = (size_t)x.p.pauli.cp_mask_idx * v->words;
+                Row& r = rec[x.p.pauli.condition_idx];
+                each_bit(v->pauli_x + m, [&](uint32_t q) { add(r, rx[q]); });
+                each_bit(v->pauli_z + m, [&](uint32_t q) { add(r, rz[q]); });
+                break;
+            }
+            case CLIFFT_OP_NOISE:
+            case CLIFFT_OP_NOISE_BLOCK: {
+                const uint64_t s0 = x.p.pauli.cp_mask_idx;
+                const uint64_t s1 = std::min<uint64_t>(v->num_sites, op == CLIFFT_OP_NOISE ? s0 + 1 : s0 + x.p.pauli.condition_idx);
+                if (s0 >= s1) break;
+                for (uint32_t c = v->site_chan_off[s0]; c < v->site_chan_off[s1]; ++c) {
+                    Row r(W, 0);
+                    each_bit(v->chan_x + (size_t)c * v->words, [&](uint32_t q) { add(r, rx[q]); });
+                    each_bit(v->chan_z + (size_t)c * v->words, [&](uint32_t q) { add(r, rz[q]); });
+                    out.chans[c].first = (uint32_t)(out.chan_rows.size() / 2);
+                    entries(r, out.chan_rows);
+                    out.chans[c].n = (uint32_t)(out.chan_rows.size() / 2) - out.chans[c].first;
+                    if (out.chans[c].n & 1) out.chan_rows.resize(out.chan_rows.size() + 2, 0);
+                }
+                both(make(kLpNoise, 0, s0, s1));
+                break;
+            }
+            case CLIFFT_OP_READOUT_NOISE:
+                both(make(kLpReadout, 1, idx, add_row(rec[v->ro_meas_idx[idx]])));
+                break;
+            case CLIFFT_OP_DETECTOR:
+                parity_into(idx, false, det_bit(x.p.pauli.condition_idx));
+                if (x.flags & CLIFFT_FLAG_EXPECTED_ONE) flip(constant, det_bit(x.p.pauli.condition_idx));
+                break;
+            case CLIFFT_OP_POSTSELECT:
+                parity_into(idx, false, read_at[i]);
+                if (x.flags & CLIFFT_FLAG_EXPECTED_ONE) flip(constant, read_at[i]);
+                both(make(kLpPostselect, 0, read_at[i], add_row(written(i))));
+                break;
+            case CLIFFT_OP_OBSERVABLE:
+                parity_into(idx, true, obs_bit(x.p.pauli.condition_idx));
+                break;
+        }
+    }
+    // the frame bits of a choice or node, from bit `at` on: p_x (and p_z) of
+    // axis_1, then of axis_2
+    void read_frame(const clifft_instruction& x, uint32_t at) {
+        flip(rx[x.axis_1], at);
+        if (x.reserved >= 2) flip(rz[x.axis_1], at + 1);
+        if (x.reserved == 4) {
+            flip(rx[x.axis_2], at + 2);
+            flip(rz[x.axis_2], at + 3);
+        }
+    }
+    // Runs of coin flips and of readout entries become one instruction (their
+    // rows lie in program order only if reversed, so they are copied), and so
+    // do noise sites that follow one another.
+    std::vector<clifft_instruction> merged(const std::vector<clifft_instruction>& code) {
+        std::vector<clifft_instruction> o;
+        for (size_t i = 0; i < code.size();) {
+            const uint32_t op = code[i].opcode;
+            auto i0 = [&](size_t j) { return code[j].p.classical.classical_idx; };
+            auto i1 = [&](size_t j) { return code[j].p.classical.expected_val; };
+            size_t j = i + 1;
+            if (op == kLpNoise) {
+                while (j < code.size() && code[j].opcode == op && i0(j) == i1(j - 1)) ++j;
+                o.push_back(make(kLpNoise, 0, i0(i), i1(j - 1)));
+            } else if (op == kLpRandom || op == kLpReadout) {
+                while (j < code.size() && j - i < 0xFFFF && code[j].opcode == op && (op == kLpRandom || i0(j) == i0(j - 1) + 1)) ++j;
+                uint32_t first = 0;
+                for (size_t k = i; k < j; ++k) {
+                    const uint32_t at = add_row(Row(all[i1(k)]));
+                    if (k == i) first = at;
+                }
+                o.push_back(make(op, (uint32_t)(j - i), i0(i), first));
+            } else {
+                o.push_back(code[i]);
+            }
+            i = j;
+        }
+        return o;
+    }
 };
 
 class TreePlanner {
@@ -52,10 +429,12 @@ class TreePlanner {
     TreePlanner(const clifft_program_view* view, const std::vector<int32_t>& khist) : v(view), kh(khist) {}
 
     TreePlan run() {
-        if (v->words != 1 || v->peak_rank > kTreeMaxRank) return TreePlan();
+        if (v->peak_rank > kTreeMaxRank) return TreePlan();
+        mx.assign(v->words, 0);
+        mz.assign(v->words, 0);
         for (uint64_t i = 0; i < v->num_instructions; ++i)
             if (!step(v->bytecode[i], (uint32_t)kh[i])) return TreePlan();
-        out.ok = true;
+        out.ok = ResponsePlanner(v, code, out).run();
         return std::move(out);
     }
 
@@ -134,20 +513,21 @@ class TreePlanner {
     std::vector<Gen> gens;       // in order
     uint32_t nchoice = 0;        // choice bits in use
     uint32_t splits = 0;         // bits that may have parted the shots so far
-    uint64_t mx = 0, mz = 0;     // frame bits that may be nonzero
+    std::vector<uint64_t> mx, mz;  // frame bits that may be nonzero
+    std::vector<clifft_instruction> code;  // frame opcodes and the planner's
 
     static uint32_t par(uint32_t x) { return (uint32_t)__builtin_popcount(x) & 1u; }
-    static uint64_t bit(uint32_t q) { return 1ull << q; }
-    bool hx(uint32_t q) const { return (mx >> q) & 1ull; }
-    bool hz(uint32_t q) const { return (mz >> q) & 1ull; }
+    static bool has(const std::vector<uint64_t>& m, uint32_t q) { return (m[q / 64] >> (q % 64)) & 1ull; }
+    static void set(std::vector<uint64_t>& m, uint32_t q, bool b) {
+        m[q / 64] = (m[q / 64] & ~(1ull << (q % 64))) | ((uint64_t)b << (q % 64));
+    }
+    bool hx(uint32_t q) const { return has(mx, q); }
+    bool hz(uint32_t q) const { return has(mz, q); }
+    bool on_frame(uint32_t q) const { return q < 64 * v->words; }
     uint32_t rank() const { return r0 + (uint32_t)exps.size(); }
 
     // ------------------------------------------------------------ emission
-    clifft_instruction& emit(const clifft_instruction& in, bool idle = false) {
-        out.code.push_back(in);
-        out.idle.push_back(idle ? 1 : 0);
-        return out.code.back();
-    }
+    void emit(const clifft_instruction& in) { code.push_back(in); }
     clifft_instruction blank(uint32_t op, uint32_t a1 = 0, uint32_t a2 = 0) {
         clifft_instruction in;
         memset(&in, 0, sizeof(in));
@@ -157,43 +537,41 @@ class TreePlanner {
         return in;
     }
     static void word(clifft_instruction& in, int w, uint64_t x) { memcpy(in.p.raw + 8 * w, &x, 8); }
-    // a frame opcode, with the bits it may set (the rules of the frame
-    // handlers); marked idle when every bit it reads is known zero
+    // a frame opcode, and the bits it may set (the rules of the frame handlers)
     void frame(uint32_t op, uint32_t a, uint32_t b) {
-        bool idle = false;
         const bool xa = hx(a), za = hz(a);
         switch (op) {
             case CLIFFT_OP_FRAME_CNOT:
-                idle = !xa && !hz(b);
-                if (hz(b)) mz |= bit(a);
-                if (xa) mx |= bit(b);
+                if (hz(b)) set(mz, a, true);
+                if (xa) set(mx, b, true);
                 break;
             case CLIFFT_OP_FRAME_CZ: {
                 const bool xb = hx(b);
-                idle = !xa && !xb;
-                if (xa) mz |= bit(b);
-                if (xb) mz |= bit(a);
+                if (xa) set(mz, b, true);
+                if (xb) set(mz, a, true);
                 break;
             }
             case CLIFFT_OP_FRAME_H:
-                idle = !xa && !za;
-                if (!idle) mx |= bit(a), mz |= bit(a);
+                set(mx, a, za);
+                set(mz, a, xa);
                 break;
             case CLIFFT_OP_FRAME_S:
             case CLIFFT_OP_FRAME_S_DAG:
-                idle = !xa;
-                if (xa) mz |= bit(a);
+                if (xa) set(mz, a, true);
                 break;
             default: {  // FRAME_SWAP
                 const bool xb = hx(b), zb = hz(b);
-                idle = !xa && !za && !xb && !zb;
-                const uint64_t m = ~(bit(a) | bit(b));
-                mx = (mx & m) | (xb ? bit(a) : 0) | (xa ? bit(b) : 0);
-                mz = (mz & m) | (zb ? bit(a) : 0) | (za ? bit(b) : 0);
+                set(mx, a, xb);
+                set(mx, b, xa);
+                set(mz, a, zb);
+                set(mz, b, za);
                 break;
             }
         }
-        emit(blank(op, a, b), idle);
+        emit(blank(op, a, b));
+    }
+    void any(std::vector<uint64_t>& m, const uint64_t* bits) {
+        for (uint32_t w = 0; w < v->words; ++w) m[w] |= bits[w];
     }
     // the shots part by `bits` frame bits; their place in the choice word
     int choice(uint32_t a, uint32_t b, uint32_t bits) {
@@ -413,8 +791,8 @@ class TreePlanner {
         emit(m);
         consumed(p, identity(r - 1), t.below(r - 1));
         splits += 1;
-        mx |= bit(axis);
-        mz &= ~bit(axis);
+        set(mx, axis, true);
+        set(mz, axis, false);
     }
     static bool unit(double re, double im) { return std::fabs(std::hypot(re, im) - 1.0) < 1e-9; }
 
@@ -423,11 +801,11 @@ class TreePlanner {
         double zr = 0.70710678118654752440, zi = zr;
         switch (op) {
             case CLIFFT_OP_FRAME_CNOT: case CLIFFT_OP_FRAME_CZ: case CLIFFT_OP_FRAME_SWAP:
-                if (a >= 64 || b >= 64) return false;
+                if (!on_frame(a) || !on_frame(b)) return false;
                 frame(op, a, b);
                 return true;
             case CLIFFT_OP_FRAME_H: case CLIFFT_OP_FRAME_S: case CLIFFT_OP_FRAME_S_DAG:
-                if (a >= 64) return false;
+                if (!on_frame(a)) return false;
                 frame(op, a, 0);
                 return true;
             case CLIFFT_OP_ARRAY_CNOT:
@@ -471,7 +849,7 @@ class TreePlanner {
             case CLIFFT_OP_ARRAY_T:
             case CLIFFT_OP_ARRAY_T_DAG:
             case CLIFFT_OP_ARRAY_ROT: {
-                if (a >= 64) return false;
+                if (!on_frame(a)) return false;
                 if (op == CLIFFT_OP_ARRAY_T_DAG) zi = -zi;
                 if (op == CLIFFT_OP_ARRAY_ROT) zr = in.p.math.weight_re, zi = in.p.math.weight_im;
                 if (!unit(zr, zi)) return false;
@@ -491,7 +869,7 @@ class TreePlanner {
                 frame(CLIFFT_OP_FRAME_H, a, 0);
                 return true;
             case CLIFFT_OP_ARRAY_U2: {
-                if (a >= 64) return false;
+                if (!on_frame(a)) return false;
                 if (a >= k) {
                     // the amplitudes stay; |gamma| must not tell shots apart
                     for (const double* g : {v->u2_nodes[in.p.u.cp_idx].gamma[0], v->u2_nodes[in.p.u.cp_idx].gamma[1],
@@ -504,10 +882,11 @@ class TreePlanner {
                     out.passes[p].choice = (uint32_t)c;
                 }
                 clifft_instruction n = blank(kTreeNode, a);
+                n.reserved = 2;
                 word(n, 0, in.p.u.cp_idx);
                 emit(n);
-                mx |= bit(a);
-                mz |= bit(a);
+                set(mx, a, true);
+                set(mz, a, true);
                 return true;
             }
             case CLIFFT_OP_ARRAY_U4: {
@@ -529,18 +908,20 @@ class TreePlanner {
                 for (uint32_t l = 0; l < r; ++l) stored[__builtin_ctz(q[l])] = 1u << l;
                 consumed(p, stored, t.below(r - 2).on(stored));
                 clifft_instruction n = blank(kTreeNode, a, b);
-                n.reserved = 1;
+                n.reserved = 4;
                 word(n, 0, in.p.u.cp_idx);
                 emit(n);
-                mx |= bit(a) | bit(b);
-                mz |= bit(a) | bit(b);
+                for (uint32_t q : {a, b}) {
+                    set(mx, q, true);
+                    set(mz, q, true);
+                }
                 return true;
             }
             case CLIFFT_OP_EXPAND:
             case CLIFFT_OP_EXPAND_T:
             case CLIFFT_OP_EXPAND_T_DAG:
             case CLIFFT_OP_EXPAND_ROT: {
-                if (a >= 64) return false;
+                if (!on_frame(a)) return false;
                 if (op == CLIFFT_OP_EXPAND_T_DAG) zi = -zi;
                 if (op == CLIFFT_OP_EXPAND_ROT) zr = in.p.math.weight_re, zi = in.p.math.weight_im;
                 Expand e;
@@ -555,23 +936,23 @@ class TreePlanner {
                 return true;
             }
             case CLIFFT_OP_MEAS_ACTIVE_DIAGONAL:
-                if (a >= 64) return false;
+                if (!on_frame(a)) return false;
                 meas(in, a, k - 1, false);
                 return true;
             case CLIFFT_OP_MEAS_ACTIVE_INTERFERE:
-                if (a >= 64) return false;
+                if (!on_frame(a)) return false;
                 meas(in, a, k - 1, true);
                 return true;
             case CLIFFT_OP_SWAP_MEAS_INTERFERE:
-                if (a >= 64 || b >= 64) return false;
+                if (!on_frame(a) || !on_frame(b)) return false;
                 if (a != b) frame(CLIFFT_OP_FRAME_SWAP, a, b);
                 meas(in, b, a == b ? k - 1 : a, true);
                 return true;
             case CLIFFT_OP_MEAS_DORMANT_RANDOM:
-                if (a >= 64) return false;
+                if (!on_frame(a)) return false;
                 emit(in);
-                mx |= bit(a);
-                mz &= ~bit(a);
+                set(mx, a, true);
+                set(mz, a, false);
                 return true;
             case CLIFFT_OP_MEAS_DORMANT_STATIC:
             case CLIFFT_OP_READOUT_NOISE:
@@ -582,8 +963,8 @@ class TreePlanner {
                 return true;
             case CLIFFT_OP_APPLY_PAULI:
                 emit(in);
-                mx |= v->pauli_x[in.p.pauli.cp_mask_idx];
-                mz |= v->pauli_z[in.p.pauli.cp_mask_idx];
+                any(mx, v->pauli_x + (size_t)in.p.pauli.cp_mask_idx * v->words);
+                any(mz, v->pauli_z + (size_t)in.p.pauli.cp_mask_idx * v->words);
                 return true;
             case CLIFFT_OP_NOISE:
             case CLIFFT_OP_NOISE_BLOCK: {
@@ -592,16 +973,19 @@ class TreePlanner {
                 const uint64_t s1 = std::min<uint64_t>(v->num_sites, op == CLIFFT_OP_NOISE ? s0 + 1 : s0 + in.p.pauli.condition_idx);
                 for (uint64_t s = s0; s < s1; ++s)
                     for (uint32_t c = v->site_chan_off[s]; c < v->site_chan_off[s + 1]; ++c) {
-                        mx |= v->chan_x[c];
-                        mz |= v->chan_z[c];
+                        any(mx, v->chan_x + (size_t)c * v->words);
+                        any(mz, v->chan_z + (size_t)c * v->words);
                     }
                 return true;
             }
             case CLIFFT_OP_EXP_VAL: {
                 const uint32_t ci = in.p.exp_val.cp_exp_val_idx;
-                const uint64_t am = (1ull << k) - 1ull, x = v->ev_x[ci], z = v->ev_z[ci];
+                const uint64_t am = (1ull << k) - 1ull;
+                const uint64_t x = v->ev_x[(size_t)ci * v->words], z = v->ev_z[(size_t)ci * v->words];
+                bool dormant = (x & ~am) != 0;
+                for (uint32_t w = 1; w < v->words; ++w) dormant = dormant || v->ev_x[(size_t)ci * v->words + w];
                 uint32_t kind = 0;
-                if (x & ~am) {
+                if (dormant) {
                     kind = 1;
                 } else if (k == 0) {
                     kind = 2;

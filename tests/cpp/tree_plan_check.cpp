@@ -33,18 +33,19 @@ struct Shot {
     const TreePlan& P;
     std::vector<cd> st{cd(1, 0)};
     uint32_t choice = 0;
-    uint64_t x = 0, z = 0;
+    std::vector<uint32_t> R;  // the response
     Rng rng;
     uint32_t next_noise = 0;
     double p[2] = {0, 0}, num = 0, den = 0;
     size_t next_pass = 0;
-    uint8_t *meas, *det, *obs;
     double* ev;
+    bool discarded = false;
 
-    uint32_t gx(uint32_t q) const { return (uint32_t)(x >> q) & 1u; }
-    uint32_t gz(uint32_t q) const { return (uint32_t)(z >> q) & 1u; }
-    void setx(uint32_t q, uint32_t b) { x = (x & ~(1ull << q)) | ((uint64_t)b << q); }
-    void setz(uint32_t q, uint32_t b) { z = (z & ~(1ull << q)) | ((uint64_t)b << q); }
+    uint32_t bits(uint32_t at, uint32_t n) const { return (R[at / 32] >> (at % 32)) & ((1u << n) - 1u); }
+    // the row of `units` units from unit r on
+    void add_row(uint32_t r, uint32_t units) {
+        for (uint32_t e = 4 * r; e < 4 * (r + units); ++e) R.at(P.rows[2 * e] >> 6) ^= P.rows[2 * e + 1];
+    }
     void draw(double cur) {
         if (next_noise >= v->num_sites) {
             next_noise = ~0u;
@@ -144,37 +145,46 @@ struct Shot {
         if (q.reset) choice = 0;
     }
     void run() {
-        for (const clifft_instruction& in : P.code) {
-            const uint32_t a = in.axis_1, b = in.axis_2;
+        R.assign(P.dense.begin(), P.dense.begin() + P.words);
+        for (size_t pc = 0; pc + 1 < P.code.size(); ++pc) {
+            const clifft_instruction& in = P.code[pc];
             uint64_t w0, w1;
             memcpy(&w0, in.p.raw, 8);
             memcpy(&w1, in.p.raw + 8, 8);
-            const uint32_t i0 = (uint32_t)w0, i1 = (uint32_t)(w0 >> 32), sign = in.flags & CLIFFT_FLAG_SIGN;
+            const uint32_t i0 = (uint32_t)w0, i1 = (uint32_t)(w0 >> 32), n = in.reserved;
             switch (in.opcode) {
-                case CLIFFT_OP_FRAME_CNOT: x ^= (uint64_t)gx(a) << b, z ^= (uint64_t)gz(b) << a; break;
-                case CLIFFT_OP_FRAME_CZ: {
-                    const uint64_t xa = gx(a), xb = gx(b);
-                    z ^= (xa << b) ^ (xb << a);
+                case kLpRandom:
+                    for (uint32_t j = 0; j < in.axis_1; ++j)
+                        if (!(rng.uniform() < 0.5)) add_row(i1 + j * in.axis_2, in.axis_2);
                     break;
-                }
-                case CLIFFT_OP_FRAME_H: {
-                    const uint64_t d = (uint64_t)(gx(a) ^ gz(a)) << a;
-                    x ^= d, z ^= d;
+                case kLpNoise:
+                    while (next_noise >= i0 && next_noise < i1) {
+                        const TreeSite t = P.sites[next_noise];
+                        const double u = rng.uniform();
+                        for (uint32_t c = t.first; c < t.first + t.n; ++c)
+                            if (u * P.chans[t.first + t.n - 1].cum < P.chans[c].cum) {
+                                const TreeChan& ch = P.chans[c];
+                                if (ch.first & 1) R[0] = 0xDEADBEEF;  // not aligned
+                                for (uint32_t e = ch.first; e < ch.first + ch.n; ++e)
+                                    R.at(P.chan_rows[2 * e] >> 6) ^= P.chan_rows[2 * e + 1];
+                                break;
+                            }
+                        next_noise++;
+                        draw(t.hazard);
+                    }
                     break;
-                }
-                case CLIFFT_OP_FRAME_S: case CLIFFT_OP_FRAME_S_DAG: z ^= (uint64_t)gx(a) << a; break;
-                case CLIFFT_OP_FRAME_SWAP: {
-                    const uint32_t xa = gx(a), xb = gx(b), za = gz(a), zb = gz(b);
-                    setx(a, xb), setx(b, xa), setz(a, zb), setz(b, za);
+                case kLpReadout:
+                    for (uint32_t j = 0; j < in.axis_1; ++j)
+                        if (rng.uniform() < v->ro_prob[i0 + j]) add_row(i1 + j * in.axis_2, in.axis_2);
                     break;
-                }
-                case kTreeChoice: {
-                    uint32_t c = gx(a);
-                    if (in.reserved >= 2) c |= gz(a) << 1;
-                    if (in.reserved == 4) c |= gx(b) << 2 | gz(b) << 3;
-                    choice |= c << i0;
+                case kLpPostselect:
+                    if (bits(i0, 1)) {
+                        for (uint32_t w = 0; w < P.words; ++w) R[w] &= P.dense[(size_t)i1 * P.words + w];
+                        discarded = true;
+                        return;
+                    }
                     break;
-                }
+                case kTreeChoice: choice |= bits(i0, n) << w1; break;
                 case kTreePass: pass(P.passes[next_pass++]); break;
                 case kTreeMeas: {
                     const TreePass& q = P.passes[next_pass++];
@@ -186,66 +196,20 @@ struct Shot {
                     else o = rng.uniform() * tot < p[0] ? 0 : 1;
                     const uint32_t half = 1u << (q.r - 1);
                     st = std::vector<cd>(st.begin() + (o ? half : 0), st.begin() + (o ? 2 * half : half));
-                    const uint32_t m = o ^ ((in.reserved & 1) ? gz(a) : gx(a));
-                    setx(a, m), setz(a, 0);
-                    meas[i0] = (uint8_t)(m ^ sign);
+                    if (o) add_row(i1, in.axis_2);
                     break;
                 }
                 case kTreeNode: {
-                    const uint32_t s = gz(a) << 1 | gx(a);
-                    const uint32_t o = in.reserved ? v->u4_nodes[i0].entries[gz(b) << 3 | gx(b) << 2 | s].out_state
-                                                   : v->u2_nodes[i0].out_states[s];
-                    setx(a, o & 1), setz(a, (o >> 1) & 1);
-                    if (in.reserved) setx(b, (o >> 2) & 1), setz(b, (o >> 3) & 1);
+                    const uint32_t s = bits(i1, n);
+                    const uint32_t o = n == 4 ? v->u4_nodes[i0].entries[s].out_state : v->u2_nodes[i0].out_states[s];
+                    for (uint32_t b = 0; b < n; ++b)
+                        if ((o >> b) & 1) add_row((uint32_t)w1 + b * in.axis_2, in.axis_2);
                     break;
                 }
                 case kTreeEv: {
-                    const uint32_t kind = (uint32_t)w1, f = (v->ev_sign[i0] ? 1u : 0u) ^ par(v->ev_x[i0] & z) ^ par(v->ev_z[i0] & x);
-                    if (kind == 0) pass(P.passes[next_pass++]);
-                    const double r = kind == 1 ? 0.0 : kind == 2 ? 1.0 : (den > 0 ? num / den : 0.0);
-                    ev[i1] = std::fmax(-1.0, std::fmin(1.0, f ? -r : r));
-                    break;
-                }
-                case CLIFFT_OP_MEAS_DORMANT_STATIC:
-                    meas[i0] = (uint8_t)((in.flags & CLIFFT_FLAG_IDENTITY) ? sign : gx(a) ^ sign);
-                    break;
-                case CLIFFT_OP_MEAS_DORMANT_RANDOM: {
-                    const uint32_t m = rng.uniform() < 0.5 ? 0 : 1;
-                    setx(a, m), setz(a, 0);
-                    meas[i0] = (uint8_t)(m ^ sign);
-                    break;
-                }
-                case CLIFFT_OP_APPLY_PAULI:
-                    if (meas[i1]) x ^= v->pauli_x[i0], z ^= v->pauli_z[i0];
-                    break;
-                case CLIFFT_OP_NOISE: case CLIFFT_OP_NOISE_BLOCK: {
-                    const uint32_t end = in.opcode == CLIFFT_OP_NOISE ? i0 + 1 : i0 + i1;
-                    while (next_noise >= i0 && next_noise < end) {
-                        const uint32_t s = next_noise, c1 = v->site_chan_off[s + 1];
-                        double tot = 0, acc = 0;
-                        for (uint32_t c = v->site_chan_off[s]; c < c1; ++c) tot += v->chan_prob[c];
-                        const double r = rng.uniform() * tot;
-                        for (uint32_t c = v->site_chan_off[s]; c < c1; ++c)
-                            if (r < (acc += v->chan_prob[c])) {
-                                x ^= v->chan_x[c], z ^= v->chan_z[c];
-                                break;
-                            }
-                        next_noise++;
-                        draw(v->hazards[s]);
-                    }
-                    break;
-                }
-                case CLIFFT_OP_READOUT_NOISE:
-                    if (rng.uniform() < v->ro_prob[i0]) meas[v->ro_meas_idx[i0]] ^= 1;
-                    break;
-                case CLIFFT_OP_DETECTOR: case CLIFFT_OP_POSTSELECT: case CLIFFT_OP_OBSERVABLE: {
-                    const bool ob = in.opcode == CLIFFT_OP_OBSERVABLE;
-                    const uint32_t *off = ob ? v->obs_off : v->det_off, *tgt = ob ? v->obs_tgt : v->det_tgt;
-                    uint8_t q = !ob && (in.flags & CLIFFT_FLAG_EXPECTED_ONE) ? 1 : 0;
-                    for (uint32_t j = off[i0]; j < off[i0 + 1]; ++j) q ^= meas[tgt[j]];
-                    if (ob) obs[i1] ^= q;
-                    else det[i1] = in.opcode == CLIFFT_OP_POSTSELECT ? 0 : q;
-                    if (in.opcode == CLIFFT_OP_POSTSELECT && q) return;
+                    if (w1 == 0) pass(P.passes[next_pass++]);
+                    const double r = w1 == 1 ? 0.0 : w1 == 2 ? 1.0 : (den > 0 ? num / den : 0.0);
+                    ev[i0] = std::fmax(-1.0, std::fmin(1.0, bits(i1, 1) ? -r : r));
                     break;
                 }
             }
@@ -273,15 +237,15 @@ extern "C" int tree_sample(const clifft_program_view* v, const int32_t* khist, u
     for (uint64_t s = 0; s < shots; ++s) {
         Shot S{v, P};
         for (auto& r : S.rng.s) r = split();
-        std::vector<uint8_t> rec(v->total_meas_slots + 1, 0);
-        S.meas = rec.data();
-        S.det = det + s * v->num_detectors;
-        S.obs = obs + s * v->num_observables;
         S.ev = ev + s * v->num_exp_vals;
         S.draw(0.0);
         S.run();
-        memcpy(meas + s * v->num_measurements, rec.data(), v->num_measurements);
-        for (uint32_t i = 0; i < v->num_observables && i < v->num_expected_observables; ++i) S.obs[i] ^= v->expected_observables[i];
+        const uint32_t wm = (v->num_measurements + 31) / 32, wd = (v->num_detectors + 31) / 32;
+        for (uint32_t i = 0; i < v->num_measurements; ++i) meas[s * v->num_measurements + i] = (uint8_t)S.bits(i, 1);
+        for (uint32_t i = 0; i < v->num_detectors; ++i) det[s * v->num_detectors + i] = (uint8_t)S.bits(32 * wm + i, 1);
+        for (uint32_t i = 0; i < v->num_observables; ++i)
+            obs[s * v->num_observables + i] =
+                (uint8_t)(S.bits(32 * (wm + wd) + i, 1) ^ (i < v->num_expected_observables ? v->expected_observables[i] : 0));
     }
     return (int)P.passes.size();
 }

@@ -52,17 +52,32 @@ def check(lib, orc, p, shots, seed):
     n = lib.tree_sample(ctypes.addressof(v), kh.ctypes.data, shots, seed, *(a.ctypes.data for a in (m, d, o, e)))
     if n < 0:
         return n
-    rm, rd, ro, re, _ = orc.sample(p, shots, seed=seed, per_shot=True)
-    assert np.array_equal(m, rm) and np.array_equal(d, rd) and np.array_equal(o, ro)
+    rm, rd, ro, re, gone = orc.sample(p, shots, seed=seed, per_shot=True)
+    m, d, o, e, rm, rd, ro, re = (a[gone == 0] for a in (m, d, o, e, rm, rd, ro, re))
+    assert len(m) and np.array_equal(m, rm) and np.array_equal(d, rd) and np.array_equal(o, ro)
     np.testing.assert_allclose(e, re, atol=1e-12, rtol=0)
     return n
 
 
 @pytest.mark.parametrize("seed", range(40))
 def test_random_programs(lib, orc, seed):
-    p = random_program(9000 + seed, num_qubits=(6, 9, 14, 40, 64)[seed % 5], peak=(1, 3, 5, 6, 9)[seed % 5],
+    p = random_program(9000 + seed, num_qubits=(6, 9, 14, 70, 150)[seed % 5], peak=(1, 3, 5, 6, 9)[seed % 5],
                        length=(60, 160, 300)[seed % 3], noise=seed % 4 != 0, u_nodes=seed % 2 == 0)
     assert check(lib, orc, p, 24, seed) >= 0
+
+
+@pytest.mark.parametrize("distance,rounds", [(3, 3), (5, 2), (7, 2)])
+def test_memories(lib, orc, distance, rounds):
+    """Noisy surface-code memories (17, 49 and 97 qubits), also post-selected
+    on the first round's detectors (the surviving shots' rows)."""
+    from clifft_amd.compiler import compile as ccompile
+    from memory_circuit import memory_text
+    p = ccompile(memory_text(distance, rounds, 0.004))
+    assert check(lib, orc, p, 60, distance) >= 0
+    first = np.flatnonzero(p.bytecode["opcode"] == Op.DETECTOR)[: (distance ** 2 - 1) // 2]
+    p.bytecode["opcode"][first] = Op.POSTSELECT
+    p.has_postselection = True
+    assert check(lib, orc, p, 60, distance) >= 0
 
 
 @pytest.mark.parametrize("peak", [1, 2, 5, 6, 7, 11])
@@ -79,9 +94,11 @@ def test_clifford_t(lib, orc, t, resets):
 
 
 def test_refusals(lib, orc):
-    """Wide frames and non-unit rotation weights go to the other executors."""
-    assert check(lib, orc, random_program(1, num_qubits=70, peak=3, length=60), 2, 1) == -1
+    """Rotation weights off the unit circle and records written twice go to
+    the other executors."""
     from clifft_amd.program import build_program, make_array_rot, make_expand, make_meas
+    twice = [make_meas(Op.MEAS_DORMANT_RANDOM, 0, 0), make_meas(Op.MEAS_DORMANT_STATIC, 0, 0)]
+    assert check(lib, orc, build_program(twice, peak_rank=0, num_qubits=1, num_measurements=1), 2, 1) == -1
     p = build_program([make_expand(0), make_array_rot(0, 0.9, 0.1), make_meas(Op.MEAS_ACTIVE_DIAGONAL, 0, 0)],
                       peak_rank=1, num_qubits=1, num_measurements=1)
     assert check(lib, orc, p, 2, 1) == -1
