@@ -24,7 +24,7 @@ INCLUDE = os.path.join(ROOT, "include")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 LIB_SVM = os.path.join(HERE, "libclifft_svm.so")
-SVM_SOURCES = ["svm_kernels.hip", "svm_tree.hip", "svm_host.cpp"]
+SVM_SOURCES = ["svm_kernels.hip", "svm_tree.hip", "svm_terms.hip", "svm_host.cpp"]
 LIB_PROBE = os.path.join(HERE, "libclifft_probe.so")
 
 HIP_FLAGS = [

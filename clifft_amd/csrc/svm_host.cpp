@@ -296,6 +296,8 @@ struct clifft_svm_program {
     std::vector<clifft_instruction> host_bc;
     std::vector<int32_t> khist;
     std::vector<uint8_t> expected_obs;
+    std::vector<uint64_t> ev_x, ev_z;  // EXP_VAL masks
+    std::vector<uint8_t> ev_sign;
     uint32_t num_qubits = 0, peak_rank = 0, words = 1, nw = 1;
     uint32_t num_meas = 0, total_slots = 0, num_det = 0, num_obs = 0, num_ev = 0;
     bool has_postselection = false;
@@ -1369,6 +1371,9 @@ int clifft_svm_program_create(const clifft_program_view* view, clifft_svm_progra
     size_t o_ex = add(view->ev_x, view->num_ev_masks * W * 8);
     size_t o_ez = add(view->ev_z, view->num_ev_masks * W * 8);
     size_t o_es = add(view->ev_sign, view->num_ev_masks);
+    p->ev_x.assign(view->ev_x, view->ev_x + view->num_ev_masks * W);
+    p->ev_z.assign(view->ev_z, view->ev_z + view->num_ev_masks * W);
+    p->ev_sign.assign(view->ev_sign, view->ev_sign + view->num_ev_masks);
     size_t o_so = add(view->site_chan_off, view->num_sites > 0 ? (view->num_sites + 1) * 4 : 0);
     size_t o_cx = add(view->chan_x, view->num_channels * W * 8);
     size_t o_cz = add(view->chan_z, view->num_channels * W * 8);
@@ -3034,6 +3039,8 @@ struct clifft_svm_adjoint {
     double* psign = nullptr;
     AdjArgs* args_dev = nullptr;
     uint32_t args_slot = 0;
+    bool by_terms = false;  // runs from the tables of a TermPlan
+    TermArgs terms{};       // their addresses and sizes
     bool global_amps = false;
     uint32_t block = 256;
     size_t lds_bytes = 0;
@@ -3061,6 +3068,21 @@ bool adjoint_op_ok(uint8_t op) {
         default:
             return false;
     }
+}
+
+// Terms up to which their sums are taken instead of the state: half of what
+// makes the two equal.  Measured on one MI355X at 16 and at 512 angle vectors
+// (rank 6 to 14, one X probe over all axes whose terms double with every
+// second rotation): the terms take 6 us + 5.5 ns a term and parameter (1064
+// terms of 16 parameters 110 us, 4148 of 26 540), the sweeps 2 to 2.2 us an
+// operation to rank 8, 3.6 and 5.6 at rank 10 and 12 (16 vectors) and 9.5 to
+// 39 at rank 14 (16 and 512 vectors).
+size_t term_limit(const clifft_svm_program* p, uint32_t num_params) {
+    size_t ops = 0;
+    for (const clifft_instruction& in : p->host_bc) ops += in.opcode > CLIFFT_OP_FRAME_SWAP;
+    const double sweeps = (double)ops * (2.0 + std::ldexp(0.4e-3, (int)p->peak_rank));
+    const double even = (sweeps - 6.0) / (5.5e-3 * std::max(1.0, (double)num_params));
+    return (size_t)std::clamp(0.5 * even, 0.0, 65536.0);
 }
 
 int adjoint_ensure(void** ptr, size_t* cur, size_t bytes) {
@@ -3109,8 +3131,29 @@ int clifft_svm_adjoint_create(clifft_svm_program* p, const uint32_t* param_instr
     a->num_params = num_params;
     const size_t o_ps = align_up(std::max<size_t>(n, 1) * 4, 256);
     const size_t o_args = o_ps + align_up(psign.size() * 8, 256);
-    const size_t total = o_args + kAdjArgSlots * sizeof(AdjArgs);
+    const TermPlan plan = TermPlanner(p->host_bc.data(), n, p->khist.data(), slot_of.data(), num_params, p->num_ev, p->ev_x.data(),
+                                      p->ev_z.data(), p->ev_sign.data(), p->words)
+                              .run(term_limit(p, num_params));
+    const size_t o_terms = o_args + align_up(kAdjArgSlots * sizeof(AdjArgs), 256);
+    const size_t o_before = o_terms + align_up(plan.terms.size() * sizeof(AdjTerm), 256);
+    const size_t o_first = o_before + align_up(plan.before.size() * 8, 256);
+    const size_t total = o_first + align_up(plan.first.size() * 4 + 4, 256);
     hipError_t e = hipMalloc(&a->dev, total);
+    if (plan.ok && p->num_ev) {
+        auto* base = static_cast<uint8_t*>(a->dev);
+        a->by_terms = true;
+        a->terms.terms = reinterpret_cast<const AdjTerm*>(base + o_terms);
+        a->terms.before = reinterpret_cast<const uint64_t*>(base + o_before);
+        a->terms.first = reinterpret_cast<const uint32_t*>(base + o_first);
+        a->terms.active = plan.active;
+        a->terms.num_params = num_params;
+        a->terms.num_ev = p->num_ev;
+        a->terms.num_terms = (uint32_t)plan.terms.size();
+        if (e == hipSuccess && !plan.terms.empty())
+            e = hipMemcpy(base + o_terms, plan.terms.data(), plan.terms.size() * sizeof(AdjTerm), hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(base + o_before, plan.before.data(), plan.before.size() * 8, hipMemcpyHostToDevice);
+        if (e == hipSuccess) e = hipMemcpy(base + o_first, plan.first.data(), plan.first.size() * 4, hipMemcpyHostToDevice);
+    }
     if (e == hipSuccess && n) e = hipMemcpy(a->dev, slot_of.data(), n * 4, hipMemcpyHostToDevice);
     if (e == hipSuccess)
         e = hipMemcpy(static_cast<uint8_t*>(a->dev) + o_ps, psign.data(), psign.size() * 8, hipMemcpyHostToDevice);
@@ -3185,7 +3228,7 @@ int clifft_svm_adjoint_run(clifft_svm_adjoint* a, const double* thetas, uint64_t
     }
     DeviceInfo& di = device_info();
     uint64_t grid = std::min<uint64_t>(batch, (uint64_t)a->per_cu * di.num_cus);
-    if (a->global_amps) {
+    if (a->global_amps && !a->by_terms) {
         size_t free_b = 0, total_b = 0;
         if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) free_b = 8ull << 30;
         const size_t per_team = (size_t)32 << p->peak_rank;
@@ -3194,20 +3237,31 @@ int clifft_svm_adjoint_run(clifft_svm_adjoint* a, const double* thetas, uint64_t
         int rc = adjoint_ensure(&a->gscratch, &a->gscratch_bytes, grid * per_team);
         if (rc) return rc;
     }
-    AdjArgs A{};
-    A.thetas = d_th;
-    A.psign = a->psign;
-    A.slot_of = a->slot_of;
-    A.coeffs = d_c;
-    A.ev_out = d_ev;
-    A.grad_out = d_g;
-    A.gscratch = reinterpret_cast<dv2*>(a->gscratch);
-    A.batch = batch;
-    A.num_params = (uint32_t)np;
-    A.amp_elems = 1u << p->peak_rank;
-    AdjArgs* slot = a->args_dev + (a->args_slot++ % kAdjArgSlots);
-    HIP_TRY(hipMemcpyAsync(slot, &A, sizeof(A), hipMemcpyHostToDevice, st));
-    HIP_TRY(launch_adjoint(a->global_amps, (uint32_t)grid, a->block, a->lds_bytes, p->dp_dev, slot, st));
+    if (a->by_terms) {
+        TermArgs T = a->terms;
+        T.thetas = d_th;
+        T.psign = a->psign;
+        T.coeffs = d_c;
+        T.ev_out = d_ev;
+        T.grad_out = d_g;
+        T.batch = batch;
+        HIP_TRY(launch_terms(T, di.num_cus, st));
+    } else {
+        AdjArgs A{};
+        A.thetas = d_th;
+        A.psign = a->psign;
+        A.slot_of = a->slot_of;
+        A.coeffs = d_c;
+        A.ev_out = d_ev;
+        A.grad_out = d_g;
+        A.gscratch = reinterpret_cast<dv2*>(a->gscratch);
+        A.batch = batch;
+        A.num_params = (uint32_t)np;
+        A.amp_elems = 1u << p->peak_rank;
+        AdjArgs* slot = a->args_dev + (a->args_slot++ % kAdjArgSlots);
+        HIP_TRY(hipMemcpyAsync(slot, &A, sizeof(A), hipMemcpyHostToDevice, st));
+        HIP_TRY(launch_adjoint(a->global_amps, (uint32_t)grid, a->block, a->lds_bytes, p->dp_dev, slot, st));
+    }
     if (!dev) {
         if (exp_vals && nev) HIP_TRY(hipMemcpyAsync(exp_vals, d_ev, batch * nev * 8, hipMemcpyDeviceToHost, st));
         if (grads && np) HIP_TRY(hipMemcpyAsync(grads, d_g, batch * np * 8, hipMemcpyDeviceToHost, st));

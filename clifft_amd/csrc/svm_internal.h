@@ -11,6 +11,7 @@
 #include "clifft_svm.h"
 #include "svm_device.h"
 #include "svm_adjoint_args.h"
+#include "svm_terms.h"
 
 namespace csvm {
 
@@ -71,5 +72,8 @@ hipError_t launch_tree(const LaunchShape& L, const DevProgram* P, const ShotArgs
 hipError_t adjoint_occupancy(bool global_amps, uint32_t block, size_t lds_bytes, int* blocks_per_cu);
 hipError_t launch_adjoint(bool global_amps, uint32_t grid, uint32_t block, size_t lds_bytes, const DevProgram* P,
                           const AdjArgs* A, hipStream_t st);
+
+// Expectation values and gradients from a TermPlan.
+hipError_t launch_terms(const TermArgs& A, uint32_t num_cus, hipStream_t st);
 
 }  // namespace csvm

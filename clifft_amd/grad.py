@@ -11,8 +11,10 @@ R_Z(theta_i / pi) is one ARRAY_ROT / EXPAND_ROT instruction
     exp_vals, grads = adj.run(thetas, coeffs)            # numpy in, numpy out
     F = expectation(adj, thetas_tensor, coeffs_tensor)    # torch, differentiable
 
-F[b] = sum_j coeffs[j] * exp_vals[b, j]; dF/dtheta comes from one forward and
-one backward (adjoint) sweep per theta vector in a hand-written HIP kernel.
+F[b] = sum_j coeffs[j] * exp_vals[b, j].  Hand-written HIP kernels compute it
+and dF/dtheta, per theta vector from the probes' sums of products of sines and
+cosines where these are few, else by one forward and one backward (adjoint)
+sweep over the state.
 """
 
 from __future__ import annotations
