@@ -97,10 +97,10 @@ def sample(program, shots: int, seed=None, packed: bool = False) -> SampleResult
     def cols(n):
         return (n + 7) // 8 if packed else n
 
-    m = np.zeros((shots, cols(prog.num_measurements)), np.uint8)
-    d = np.zeros((shots, cols(prog.num_detectors)), np.uint8)
-    o = np.zeros((shots, cols(prog.num_observables)), np.uint8)
-    e = np.zeros((shots, prog.num_exp_vals), np.float64)
+    m = np.empty((shots, cols(prog.num_measurements)), np.uint8)
+    d = np.empty((shots, cols(prog.num_detectors)), np.uint8)
+    o = np.empty((shots, cols(prog.num_observables)), np.uint8)
+    e = np.empty((shots, prog.num_exp_vals), np.float64)
     rec = _lib.Records(_ptr(m), _ptr(d), _ptr(o), _ptr(e), None)
     flags = _lib.REC_PACKED if packed else 0
     _lib.check(_lib.lib().clifft_svm_sample(dp.handle, shots, _seed(seed), flags, ctypes.byref(rec), None), "sample")
@@ -271,10 +271,10 @@ def sample_k(program, shots: int, k: int, seed=None, packed: bool = False) -> Sa
     def cols(n):
         return (n + 7) // 8 if packed else n
 
-    m = np.zeros((shots, cols(prog.num_measurements)), np.uint8)
-    d = np.zeros((shots, cols(prog.num_detectors)), np.uint8)
-    o = np.zeros((shots, cols(prog.num_observables)), np.uint8)
-    e = np.zeros((shots, prog.num_exp_vals), np.float64)
+    m = np.empty((shots, cols(prog.num_measurements)), np.uint8)
+    d = np.empty((shots, cols(prog.num_detectors)), np.uint8)
+    o = np.empty((shots, cols(prog.num_observables)), np.uint8)
+    e = np.empty((shots, prog.num_exp_vals), np.float64)
     rec = _lib.Records(_ptr(m), _ptr(d), _ptr(o), _ptr(e), None)
     flags = _lib.REC_PACKED if packed else 0
     _check_k(_lib.lib().clifft_svm_sample_k(dp.handle, shots, int(k), _seed(seed), flags, ctypes.byref(rec), None),

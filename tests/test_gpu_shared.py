@@ -77,3 +77,17 @@ def test_forced_records(svm, orc, n, t):
     rec = np.concatenate([rec, flipped])
     ref = orc.record_log_probs(p.forced(), rec)
     np.testing.assert_allclose(svm.record_probabilities(p, rec), ref, atol=1e-9, rtol=0)
+
+
+@pytest.mark.parametrize("n", [8, 9, 63, 64, 65, 128, 130])
+def test_row_widths(svm, orc, n):
+    """Rows that end at, before and behind the words and bytes they are
+    spread by; the last row's end is the array's."""
+    print("CASE shared rows", n, flush=True)
+    q = " ".join(map(str, range(n)))
+    p = ccompile(f"H {q}\nM {q}")
+    for shots in (1, 3, 64, 130):
+        ref = orc.sample(p, shots, seed=n)[0]
+        assert np.array_equal(svm.sample(p, shots, seed=n).measurements, ref)
+        packed = svm.sample(p, shots, seed=n, packed=True).measurements
+        assert np.array_equal(packed, np.packbits(ref, axis=1, bitorder="little"))
