@@ -23,7 +23,9 @@ per-shot byte model (16 B per amplitude read or written by each array opcode
 at its static rank, plus the record bytes) rides along as
 algorithmic_bytes_per_launch / model_GBps; fused passes move fewer bytes
 than it charges ("effective": model above the peak).  Without a measurement
-for the kernel, the model stands in ("achieved_from": "byte model").
+for the kernel, the model stands in ("achieved_from": "byte model") where it
+can: shots that share their states move a small part of what it charges, and
+beyond the peak achieved and frac are null.
 cpu_baseline: the C oracle built with -O3 -ffast-math -fopenmp, single PRNG
 stream, shots in sequence (the reference's scheduling), on a bounded sample;
 the shot-parallel OpenMP figure on all host cores rides along as "mode_b".
@@ -252,12 +254,14 @@ def _roofline(model_gbs, traffic, kernel_ms, model_bytes, **extra):
     """HBM roofline of the dominant kernel.  `achieved` and `frac` come from
     the PMC-measured HBM bytes of that kernel (profiles/hbm_traffic.json)
     when they were profiled for it; the byte model (one sweep per opcode,
-    an upper bound: fused passes move fewer bytes) is kept as
-    `model_GBps` and stands in, flagged, only without a measurement."""
+    an upper bound: fused passes and shared states move fewer bytes) is kept
+    as `model_GBps` and stands in, flagged, only without a measurement and up
+    to the peak."""
     measured = traffic is not None
-    achieved = traffic / (kernel_ms * 1e-3) / 1e9 if measured else model_gbs
-    r = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-         "traffic": traffic, "achieved_from": "PMC traffic" if measured else "byte model",
+    achieved = traffic / (kernel_ms * 1e-3) / 1e9 if measured else model_gbs if model_gbs <= HBM_PEAK_GBS else None
+    r = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+         "frac": None if achieved is None else achieved / HBM_PEAK_GBS, "traffic": traffic,
+         "achieved_from": "PMC traffic" if measured else "byte model" if achieved is not None else "not measured",
          "kernel_ms": kernel_ms, "algorithmic_bytes_per_launch": model_bytes, "model_GBps": model_gbs,
          "effective": model_gbs > HBM_PEAK_GBS}
     r.update(extra)
@@ -583,7 +587,9 @@ def main():
         with open(tpath) as f:
             tr = json.load(f)
         w = tr["workloads"].get(args.workload)
-        if w and w["shots"] == shots:
+        # (the profiles of the per-shot kernels, which ran these programs before)
+        per_shot = os.environ.get("CLIFFT_SHARED_STATE") == "0"
+        if w and w["shots"] == shots and w["kernel"].startswith("tree_kernel") != per_shot:
             traffic = (w["fetch_kib"] * tr["fetch_scale"] + w["write_kib"] * tr["write_scale"]) * 1024.0
     rec_bytes = nb(prog.num_measurements) + nb(prog.num_detectors) + nb(prog.num_observables)
     bytes_per_launch = (info["bytes_per_shot"] + rec_bytes) * shots

@@ -138,6 +138,8 @@ class Batch:
 
     def set_tuning(self, **kw):
         cur = self.tuning
+        if set(kw) in ({"concurrent"}, set(_TUNING_FIELDS)) and all(cur[f] == int(v) for f, v in kw.items()):
+            return  # the plan stands as it is
         cur.update(kw)
         t = _lib.BatchTuning(*[int(cur[f]) for f in _TUNING_FIELDS])
         _lib.check(_lib.lib().clifft_svm_batch_set_tuning(self.handle, ctypes.byref(t)), "batch_set_tuning")

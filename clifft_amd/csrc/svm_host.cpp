@@ -1170,6 +1170,14 @@ bool tree_better(const clifft_svm_program* p, uint64_t shots) {
     return 5.0 + 0.35 * p->tree_n + 2.0 * p->tree_sizes.size() <= 0.48 * (double)p->host_bc.size();
 }
 
+// Entries of a team's buffer up to which more shots may be put into it: where
+// frame bits part the shots, nodes grow with the shots at every rank, and one
+// such program would take tens of GiB of scratch (a batch of 512 took 99 GB
+// for the one with 2^24 entries a team); smaller chunks are the faster ones
+// there (random programs, peak 12 x 20000 shots: 5.6 ms at 2^18 entries a
+// team, 3.1 ms at 2^15).
+uint64_t tree_room(const clifft_svm_program* p) { return std::max<uint64_t>(1ull << 18, 1ull << p->peak_rank); }
+
 // The shared-state shape for a launch of `shots` shots: the team size and
 // the shots per team of the lowest estimate.  False: the program has no
 // plan, or the per-shot executors are faster.
@@ -1181,7 +1189,7 @@ bool tree_shape(const clifft_svm_program* p, uint64_t shots, uint32_t faults, La
         for (uint32_t chunk = threads; chunk >= 1; chunk /= 2) {
             if (chunk > 2 * shots && chunk > 1) continue;
             LaunchShape L;
-            if (!tree_team(p, threads, chunk, faults, L)) continue;
+            if (!tree_team(p, threads, chunk, faults, L) || (chunk > 1 && L.tree_elems > tree_room(p))) continue;
             const double c = tree_cost(p, L, shots);
             if (!found || c < cost) {
                 best = L;
@@ -1204,10 +1212,11 @@ bool tree_batch_shape(const clifft_svm_program* p, uint64_t shots, LaunchShape& 
     bool found = false;
     for (uint32_t threads : {1024u, 256u, 64u}) {
         if (found && threads == 64u) break;
-        for (uint32_t chunk = threads; chunk >= 64; chunk /= 2) {
+        for (uint32_t chunk = threads; chunk >= 1; chunk /= 2) {
             if (chunk > 64 && chunk >= 2 * shots) continue;
             LaunchShape L;
             if (!tree_team(p, threads, chunk, 0, L) || (found && L.global_amps && threads < best.block)) continue;
+            if (chunk > 1 && L.tree_elems > tree_room(p)) continue;
             const double part = std::max((double)threads / 1024.0, (double)L.lds_bytes / (double)kLdsBytes);
             const double c = std::ceil((double)shots / chunk) * part * tree_team_us(p, L, 1.0 / part);
             if (!found || c < cost) {
@@ -1288,10 +1297,13 @@ class PinnedBlock {
     PinnedBlock() = default;
     PinnedBlock(const PinnedBlock&) = delete;
     PinnedBlock& operator=(const PinnedBlock&) = delete;
+    // the call has waited for its stream
+    void done() { done_ = true; }
     ~PinnedBlock() {
         if (!ptr_) return;
+        if (!done_) (void)hipDeviceSynchronize();  // the call failed: its kernel may still be writing
         std::lock_guard<std::mutex> lock(mu());
-        if (idle_bytes() + bytes_ <= kPinnedIdle) {
+        if (done_ && idle_bytes() + bytes_ <= kPinnedIdle) {
             idle().push_back({ptr_, bytes_});
             idle_bytes() += bytes_;
         } else {
@@ -1326,6 +1338,7 @@ class PinnedBlock {
   private:
     void* ptr_ = nullptr;
     size_t bytes_ = 0;
+    bool done_ = false;
     static std::mutex& mu() {
         static std::mutex* m = new std::mutex;  // (never destroyed: calls may outlive static objects)
         return *m;
@@ -1803,6 +1816,7 @@ static int run_shots(clifft_svm_program* p, uint64_t shots, uint64_t seed, uint3
                 for (const Rows& r : all)
                     if (r.to && r.bytes) HIP_TRY(hipMemcpyAsync(r.to, r.from, r.bytes, hipMemcpyDeviceToHost, st));
             HIP_TRY(hipStreamSynchronize(st));
+            block.done();
             if (pinned)
                 for (const Rows& r : all) {
                     if (!r.to || !r.bytes) continue;
@@ -2903,7 +2917,10 @@ int clifft_svm_batch_set_tuning(clifft_svm_batch* b, const clifft_svm_batch_tuni
     clifft_svm_batch_tuning old = b->tuning;
     const bool old_shared = b->shared;
     b->tuning = *t;
-    b->shared = false;  // the tuning names every program's group
+    // the tuning names every program's group, unless all it changes is their order
+    clifft_svm_batch_tuning same = *t;
+    same.concurrent = old.concurrent;
+    if (t->concurrent == old.concurrent || std::memcmp(&same, &old, sizeof(old)) != 0) b->shared = false;
     rc = batch_plan(b, ~0ull, library_stream());
     if (rc) {
         std::string msg = g_last_error;

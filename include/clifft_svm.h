@@ -375,10 +375,10 @@ int clifft_svm_execute(clifft_svm_program* prog, clifft_svm_state* state);
  * LDS-resident amplitudes (<= lds_rank_max; split by team size), one
  * shot per wavefront with amplitudes in a global slice (<= gwave_rank_max),
  * or one shot per workgroup with amplitudes in a global slice
- * (global_threads per team).  Until clifft_svm_batch_set_tuning is called,
- * programs that are faster with many shots per workgroup sharing their
- * states run that way, in groups of kind 5; a tuning that was set names the
- * group of every program.  A group's work items (a shot range of one program) are sorted by
+ * (global_threads per team).  Until clifft_svm_batch_set_tuning is called
+ * for anything but a change of `concurrent`, programs that are faster with many shots per
+ * workgroup sharing their states run that way, in groups of kind 5; a tuning
+ * that was set names the group of every program.  A group's work items (a shot range of one program) are sorted by
  * descending estimated cost and drained by its teams from a device queue.
  * The groups run one after another on the caller's stream, or side by side
  * on the batch's own streams (concurrent = 1).
