@@ -1,0 +1,50 @@
+"""Planning an expectation value's sums (clifft_amd/csrc/svm_terms.h) is
+bounded by the work it does, not by the terms that remain: a probe whose
+terms all vanish at the last operation they reach is refused as soon as the
+paths outnumber a fixed multiple of the limit, and so are fixed phases, which
+no number of parameters bounds."""
+
+from __future__ import annotations
+
+import shutil
+import time
+
+import numpy as np
+import pytest
+
+from clifft_amd import program as P
+from test_terms import lib, run  # noqa: F401  (lib: the compiled planner)
+
+pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="no host C++ compiler")
+
+
+def vanishing(turns, fixed=False):
+    """H and a turn on axis 0 beside `turns` turns between Hs on axis 1; the
+    probe Z0 X1 is 0, which shows only at axis 0's expansion."""
+    bc = [P.make_expand_rot(0, np.cos(0.3), np.sin(0.3)), P.make_expand(1)]
+    slots = [0]
+    for i in range(turns):
+        if not fixed:
+            slots.append(len(bc))
+        bc += [P.make_array_t(1) if fixed else P.make_array_rot(1, np.cos(0.1 * i), np.sin(0.1 * i)), P.make_array_h(1)]
+    bc.append(P.make_exp_val(0, 0))
+    p = P.build_program(bc, peak_rank=2, num_qubits=2, num_exp_vals=1, exp_val_masks=[(2, 1, 0)])
+    return p, slots, np.array([0.3] + [0.1 * i for i in range(turns)])[: len(slots)]
+
+
+@pytest.mark.parametrize("turns,fixed", [(38, False), (60, False), (38, True), (400, True)])
+def test_vanishing_probes(lib, turns, fixed):  # noqa: F811
+    """1 s: a thousand times what the bounded walk takes, and less than the
+    unbounded one (2 s at 38 turns, 1.6 times as much for each more)."""
+    p, slots, angles = vanishing(turns, fixed)
+    t = time.perf_counter()
+    n = run(lib, p, slots, angles, limit=1000)[0]
+    assert time.perf_counter() - t < 1.0
+    assert n == -1
+
+
+@pytest.mark.parametrize("turns", [1, 2, 5, 9])
+def test_few_paths_are_still_taken(lib, turns):  # noqa: F811
+    p, slots, angles = vanishing(turns)
+    n, ev, grad = run(lib, p, slots, angles, limit=1000)
+    assert n == 0 and ev[0] == 0.0 and not grad.any()
