@@ -40,7 +40,9 @@ struct TermArgs {
     double* grad_out;         // [batch x num_params] or null
     const AdjTerm* terms;     // ascending by probe
     const uint32_t* first;    // [num_ev + 1]: each probe's terms
-    const uint64_t* before;   // [num_ev]: parameters whose phase the state holds at the probe
+    // [num_ev]: parameters whose phase the state holds at the probe, none where
+    // the probe is 0 for its X on a dormant axis
+    const uint64_t* before;
     uint64_t active;          // parameters that turn some axis of the state
     uint64_t batch;
     uint32_t num_params, num_ev, num_terms, pad;
@@ -133,12 +135,12 @@ class TermPlanner {
         uint64_t held = 0;
         for (size_t i = 0; i < at; ++i)
             if (slot_of[i] >= 0 && ((out.active >> slot_of[i]) & 1u)) held |= 1ull << slot_of[i];
-        out.before.push_back(held);
         const uint32_t ci = code[at].p.exp_val.cp_exp_val_idx, k = (uint32_t)rank[at];
         const uint64_t on = k >= 64 ? ~0ull : (1ull << k) - 1ull;
-        if (ev_x[(size_t)ci * W] & ~on) return true;  // X on a dormant axis: no terms
-        for (uint32_t w = 1; w < W; ++w)
-            if (ev_x[(size_t)ci * W + w]) return true;
+        bool dormant = (ev_x[(size_t)ci * W] & ~on) != 0;
+        for (uint32_t w = 1; w < W; ++w) dormant = dormant || ev_x[(size_t)ci * W + w];
+        out.before.push_back(dormant ? 0 : held);
+        if (dormant) return true;  // X on a dormant axis: no terms
         std::vector<Pauli> todo(1);
         todo[0] = {at, ev_x[(size_t)ci * W] & on, ev_z[(size_t)ci * W] & on, {ev_sign[ci] ? -1.0 : 1.0, 0, 0, j, 0}};
         while (!todo.empty()) {

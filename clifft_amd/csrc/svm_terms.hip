@@ -30,6 +30,15 @@ __global__ void __launch_bounds__(64) term_kernel(TermArgs A) {
     const uint32_t lane = threadIdx.x, np = A.num_params, nt = A.num_terms;
     double *co = lds, *si = lds + 64, *value = lds + 128, *carry = lds + 192;
     double *before = lds + 256, *sum = before + np * kTermRow;  // [parameter][lane]
+    // A weight that is not finite spreads over the whole state of the sweeps
+    // (svm_adjoint.h): no angle held at its probe has a derivative.
+    uint64_t lost = 0;
+    if (A.grad_out) {
+        for (uint32_t j = lane; j < A.num_ev; j += 64u)
+            if (!isfinite(A.coeffs[j])) lost |= A.before[j];
+        if (__any(lost != 0))
+            for (int o = 32; o; o >>= 1) lost |= __shfl_xor(lost, o, 64);
+    }
     for (uint64_t b = blockIdx.x; b < A.batch; b += gridDim.x) {
         bool finite = true;
         if (lane < np) {
@@ -93,7 +102,7 @@ __global__ void __launch_bounds__(64) term_kernel(TermArgs A) {
             const uint32_t lanes = nt < 64u ? nt : 64u;
             for (uint32_t l = 0; l < lanes; ++l) g += sum[lane * kTermRow + l];
             const double nan = __longlong_as_double(0x7FF8000000000000ll);
-            A.grad_out[b * np + lane] = !((A.active >> lane) & 1u) ? 0.0 : bad ? nan : g * A.psign[lane];
+            A.grad_out[b * np + lane] = !((A.active >> lane) & 1u) ? 0.0 : bad || ((lost >> lane) & 1u) ? nan : g * A.psign[lane];
         }
         term_fence();
     }
