@@ -187,7 +187,9 @@ class ResponsePlanner {
     // Every record and detector slot has one writer, and no post-selection
     // stands between two terms of an observable: the response then holds each
     // bit's final value, and what a discarded shot leaves is a set of bits.
+    // Every noise site has one instruction: its channels keep one row each.
     bool single_writers() {
+        std::vector<uint8_t> site(v->num_sites, 0);
         std::vector<uint8_t> m(v->total_meas_slots, 0), d(v->num_detectors, 0), o(v->num_observables, 0);
         bool post = false;
         std::vector<uint8_t> o_post(v->num_observables, 0);
@@ -204,6 +206,14 @@ class ResponsePlanner {
                 case CLIFFT_OP_DETECTOR:
                     if (d[x.p.pauli.condition_idx]++) return false;
                     break;
+                case CLIFFT_OP_NOISE:
+                case CLIFFT_OP_NOISE_BLOCK: {
+                    const uint64_t s0 = x.p.pauli.cp_mask_idx;
+                    const uint64_t s1 = std::min<uint64_t>(v->num_sites, x.opcode == CLIFFT_OP_NOISE ? s0 + 1 : s0 + x.p.pauli.condition_idx);
+                    for (uint64_t s = s0; s < s1; ++s)
+                        if (site[s]++) return false;
+                    break;
+                }
                 case CLIFFT_OP_OBSERVABLE:
                     if (post && o_post[x.p.pauli.condition_idx]) return false;
                     o[x.p.pauli.condition_idx] = 1;
