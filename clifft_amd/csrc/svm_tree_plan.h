@@ -89,6 +89,9 @@ class ResponsePlanner {
         rec.assign(v->total_meas_slots, Row(W, 0));
         for (uint32_t i = 0; i < v->num_measurements; ++i) flip(rec[i], i);
         constant.assign(W, 0);
+        standing.assign(W, 0);
+        for (const clifft_instruction& x : in)
+            if (const int64_t bit = writes(x); bit >= 0) standing[bit / 32] |= 1u << (bit % 32);
         out.sites.resize(v->num_sites);
         out.chans.resize(v->num_channels);
         for (uint32_t t = 0; t < v->num_sites; ++t) {
@@ -120,6 +123,7 @@ class ResponsePlanner {
     std::vector<uint32_t> read_at;
     std::vector<Row> rx, rz, rec;
     Row constant;
+    Row standing;  // the bits written before the instruction at hand
     std::vector<Row> all;  // rows by number, until they are laid down
 
     static void add(Row& a, const Row& b) {
@@ -224,22 +228,15 @@ class ResponsePlanner {
         for (uint8_t n : m) out.can_force = out.can_force && n == 1;
         return true;
     }
-    // the bits that stand when the walk has come to instruction i
-    Row written(size_t i) const {
-        Row a(W, 0);
-        for (size_t j = 0; j < i; ++j) {
-            const clifft_instruction& x = in[j];
-            uint32_t bit = ~0u;
-            if (x.opcode == CLIFFT_OP_MEAS_DORMANT_STATIC || x.opcode == CLIFFT_OP_MEAS_DORMANT_RANDOM || x.opcode == kTreeMeas) {
-                if (x.p.classical.classical_idx < v->num_measurements) bit = x.p.classical.classical_idx;
-            } else if (x.opcode == CLIFFT_OP_DETECTOR) {
-                bit = det_bit(x.p.pauli.condition_idx);
-            } else if (x.opcode == CLIFFT_OP_OBSERVABLE) {
-                bit = obs_bit(x.p.pauli.condition_idx);
-            }
-            if (bit != ~0u) a[bit / 32] |= 1u << (bit % 32);
+    // the visible bit that an instruction writes, or -1
+    int64_t writes(const clifft_instruction& x) const {
+        switch (x.opcode) {
+            case CLIFFT_OP_MEAS_DORMANT_STATIC: case CLIFFT_OP_MEAS_DORMANT_RANDOM: case kTreeMeas:
+                return x.p.classical.classical_idx < v->num_measurements ? x.p.classical.classical_idx : -1;
+            case CLIFFT_OP_DETECTOR: return det_bit(x.p.pauli.condition_idx);
+            case CLIFFT_OP_OBSERVABLE: return obs_bit(x.p.pauli.condition_idx);
         }
-        return a;
+        return -1;
     }
     template <class F>
     void each_bit(const uint64_t* mask, F f) const {
@@ -260,6 +257,7 @@ class ResponsePlanner {
             code.push_back(y);
             forced.push_back(y);
         };
+        if (const int64_t bit = writes(x); bit >= 0) standing[bit / 32] &= ~(1u << (bit % 32));
         switch (op) {
             case CLIFFT_OP_FRAME_CNOT:  // x_b ^= x_a, z_a ^= z_b
                 add(rx[a], rx[b]);
@@ -387,7 +385,7 @@ class ResponsePlanner {
             case CLIFFT_OP_POSTSELECT:
                 parity_into(idx, false, read_at[i]);
                 if (x.flags & CLIFFT_FLAG_EXPECTED_ONE) flip(constant, read_at[i]);
-                both(make(kLpPostselect, 0, read_at[i], add_row(written(i))));
+                both(make(kLpPostselect, 0, read_at[i], add_row(standing)));
                 break;
             case CLIFFT_OP_OBSERVABLE:
                 parity_into(idx, true, obs_bit(x.p.pauli.condition_idx));
