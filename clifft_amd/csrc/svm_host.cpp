@@ -12,6 +12,7 @@
 
 #include <immintrin.h>
 
+#include "svm_block_pool.h"
 #include "svm_internal.h"
 #include "svm_tree_plan.h"
 
@@ -1289,9 +1290,10 @@ void expand_rows(uint8_t* dst, const uint8_t* src, uint64_t rows, uint32_t n) {
 
 // Pinned host memory for one call's rows and records, from a pool shared by
 // all programs, streams and threads: a call takes a block and gives it back
-// when its stream has been waited for; at most kPinnedIdle bytes stay behind.
+// when its stream has been waited for.  The pool's bound has room for the
+// largest block and for small ones of other threads beside it.
 constexpr size_t kPinnedRows = (size_t)64 << 20;
-constexpr size_t kPinnedIdle = (size_t)64 << 20;
+constexpr size_t kPinnedIdle = (size_t)128 << 20;
 class PinnedBlock {
   public:
     PinnedBlock() = default;
@@ -1300,56 +1302,35 @@ class PinnedBlock {
     // the call has waited for its stream
     void done() { done_ = true; }
     ~PinnedBlock() {
-        if (!ptr_) return;
-        if (!done_) (void)hipDeviceSynchronize();  // the call failed: its kernel may still be writing
-        std::lock_guard<std::mutex> lock(mu());
-        if (done_ && idle_bytes() + bytes_ <= kPinnedIdle) {
-            idle().push_back({ptr_, bytes_});
-            idle_bytes() += bytes_;
+        if (!block_.ptr) return;
+        if (done_) {
+            for (const BlockPool::Block& b : pool().give(block_)) (void)hipHostFree(b.ptr);
         } else {
-            (void)hipHostFree(ptr_);
+            (void)hipDeviceSynchronize();  // the call failed: its kernel may still be writing
+            (void)hipHostFree(block_.ptr);
         }
     }
     // null where the memory cannot be had
     uint8_t* take(size_t bytes) {
         size_t want = (size_t)64 << 10;
         while (want < bytes) want <<= 1;
-        {
-            std::lock_guard<std::mutex> lock(mu());
-            auto& v = idle();
-            for (size_t i = 0; i < v.size(); ++i)
-                if (v[i].second == want) {
-                    ptr_ = v[i].first;
-                    bytes_ = want;
-                    v[i] = v.back();
-                    v.pop_back();
-                    idle_bytes() -= want;
-                    return static_cast<uint8_t*>(ptr_);
-                }
+        block_ = pool().take(want);
+        if (!block_.ptr) {
+            block_.bytes = want;
+            if (hipHostMalloc(&block_.ptr, want, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
+                (void)hipGetLastError();
+                block_ = BlockPool::Block();
+            }
         }
-        if (hipHostMalloc(&ptr_, want, hipHostMallocPortable | hipHostMallocMapped) != hipSuccess) {
-            (void)hipGetLastError();
-            ptr_ = nullptr;
-        }
-        bytes_ = ptr_ ? want : 0;
-        return static_cast<uint8_t*>(ptr_);
+        return static_cast<uint8_t*>(block_.ptr);
     }
 
   private:
-    void* ptr_ = nullptr;
-    size_t bytes_ = 0;
+    BlockPool::Block block_;
     bool done_ = false;
-    static std::mutex& mu() {
-        static std::mutex* m = new std::mutex;  // (never destroyed: calls may outlive static objects)
-        return *m;
-    }
-    static std::vector<std::pair<void*, size_t>>& idle() {
-        static auto* v = new std::vector<std::pair<void*, size_t>>;
-        return *v;
-    }
-    static size_t& idle_bytes() {
-        static size_t n = 0;
-        return n;
+    static BlockPool& pool() {
+        static BlockPool* p = new BlockPool(kPinnedIdle);  // (never destroyed: calls may outlive static objects)
+        return *p;
     }
 };
 
