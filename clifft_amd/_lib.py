@@ -99,6 +99,8 @@ SIGNATURES = {
     "clifft_svm_batch_destroy": (ctypes.c_int, [ctypes.c_void_p]),
     "clifft_svm_batch_set_tuning": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(BatchTuning)]),
     "clifft_svm_batch_get_tuning": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(BatchTuning)]),
+    "clifft_svm_batch_set_plan": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(BatchTuning), ctypes.c_uint32]),
+    "clifft_svm_batch_get_shared": (ctypes.c_int, [ctypes.c_void_p, ctypes.POINTER(ctypes.c_uint32)]),
     "clifft_svm_batch_info": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_uint32, ctypes.POINTER(BatchGroupInfo),
                                              ctypes.POINTER(ctypes.c_uint32)]),
     "clifft_svm_batch_time_groups": (ctypes.c_int, [ctypes.c_void_p, ctypes.c_uint32]),

@@ -105,7 +105,7 @@ class Batch:
     def groups(self) -> list:
         """The current plan's launch groups (kind: wave / lds / global / lane /
         gwave, one shot per wavefront on global amplitudes, / shared, many
-        shots per workgroup on shared states; set_tuning names the others)."""
+        shots per workgroup on shared states; the tuning names the others)."""
         n = ctypes.c_uint32()
         _lib.check(_lib.lib().clifft_svm_batch_info(self.handle, 0, None, ctypes.byref(n)), "batch_info")
         arr = (_lib.BatchGroupInfo * max(n.value, 1))()
@@ -130,25 +130,38 @@ class Batch:
         _lib.check(_lib.lib().clifft_svm_batch_group_times(self.handle, g, ms, ctypes.byref(n)), "batch_group_times")
         return [float(x) for x in ms[:n.value]]
 
+    def _plan(self, tuning) -> dict:
+        shared = ctypes.c_uint32()
+        _lib.check(_lib.lib().clifft_svm_batch_get_shared(self.handle, ctypes.byref(shared)), "batch_get_shared")
+        return {**{f: getattr(tuning, f) for f in _TUNING_FIELDS}, "shared": shared.value}
+
     @property
     def tuning(self) -> dict:
+        """The tuning fields, and `shared`: whether programs may share states (1) or not (0)."""
         t = _lib.BatchTuning()
         _lib.check(_lib.lib().clifft_svm_batch_get_tuning(self.handle, ctypes.byref(t)), "batch_get_tuning")
-        return {f: getattr(t, f) for f in _TUNING_FIELDS}
+        return self._plan(t)
 
     def set_tuning(self, **kw):
+        """Fields that are not named keep their values.  Naming some of them
+        (`concurrent` apart) names the groups, and turns `shared` off unless it
+        is named too; a whole tuning without it leaves it as it is."""
         cur = self.tuning
-        if set(kw) in ({"concurrent"}, set(_TUNING_FIELDS)) and all(cur[f] == int(v) for f, v in kw.items()):
-            return  # the plan stands as it is
+        named = set(kw) & set(_TUNING_FIELDS)
+        if "shared" not in kw and not named <= {"concurrent"} and named != set(_TUNING_FIELDS):
+            cur["shared"] = 0
         cur.update(kw)
         t = _lib.BatchTuning(*[int(cur[f]) for f in _TUNING_FIELDS])
-        _lib.check(_lib.lib().clifft_svm_batch_set_tuning(self.handle, ctypes.byref(t)), "batch_set_tuning")
+        _lib.check(_lib.lib().clifft_svm_batch_set_plan(self.handle, ctypes.byref(t), int(cur["shared"])),
+                   "batch_set_tuning")
 
     def tune(self, sample_shots: int = 0, stream=None) -> dict:
+        """The fastest tuning found, which is then set; set_tuning(**it) gives
+        another batch of these programs the same plan."""
         t = _lib.BatchTuning()
         _lib.check(_lib.lib().clifft_svm_batch_tune(self.handle, int(sample_shots), stream, ctypes.byref(t)),
                    "batch_tune")
-        return {f: getattr(t, f) for f in _TUNING_FIELDS}
+        return self._plan(t)
 
     def _seeds(self, seeds):
         return _u64(seeds if np.ndim(seeds) else [seeds] * self.n, self.n)

@@ -2265,7 +2265,7 @@ struct clifft_svm_batch {
     std::vector<clifft_svm_records> outs;
     uint32_t flags = 0;
     clifft_svm_batch_tuning tuning{};
-    bool shared = true;  // shared-state groups; off once the caller sets a tuning
+    bool shared = true;  // shared-state groups (clifft_svm_batch_set_plan)
     std::vector<BatchGroup> groups;
     std::vector<uint32_t> group_of;  // per program
     std::vector<ShotArgs> args;      // per program, for the current plan
@@ -2891,17 +2891,16 @@ int clifft_svm_batch_destroy(clifft_svm_batch* b) {
     return CLIFFT_OK;
 }
 
-int clifft_svm_batch_set_tuning(clifft_svm_batch* b, const clifft_svm_batch_tuning* t) {
+int clifft_svm_batch_set_plan(clifft_svm_batch* b, const clifft_svm_batch_tuning* t, uint32_t shared) {
     if (!b || !t) return fail(CLIFFT_E_INVALID, "null argument");
     int rc = batch_check_tuning(*t);
     if (rc) return rc;
-    clifft_svm_batch_tuning old = b->tuning;
+    if (shared > 1) return fail(CLIFFT_E_INVALID, "shared must be 0 or 1");
+    const clifft_svm_batch_tuning old = b->tuning;
     const bool old_shared = b->shared;
+    if (std::memcmp(t, &old, sizeof(old)) == 0 && old_shared == (shared != 0)) return CLIFFT_OK;
     b->tuning = *t;
-    // the tuning names every program's group, unless all it changes is their order
-    clifft_svm_batch_tuning same = *t;
-    same.concurrent = old.concurrent;
-    if (t->concurrent == old.concurrent || std::memcmp(&same, &old, sizeof(old)) != 0) b->shared = false;
+    b->shared = shared != 0;
     rc = batch_plan(b, ~0ull, library_stream());
     if (rc) {
         std::string msg = g_last_error;
@@ -2910,6 +2909,20 @@ int clifft_svm_batch_set_tuning(clifft_svm_batch* b, const clifft_svm_batch_tuni
         (void)batch_plan(b, ~0ull, library_stream());
         return fail(rc, msg);
     }
+    return CLIFFT_OK;
+}
+
+int clifft_svm_batch_set_tuning(clifft_svm_batch* b, const clifft_svm_batch_tuning* t) {
+    if (!b || !t) return fail(CLIFFT_E_INVALID, "null argument");
+    // a tuning that changes more than the groups' order names every program's group
+    clifft_svm_batch_tuning same = *t;
+    same.concurrent = b->tuning.concurrent;
+    return clifft_svm_batch_set_plan(b, t, b->shared && std::memcmp(&same, &b->tuning, sizeof(same)) == 0 ? 1u : 0u);
+}
+
+int clifft_svm_batch_get_shared(const clifft_svm_batch* b, uint32_t* shared) {
+    if (!b || !shared) return fail(CLIFFT_E_INVALID, "null argument");
+    *shared = b->shared ? 1u : 0u;
     return CLIFFT_OK;
 }
 

@@ -375,10 +375,10 @@ int clifft_svm_execute(clifft_svm_program* prog, clifft_svm_state* state);
  * LDS-resident amplitudes (<= lds_rank_max; split by team size), one
  * shot per wavefront with amplitudes in a global slice (<= gwave_rank_max),
  * or one shot per workgroup with amplitudes in a global slice
- * (global_threads per team).  Until clifft_svm_batch_set_tuning is called
- * for anything but a change of `concurrent`, programs that are faster with many shots per
- * workgroup sharing their states run that way, in groups of kind 5; a tuning
- * that was set names the group of every program.  A group's work items (a shot range of one program) are sorted by
+ * (global_threads per team).  Unless that is turned off (shared 0), programs
+ * that are faster with many shots per workgroup sharing their states run that
+ * way, in groups of kind 5, and the tuning names the groups of the others.
+ * A group's work items (a shot range of one program) are sorted by
  * descending estimated cost and drained by its teams from a device queue.
  * The groups run one after another on the caller's stream, or side by side
  * on the batch's own streams (concurrent = 1).
@@ -425,8 +425,16 @@ int clifft_svm_batch_create(clifft_svm_program* const* programs, const uint64_t*
                             uint32_t num_programs, uint32_t flags, const clifft_svm_records* outs,
                             clifft_svm_batch** out);
 int clifft_svm_batch_destroy(clifft_svm_batch* batch);
+/* A tuning that changes any field but `concurrent` names the group of every
+ * program: it turns shared states off.  One that changes nothing, or only
+ * `concurrent`, leaves them as they are. */
 int clifft_svm_batch_set_tuning(clifft_svm_batch* batch, const clifft_svm_batch_tuning* tuning);
 int clifft_svm_batch_get_tuning(const clifft_svm_batch* batch, clifft_svm_batch_tuning* tuning);
+/* The whole plan, as clifft_svm_batch_get_tuning and _get_shared returned it
+ * (from this batch, or another of the same programs, tuned or not): the tuning,
+ * and whether programs may share states (1, as a new batch has it) or not (0). */
+int clifft_svm_batch_set_plan(clifft_svm_batch* batch, const clifft_svm_batch_tuning* tuning, uint32_t shared);
+int clifft_svm_batch_get_shared(const clifft_svm_batch* batch, uint32_t* shared);
 /* The current plan: *num_groups groups, the first max_groups of them
  * described in info (may be NULL). */
 int clifft_svm_batch_info(const clifft_svm_batch* batch, uint32_t max_groups, clifft_svm_batch_group_info* info,
@@ -439,7 +447,8 @@ int clifft_svm_batch_time_groups(clifft_svm_batch* batch, uint32_t enable);
 int clifft_svm_batch_group_times(clifft_svm_batch* batch, uint32_t max_groups, float* ms, uint32_t* num_groups);
 /* Autotuner: times candidate tunings on the batch itself (each program
  * capped at `sample_shots` shots, outputs overwritten) with HIP events on
- * `stream`, keeps the fastest and returns it in `chosen` (may be NULL). */
+ * `stream`, keeps the fastest and returns it in `chosen` (may be NULL).  Shared
+ * states stay on or off as they are. */
 int clifft_svm_batch_tune(clifft_svm_batch* batch, uint64_t sample_shots, void* stream,
                           clifft_svm_batch_tuning* chosen);
 /* Every group's launch with per-program seeds (host array).  Asynchronous
