@@ -15,6 +15,7 @@
 #include "svm_block_pool.h"
 #include "svm_internal.h"
 #include "svm_tree_plan.h"
+#include "svm_tree_shape.h"
 
 using namespace csvm;
 
@@ -320,14 +321,8 @@ struct clifft_svm_program {
     int64_t kf_k = -1;
     // launch planning
     LaunchShape base_shape;
-    // shared-state executor: whether the program has a plan, its code length
-    // and response words, and (bits that may part the shots, rank) of every
-    // writing pass
-    bool tree = false;
-    bool tree_force = false;    // ... for forced records too
-    bool tree_choices = false;  // frame bits, not outcomes alone, part the shots
-    uint32_t tree_n = 0, tree_words = 0;
-    std::vector<std::pair<uint32_t, uint32_t>> tree_sizes;
+    TreeProfile tree;         // shared-state executor
+    bool tree_force = false;  // its plan does for forced records too
     // staging for host outputs (grown on demand)
     void* out_dev = nullptr;
     size_t out_dev_bytes = 0;
@@ -1097,137 +1092,15 @@ int finalize_shape(clifft_svm_program* p, LaunchShape& L, uint64_t shots, hipStr
     return CLIFFT_OK;
 }
 
-// Entries of each amplitude buffer of a team of `chunk` shots, and the
-// entries all its passes visit: a pass over N nodes of rank r writes N 2^r,
-// and before it at most min(chunk, 2^bits) groups of shots can have parted.
-struct TreeWork {
-    uint64_t elems = 1, visited = 0;
-};
-TreeWork tree_work(const clifft_svm_program* p, uint32_t chunk) {
-    TreeWork w;
-    for (const auto& sr : p->tree_sizes) {
-        const uint64_t nodes = sr.first < 12 ? std::min<uint64_t>(chunk, 1ull << sr.first) : chunk;
-        w.elems = std::max(w.elems, nodes << sr.second);
-        w.visited += nodes << sr.second;
-    }
-    return w;
-}
-
-// A team shape of the shared-state executor for `chunk` shots on `threads`
-// threads, each with room for `faults` forced faults; false where its tables
-// do not fit.
-bool tree_team(const clifft_svm_program* p, uint32_t threads, uint32_t chunk, uint32_t faults, LaunchShape& L) {
-    const TreeWork w = tree_work(p, chunk);
-    if (w.elems > (1ull << 31)) return false;
-    L = LaunchShape();
+LaunchShape tree_launch(const TreeShape& t) {
+    LaunchShape L;
     L.tree = true;
-    L.tree_chunk = chunk;
-    L.tree_elems = (uint32_t)w.elems;
-    L.block = threads;
-    L.lds_bytes = tree_team_lds(threads, chunk, p->tree_words + 5 * faults);
-    L.global_amps = w.elems > kTreeLdsElems;
-    if (!L.global_amps) L.lds_bytes += 32u * (size_t)w.elems;
-    return L.lds_bytes <= kTreeMaxDynLds;
-}
-
-// Estimated time (us) of one chunk on a team of shape L that shares its CU
-// with `teams` - 1 others: the walk, the passes' fixed part, and the entries
-// visited at what the wavefronts in flight reach (fitted to a sweep of team
-// sizes and chunks at peak 0 to 16 on one MI355X).
-double tree_team_us(const clifft_svm_program* p, const LaunchShape& L, double teams) {
-    const double waves = L.block / 64.0, per_simd = teams * waves / 4.0;
-    const double passes = p->tree_sizes.size();
-    const double walk = 5.0 + 0.35 * p->tree_n + (2.0 + 0.3 * std::log2(waves)) * passes;
-    const double visited = (double)tree_work(p, L.tree_chunk).visited;
-    const double entry = (L.global_amps ? 0.32e-3 : 0.25e-3) * std::max(512.0 / L.block, teams);
-    return walk * (1.0 + 0.18 * std::max(0.0, per_simd - 1.0)) + visited * entry;
-}
-// ... and of `shots` shots.
-double tree_cost(const clifft_svm_program* p, const LaunchShape& L, uint64_t shots) {
-    const double cus = device_info().num_cus;
-    const double teams = std::ceil((double)shots / L.tree_chunk);
-    const double per_cu = std::max(1.0, std::floor(std::min((double)kLdsBytes / (double)L.lds_bytes, 1024.0 / L.block)));
-    const double rounds = std::ceil(teams / (cus * per_cu));
-    const double visited = (double)tree_work(p, L.tree_chunk).visited;
-    // all teams together move 32 B an entry beyond the caches
-    const double bytes = L.global_amps ? std::min(teams, cus * per_cu) * 32.0 * (double)L.tree_elems : 0.0;
-    const double memory = bytes > 64e6 ? teams * visited * 32.0 / 4.0e6 : 0.0;
-    return std::max(rounds * tree_team_us(p, L, std::min(per_cu, std::ceil(teams / cus))), memory);
-}
-
-// Whether `shots` shots of a program are better off sharing their states.
-// Measured on one MI355X, per-shot executors against this one (100 to 300000
-// shots): surface-code memories 1.3 to 3 times faster to 49 qubits (25 rounds
-// of distance 3 with 300000 shots: the same), 14 to 470 times beyond 64;
-// 24-qubit Clifford+T at peak 8 to 14 2 to 300 times; random programs, whose
-// frames part almost every shot, 1.1 to 7 times from peak 8 on.  Below that a
-// program with a pass for every few instructions can lose (random, 300
-// instructions, 60 passes: 0.72 to 0.94 times at peak 1 to 7), so it has to
-// beat the lanes' walk, 0.48 us an instruction there.
-bool tree_better(const clifft_svm_program* p, uint64_t shots) {
-    if (!p->tree || shared_state_mode() == 0) return false;
-    if (shared_state_mode() == 2 || p->words > 1 || p->peak_rank >= 8) return true;
-    if (p->peak_rank == 7 && shots >= 4096) return true;
-    return 5.0 + 0.35 * p->tree_n + 2.0 * p->tree_sizes.size() <= 0.48 * (double)p->host_bc.size();
-}
-
-// Entries of a team's buffer up to which more shots may be put into it: where
-// frame bits part the shots, nodes grow with the shots at every rank, and one
-// such program would take tens of GiB of scratch (a batch of 512 took 99 GB
-// for the one with 2^24 entries a team); smaller chunks are the faster ones
-// there (random programs, peak 12 x 20000 shots: 5.6 ms at 2^18 entries a
-// team, 3.1 ms at 2^15).
-uint64_t tree_room(const clifft_svm_program* p) { return std::max<uint64_t>(1ull << 18, 1ull << p->peak_rank); }
-
-// The shared-state shape for a launch of `shots` shots: the team size and
-// the shots per team of the lowest estimate.  False: the program has no
-// plan, or the per-shot executors are faster.
-bool tree_shape(const clifft_svm_program* p, uint64_t shots, uint32_t faults, LaunchShape& best) {
-    if (!tree_better(p, shots)) return false;
-    double cost = 0.0;
-    bool found = false;
-    for (uint32_t threads : {64u, 128u, 256u, 512u, 1024u})
-        for (uint32_t chunk = threads; chunk >= 1; chunk /= 2) {
-            if (chunk > 2 * shots && chunk > 1) continue;
-            LaunchShape L;
-            if (!tree_team(p, threads, chunk, faults, L) || (chunk > 1 && L.tree_elems > tree_room(p))) continue;
-            const double c = tree_cost(p, L, shots);
-            if (!found || c < cost) {
-                best = L;
-                cost = c;
-                found = true;
-            }
-        }
-    return found;
-}
-
-// The shape in a batch, where other programs fill the device: the least
-// time of a compute unit, each team taking its part of one.  Two team sizes,
-// the larger alone for states in memory: each more is one more launch with
-// an end of its own (512 Clifford+T programs of peak 4 to 16, 1000 shots
-// each, all of 64 to 1024 threads: 766 us, 256 and 1024: 572, 1024 alone:
-// 552, 512 alone: 735); smaller ones where the records leave no room.
-bool tree_batch_shape(const clifft_svm_program* p, uint64_t shots, LaunchShape& best) {
-    if (!tree_better(p, std::max<uint64_t>(shots, 4096))) return false;
-    double cost = 0.0;
-    bool found = false;
-    for (uint32_t threads : {1024u, 256u, 64u}) {
-        if (found && threads == 64u) break;
-        for (uint32_t chunk = threads; chunk >= 1; chunk /= 2) {
-            if (chunk > 64 && chunk >= 2 * shots) continue;
-            LaunchShape L;
-            if (!tree_team(p, threads, chunk, 0, L) || (found && L.global_amps && threads < best.block)) continue;
-            if (chunk > 1 && L.tree_elems > tree_room(p)) continue;
-            const double part = std::max((double)threads / 1024.0, (double)L.lds_bytes / (double)kLdsBytes);
-            const double c = std::ceil((double)shots / chunk) * part * tree_team_us(p, L, 1.0 / part);
-            if (!found || c < cost) {
-                best = L;
-                cost = c;
-                found = true;
-            }
-        }
-    }
-    return found;
+    L.tree_chunk = t.chunk;
+    L.tree_elems = t.elems;
+    L.block = t.threads;
+    L.lds_bytes = t.lds;
+    L.global_amps = t.global;
+    return L;
 }
 
 int tree_finalize(LaunchShape& L, uint64_t shots, hipStream_t st, void** gscratch) {
@@ -1507,12 +1380,14 @@ int clifft_svm_program_create(const clifft_program_view* view, clifft_svm_progra
     TreePlan plan;
     if (!has_forced && shared_state_mode() != 0) {
         plan = TreePlanner(view, khist).run();
-        p->tree = plan.ok;
         p->tree_force = plan.can_force;
-        p->tree_choices = plan.choices;
-        p->tree_n = (uint32_t)plan.code.size();
-        p->tree_words = plan.words;
-        p->tree_sizes = plan.sizes;
+        p->tree.ok = plan.ok;
+        p->tree.code = (uint32_t)plan.code.size();
+        p->tree.words = plan.words;
+        p->tree.frame_words = view->words;
+        p->tree.peak_rank = view->peak_rank;
+        p->tree.instructions = (uint32_t)view->num_instructions;
+        p->tree.sizes = plan.sizes;
     }
     size_t o_trb = add(plan.code.data(), plan.code.size() * sizeof(clifft_instruction));
     size_t o_trf = add(plan.forced.data(), plan.forced.size() * sizeof(clifft_instruction));
@@ -1698,8 +1573,11 @@ static int run_shots(clifft_svm_program* p, uint64_t shots, uint64_t seed, uint3
         int rc;
         PinnedBlock block;
         bool pinned = false;
-        const bool tree = (mode != MODE_FORCED || p->tree_force) && tree_shape(p, n, kfault ? (uint32_t)p->kf_k : 0u, L);
+        TreeShape t;
+        const bool tree = (mode != MODE_FORCED || p->tree_force) &&
+                          tree_shape(p->tree, n, kfault ? (uint32_t)p->kf_k : 0u, device_info().num_cus, shared_state_mode(), t);
         if (tree) {
+            L = tree_launch(t);
             rc = tree_finalize(L, n, st, &gs);
         } else {
             L = kfault ? plan_shape(p, false, true) : p->base_shape;
@@ -2451,9 +2329,10 @@ int batch_group(clifft_svm_batch* b, uint64_t cap) {
     std::vector<BatchGroup> groups;
     std::vector<uint32_t> group_of(b->progs.size());
     std::vector<LaunchShape> shape(b->progs.size());
+    std::vector<TreeShape> tree(b->progs.size());
     for (size_t i = 0; i < b->progs.size(); ++i) {
-        if (b->shared && tree_batch_shape(b->progs[i], b->shots[i], shape[i])) {
-            // (grouped by kernel and team size below)
+        if (b->shared && tree_batch_shape(b->progs[i]->tree, b->shots[i], shared_state_mode(), tree[i])) {
+            shape[i] = tree_launch(tree[i]);  // (grouped by kernel and team size below)
         } else if (!batch_shape(b->progs[i], t, shape[i]))
             return fail(CLIFFT_E_UNSUPPORTED, "batch: the records of program " + std::to_string(i) +
                                                   " do not fit the LDS of a 256-thread team");
@@ -2520,7 +2399,7 @@ int batch_group(clifft_svm_batch* b, uint64_t cap) {
             group_of[i] = (uint32_t)gi;
             const uint64_t n = std::min<uint64_t>(b->shots[i], cap);
             const uint32_t step = g.L.tree ? shape[i].tree_chunk : chunk;
-            const double c = g.L.tree ? tree_team_us(b->progs[i], shape[i], 1.0) / step : shot_cost(b->progs[i], g.L);
+            const double c = g.L.tree ? tree_team_us(b->progs[i]->tree, tree[i], 1.0) / step : shot_cost(b->progs[i], g.L);
             if (g.L.tree) {
                 b->args[i].tree_chunk = shape[i].tree_chunk;
                 b->args[i].amp_elems = shape[i].tree_elems;
@@ -2566,12 +2445,12 @@ int batch_audit(const clifft_svm_batch* b) {
             if (it.shot_lo >= it.shot_hi || it.shot_hi > b->shots[it.prog])
                 return fail(CLIFFT_E_INVALID, where + "item shot range outside the program's shots");
             if (L.tree) {
-                LaunchShape one;
+                TreeShape one;
                 if (it.shot_hi - it.shot_lo > A.tree_chunk || A.tree_chunk > L.block || A.tree_chunk == 0)
                     return fail(CLIFFT_E_INVALID, where + "item over the team's shots");
-                if (!tree_team(p, L.block, A.tree_chunk, 0, one) || one.lds_bytes > L.lds_bytes || one.global_amps != L.global_amps)
+                if (!tree_team(p->tree, L.block, A.tree_chunk, 0, one) || one.lds > L.lds_bytes || one.global != L.global_amps)
                     return fail(CLIFFT_E_INVALID, where + "team tables exceed the launch's LDS");
-                if (A.amp_elems != one.tree_elems || one.tree_elems > g.amp_elems)
+                if (A.amp_elems != one.elems || one.elems > g.amp_elems)
                     return fail(CLIFFT_E_INVALID, where + "amplitude buffers exceed the team's");
                 continue;
             }

@@ -12,6 +12,7 @@
 #include "svm_device.h"
 #include "svm_adjoint_args.h"
 #include "svm_terms.h"
+#include "svm_tree_shape.h"
 
 namespace csvm {
 
@@ -56,15 +57,8 @@ hipError_t launch_batch_group(const LaunchShape& L, const BatchArgs* B, hipStrea
 // Zero n queue heads with a fill kernel (never a memset: graph-capturable).
 hipError_t clear_counters(uint32_t* counters, uint32_t n, hipStream_t st);
 
-// Amplitude buffers up to this many entries (each of a team's two) stay in LDS.
-constexpr uint64_t kTreeLdsElems = 2048;
-// Dynamic LDS limit of its kernels (less the queue head and the block-wide
-// "or" the runtime's library keeps in static LDS).
-constexpr size_t kTreeMaxDynLds = 158 * 1024;
-// Shared-state executor (svm_tree.hip): a shape's kernel, plain or batched,
-// and the LDS of a team apart from LDS amplitudes.
+// Shared-state executor (svm_tree.hip): a shape's kernel, plain or batched.
 const void* tree_kernel_fn(const LaunchShape& L, bool batch);
-uint32_t tree_team_lds(uint32_t threads, uint32_t chunk, uint32_t lane_words);
 // The launch arguments travel with the kernel's.
 hipError_t launch_tree(const LaunchShape& L, const DevProgram* P, const ShotArgs& A, hipStream_t st);
 

@@ -60,6 +60,4 @@ hipError_t launch_tree(const LaunchShape& L, const DevProgram* P, const ShotArgs
     return hipLaunchKernel(tree_kernel_fn(L, false), dim3(L.grid), dim3(L.block), args, L.lds_bytes, st);
 }
 
-uint32_t tree_team_lds(uint32_t threads, uint32_t chunk, uint32_t lane_words) { return tree_lds_bytes(threads, chunk, lane_words); }
-
 }  // namespace csvm

@@ -133,4 +133,22 @@ struct TreePass {
     double ez_tab[1u << kTreeMaxExpand][2];
 };
 
+struct TreeStage {  // the running pass's expansion products
+    double tab[1u << kTreeMaxExpand][2];
+};
+constexpr uint32_t kTreeParts = 128;  // partial sums of a pass with several per node
+
+// LDS of one team of `threads` threads and at most `chunk` shots: per-wave
+// response columns (64 x 4 B a word; with k-fault sampling also the fault
+// lists), two node tables (source node, choice word), per-node
+// sums, partial sums, two key bitmaps (and the rescale flag), the stage.
+constexpr uint32_t tree_flag_words(uint32_t chunk) { return (chunk + 1u) / 2u + 2u; }
+constexpr uint32_t tree_lds_bytes(uint32_t threads, uint32_t chunk, uint32_t lane_words) {
+    uint32_t b = (threads >> 6) * lane_words * 256u;
+    b += (16u * chunk + 15u) / 16u * 16u;  // 4 x u32 tables
+    b += 16u * chunk + 16u * kTreeParts;
+    b += (8u * tree_flag_words(chunk) + 15u) / 16u * 16u;
+    return b + (uint32_t)sizeof(TreeStage);
+}
+
 }  // namespace csvm

@@ -50,7 +50,6 @@ struct TreePlan {
     std::vector<TreeChan> chans;
     std::vector<uint32_t> chan_rows;  // two words an entry
     bool can_force = false;           // every record slot is visible and written once
-    bool choices = false;             // some kTreeChoice parts the shots
     // per writing pass: bits that may part the shots before it, and its rank
     std::vector<std::pair<uint32_t, uint32_t>> sizes;
 };
@@ -317,7 +316,6 @@ class ResponsePlanner {
                 word(y, 1, x.p.classical.classical_idx);  // place in the choice word
                 read_frame(x, read_at[i]);
                 both(y);
-                out.choices = true;
                 break;
             }
             case kTreeNode: {  // the axes' bits become those of the state the node leaves

@@ -1,0 +1,174 @@
+// svm_tree_shape.h -- the shared-state executor's rules of dispatch: whether a
+// program's shots are better off there, on teams of how many threads, and with
+// how many shots a team.  Host code without HIP.
+#pragma once
+
+#include <stddef.h>
+#include <stdint.h>
+
+#include <algorithm>
+#include <cmath>
+#include <utility>
+#include <vector>
+
+#include "svm_tree_args.h"
+
+namespace csvm {
+
+// Amplitude buffers up to this many entries (each of a team's two) stay in LDS.
+constexpr uint64_t kTreeLdsElems = 2048;
+// Dynamic LDS limit of its kernels (less the queue head and the block-wide
+// "or" the runtime's library keeps in static LDS), and a compute unit's LDS.
+constexpr size_t kTreeMaxDynLds = 158 * 1024;
+constexpr size_t kTreeCuLds = 160 * 1024;
+
+// What the rules know of a program.
+struct TreeProfile {
+    bool ok = false;            // it has a plan
+    uint32_t code = 0;          // the plan's instructions
+    uint32_t words = 0;         // of a shot's response
+    uint32_t frame_words = 1;   // 64 qubits each
+    uint32_t peak_rank = 0;
+    uint32_t instructions = 0;  // the program's
+    // (bits that may part the shots, rank) of every writing pass
+    std::vector<std::pair<uint32_t, uint32_t>> sizes;
+};
+
+struct TreeShape {
+    uint32_t threads = 0, chunk = 0;  // of a team: threads, shots
+    uint32_t elems = 0;               // entries of each of its two buffers
+    size_t lds = 0;                   // bytes
+    bool global = false;              // the buffers are in memory, not in LDS
+};
+
+// Entries of each amplitude buffer of a team of `chunk` shots, and the
+// entries all its passes visit: a pass over N nodes of rank r writes N 2^r,
+// and before it at most min(chunk, 2^bits) groups of shots can have parted.
+struct TreeWork {
+    uint64_t elems = 1, visited = 0;
+};
+inline TreeWork tree_work(const TreeProfile& p, uint32_t chunk) {
+    TreeWork w;
+    for (const auto& sr : p.sizes) {
+        const uint64_t nodes = sr.first < 12 ? std::min<uint64_t>(chunk, 1ull << sr.first) : chunk;
+        w.elems = std::max(w.elems, nodes << sr.second);
+        w.visited += nodes << sr.second;
+    }
+    return w;
+}
+
+// The shape of a team of `chunk` shots on `threads` threads, each with room
+// for `faults` forced faults; false where its tables do not fit.
+inline bool tree_team(const TreeProfile& p, uint32_t threads, uint32_t chunk, uint32_t faults, TreeShape& s) {
+    const TreeWork w = tree_work(p, chunk);
+    if (w.elems > (1ull << 31)) return false;
+    s.threads = threads;
+    s.chunk = chunk;
+    s.elems = (uint32_t)w.elems;
+    s.lds = tree_lds_bytes(threads, chunk, p.words + 5 * faults);
+    s.global = w.elems > kTreeLdsElems;
+    if (!s.global) s.lds += 32u * (size_t)w.elems;
+    return s.lds <= kTreeMaxDynLds;
+}
+
+// Estimated time (us) of one chunk on a team of shape s that shares its CU
+// with `teams` - 1 others: the walk, the passes' fixed part, and the entries
+// visited at what the wavefronts in flight reach (fitted to a sweep of team
+// sizes and chunks at peak 0 to 16 on one MI355X).
+inline double tree_team_us(const TreeProfile& p, const TreeShape& s, double teams) {
+    const double waves = s.threads / 64.0, per_simd = teams * waves / 4.0;
+    const double passes = (double)p.sizes.size();
+    const double walk = 5.0 + 0.35 * p.code + (2.0 + 0.3 * std::log2(waves)) * passes;
+    const double visited = (double)tree_work(p, s.chunk).visited;
+    const double entry = (s.global ? 0.32e-3 : 0.25e-3) * std::max(512.0 / s.threads, teams);
+    return walk * (1.0 + 0.18 * std::max(0.0, per_simd - 1.0)) + visited * entry;
+}
+// ... and of `shots` shots on `cus` compute units.
+inline double tree_cost(const TreeProfile& p, const TreeShape& s, uint64_t shots, double cus) {
+    const double teams = std::ceil((double)shots / s.chunk);
+    const double per_cu = std::max(1.0, std::floor(std::min((double)kTreeCuLds / (double)s.lds, 1024.0 / s.threads)));
+    const double rounds = std::ceil(teams / (cus * per_cu));
+    const double visited = (double)tree_work(p, s.chunk).visited;
+    // all teams together move 32 B an entry beyond the caches
+    const double bytes = s.global ? std::min(teams, cus * per_cu) * 32.0 * (double)s.elems : 0.0;
+    const double memory = bytes > 64e6 ? teams * visited * 32.0 / 4.0e6 : 0.0;
+    return std::max(rounds * tree_team_us(p, s, std::min(per_cu, std::ceil(teams / cus))), memory);
+}
+
+// Whether `shots` shots of a program are better off sharing their states.
+// Measured on one MI355X, per-shot executors against this one (100 to 300000
+// shots): surface-code memories 1.3 to 3 times faster to 49 qubits (25 rounds
+// of distance 3 with 300000 shots: the same), 14 to 470 times beyond 64;
+// 24-qubit Clifford+T at peak 8 to 14 2 to 300 times; random programs, whose
+// frames part almost every shot, 1.1 to 7 times from peak 8 on.  Below that a
+// program with a pass for every few instructions can lose (random, 300
+// instructions, 60 passes: 0.72 to 0.94 times at peak 1 to 7), so it has to
+// beat the lanes' walk, 0.48 us an instruction there.
+// `mode`: CLIFFT_SHARED_STATE (0 never, 2 wherever there is a plan).
+inline bool tree_better(const TreeProfile& p, uint64_t shots, int mode) {
+    if (!p.ok || mode == 0) return false;
+    if (mode == 2 || p.frame_words > 1 || p.peak_rank >= 8) return true;
+    if (p.peak_rank == 7 && shots >= 4096) return true;
+    return 5.0 + 0.35 * p.code + 2.0 * (double)p.sizes.size() <= 0.48 * (double)p.instructions;
+}
+
+// Entries of a team's buffer up to which more shots may be put into it: where
+// frame bits part the shots, nodes grow with the shots at every rank, and one
+// such program would take tens of GiB of scratch (a batch of 512 took 99 GB
+// for the one with 2^24 entries a team); smaller chunks are the faster ones
+// there (random programs, peak 12 x 20000 shots: 5.6 ms at 2^18 entries a
+// team, 3.1 ms at 2^15).
+inline uint64_t tree_room(const TreeProfile& p) { return std::max<uint64_t>(1ull << 18, 1ull << p.peak_rank); }
+
+// The shape for a launch of `shots` shots: the team size and the shots per
+// team of the lowest estimate.  False: the program has no plan, or the
+// per-shot executors are faster.
+inline bool tree_shape(const TreeProfile& p, uint64_t shots, uint32_t faults, uint32_t cus, int mode, TreeShape& best) {
+    if (!tree_better(p, shots, mode)) return false;
+    double cost = 0.0;
+    bool found = false;
+    for (uint32_t threads : {64u, 128u, 256u, 512u, 1024u})
+        for (uint32_t chunk = threads; chunk >= 1; chunk /= 2) {
+            if (chunk > 2 * shots && chunk > 1) continue;
+            TreeShape s;
+            if (!tree_team(p, threads, chunk, faults, s) || (chunk > 1 && s.elems > tree_room(p))) continue;
+            const double c = tree_cost(p, s, shots, cus);
+            if (!found || c < cost) {
+                best = s;
+                cost = c;
+                found = true;
+            }
+        }
+    return found;
+}
+
+// The shape in a batch, where other programs fill the device: the least
+// time of a compute unit, each team taking its part of one.  Two team sizes,
+// the larger alone for states in memory: each more is one more launch with
+// an end of its own (512 Clifford+T programs of peak 4 to 16, 1000 shots
+// each, all of 64 to 1024 threads: 766 us, 256 and 1024: 572, 1024 alone:
+// 552, 512 alone: 735); smaller ones where the records leave no room.
+inline bool tree_batch_shape(const TreeProfile& p, uint64_t shots, int mode, TreeShape& best) {
+    if (!tree_better(p, std::max<uint64_t>(shots, 4096), mode)) return false;
+    double cost = 0.0;
+    bool found = false;
+    for (uint32_t threads : {1024u, 256u, 64u}) {
+        if (found && threads == 64u) break;
+        for (uint32_t chunk = threads; chunk >= 1; chunk /= 2) {
+            if (chunk > 64 && chunk >= 2 * shots) continue;
+            TreeShape s;
+            if (!tree_team(p, threads, chunk, 0, s) || (found && s.global && threads < best.threads)) continue;
+            if (chunk > 1 && s.elems > tree_room(p)) continue;
+            const double part = std::max((double)threads / 1024.0, (double)s.lds / (double)kTreeCuLds);
+            const double c = std::ceil((double)shots / chunk) * part * tree_team_us(p, s, 1.0 / part);
+            if (!found || c < cost) {
+                best = s;
+                cost = c;
+                found = true;
+            }
+        }
+    }
+    return found;
+}
+
+}  // namespace csvm
