@@ -22,6 +22,13 @@ constexpr uint64_t kTreeLdsElems = 2048;
 constexpr size_t kTreeMaxDynLds = 158 * 1024;
 constexpr size_t kTreeCuLds = 160 * 1024;
 
+constexpr uint32_t kTreeChunks = 11;  // shots a team: powers of two to 1024
+
+// Entries of each amplitude buffer of a team, and those all its passes visit.
+struct TreeWork {
+    uint64_t elems = 1, visited = 0;
+};
+
 // What the rules know of a program.
 struct TreeProfile {
     bool ok = false;            // it has a plan
@@ -30,9 +37,26 @@ struct TreeProfile {
     uint32_t frame_words = 1;   // 64 qubits each
     uint32_t peak_rank = 0;
     uint32_t instructions = 0;  // the program's
-    // (bits that may part the shots, rank) of every writing pass
-    std::vector<std::pair<uint32_t, uint32_t>> sizes;
+    uint32_t operations = 0;    // those that do not only move frames
+    uint32_t passes = 0;        // that write
+    TreeWork work[kTreeChunks];
+
+    // from (bits that may part the shots, rank) of every writing pass: over N
+    // nodes of rank r it writes N 2^r, and before it at most min(chunk, 2^bits)
+    // groups of shots can have parted
+    void set_passes(const std::vector<std::pair<uint32_t, uint32_t>>& sizes) {
+        passes = (uint32_t)sizes.size();
+        for (uint32_t e = 0; e < kTreeChunks; ++e) {
+            work[e] = TreeWork();
+            for (const auto& sr : sizes) {
+                const uint64_t entries = 1ull << (std::min(e, sr.first) + sr.second);
+                work[e].elems = std::max(work[e].elems, entries);
+                work[e].visited += entries;
+            }
+        }
+    }
 };
+inline const TreeWork& tree_work(const TreeProfile& p, uint32_t chunk) { return p.work[__builtin_ctz(chunk)]; }
 
 struct TreeShape {
     uint32_t threads = 0, chunk = 0;  // of a team: threads, shots
@@ -41,26 +65,10 @@ struct TreeShape {
     bool global = false;              // the buffers are in memory, not in LDS
 };
 
-// Entries of each amplitude buffer of a team of `chunk` shots, and the
-// entries all its passes visit: a pass over N nodes of rank r writes N 2^r,
-// and before it at most min(chunk, 2^bits) groups of shots can have parted.
-struct TreeWork {
-    uint64_t elems = 1, visited = 0;
-};
-inline TreeWork tree_work(const TreeProfile& p, uint32_t chunk) {
-    TreeWork w;
-    for (const auto& sr : p.sizes) {
-        const uint64_t nodes = sr.first < 12 ? std::min<uint64_t>(chunk, 1ull << sr.first) : chunk;
-        w.elems = std::max(w.elems, nodes << sr.second);
-        w.visited += nodes << sr.second;
-    }
-    return w;
-}
-
 // The shape of a team of `chunk` shots on `threads` threads, each with room
 // for `faults` forced faults; false where its tables do not fit.
 inline bool tree_team(const TreeProfile& p, uint32_t threads, uint32_t chunk, uint32_t faults, TreeShape& s) {
-    const TreeWork w = tree_work(p, chunk);
+    const TreeWork& w = tree_work(p, chunk);
     if (w.elems > (1ull << 31)) return false;
     s.threads = threads;
     s.chunk = chunk;
@@ -77,13 +85,21 @@ inline bool tree_team(const TreeProfile& p, uint32_t threads, uint32_t chunk, ui
 // sizes and chunks at peak 0 to 16 on one MI355X).
 inline double tree_team_us(const TreeProfile& p, const TreeShape& s, double teams) {
     const double waves = s.threads / 64.0, per_simd = teams * waves / 4.0;
-    const double passes = (double)p.sizes.size();
-    const double walk = 5.0 + 0.35 * p.code + (2.0 + 0.3 * std::log2(waves)) * passes;
+    const double walk = 5.0 + 0.35 * p.code + (2.0 + 0.3 * std::log2(waves)) * p.passes;
     const double visited = (double)tree_work(p, s.chunk).visited;
     const double entry = (s.global ? 0.32e-3 : 0.25e-3) * std::max(512.0 / s.threads, teams);
     return walk * (1.0 + 0.18 * std::max(0.0, per_simd - 1.0)) + visited * entry;
 }
-// ... and of `shots` shots on `cus` compute units.
+// ... and of `shots` shots on `cus` compute units: the teams' own time or, where
+// it is longer, that of the memory, which is the same for many shapes.  Two small
+// terms decide between those: a tenth of the lesser time, for teams that are
+// slow by themselves also use the memory badly, and a twentieth of the memory's
+// for each halving of the threads below 512.  (The longer time alone took 64
+// threads and the most shots where frame bits part them.  All shapes of 84
+// calls, peak 8 to 19 and 100 to 30000 shots: its choice took 1.45 times the best
+// one's time on average, 2.8 at most and up to 1.7 times the per-shot
+// executors'; with both terms 1.09, 1.67 and never that.  The sum of both times:
+// 1.15, and more where nothing parts the shots.)
 inline double tree_cost(const TreeProfile& p, const TreeShape& s, uint64_t shots, double cus) {
     const double teams = std::ceil((double)shots / s.chunk);
     const double per_cu = std::max(1.0, std::floor(std::min((double)kTreeCuLds / (double)s.lds, 1024.0 / s.threads)));
@@ -91,25 +107,38 @@ inline double tree_cost(const TreeProfile& p, const TreeShape& s, uint64_t shots
     const double visited = (double)tree_work(p, s.chunk).visited;
     // all teams together move 32 B an entry beyond the caches
     const double bytes = s.global ? std::min(teams, cus * per_cu) * 32.0 * (double)s.elems : 0.0;
-    const double memory = bytes > 64e6 ? teams * visited * 32.0 / 4.0e6 : 0.0;
-    return std::max(rounds * tree_team_us(p, s, std::min(per_cu, std::ceil(teams / cus))), memory);
+    const double small = 1.0 + 0.05 * std::max(0.0, std::log2(512.0 / s.threads));
+    const double memory = bytes > 64e6 ? small * teams * visited * 32.0 / 4.0e6 : 0.0;
+    const double own = rounds * tree_team_us(p, s, std::min(per_cu, std::ceil(teams / cus)));
+    return std::max(own, memory) + 0.1 * std::min(own, memory);
+}
+
+// Estimated time (us) of `shots` shots on the per-shot executors at peak 8 to
+// 10: one shot's walk, 1 us an operation, until the wavefronts are more than
+// the device holds at once (18 programs of 150 to 700 instructions, 1 to 30000
+// shots; an operation is any instruction but a frame one).
+inline double per_shot_us(const TreeProfile& p, uint64_t shots) {
+    const double many = (double)shots * (p.peak_rank > 9 ? 1.6e-3 : 0.8e-3);
+    return 20.0 + (double)p.operations * std::max(1.0, many);
 }
 
 // Whether `shots` shots of a program are better off sharing their states.
 // Measured on one MI355X, per-shot executors against this one (100 to 300000
 // shots): surface-code memories 1.3 to 3 times faster to 49 qubits (25 rounds
 // of distance 3 with 300000 shots: the same), 14 to 470 times beyond 64;
-// 24-qubit Clifford+T at peak 8 to 14 2 to 300 times; random programs, whose
-// frames part almost every shot, 1.1 to 7 times from peak 8 on.  Below that a
+// 24-qubit Clifford+T at peak 8 to 14 2 to 300 times, with noise that parts the
+// shots at their T gates 1.04 to 25 times at peak 8 to 19; random programs, whose
+// frames part almost every shot, 1.1 to 14 times from peak 11 on.  Below that a
 // program with a pass for every few instructions can lose (random, 300
 // instructions, 60 passes: 0.72 to 0.94 times at peak 1 to 7), so it has to
-// beat the lanes' walk, 0.48 us an instruction there.
+// beat the lanes' walk, 0.48 us an instruction there, and at peak 8 to 10
+// per_shot_us (tree_shape).
 // `mode`: CLIFFT_SHARED_STATE (0 never, 2 wherever there is a plan).
 inline bool tree_better(const TreeProfile& p, uint64_t shots, int mode) {
     if (!p.ok || mode == 0) return false;
     if (mode == 2 || p.frame_words > 1 || p.peak_rank >= 8) return true;
     if (p.peak_rank == 7 && shots >= 4096) return true;
-    return 5.0 + 0.35 * p.code + 2.0 * (double)p.sizes.size() <= 0.48 * (double)p.instructions;
+    return 5.0 + 0.35 * p.code + 2.0 * p.passes <= 0.48 * (double)p.instructions;
 }
 
 // Entries of a team's buffer up to which more shots may be put into it: where
@@ -139,6 +168,10 @@ inline bool tree_shape(const TreeProfile& p, uint64_t shots, uint32_t faults, ui
                 found = true;
             }
         }
+    // (random, 400 instructions, 95 passes, peak 10: 375 us against 310 at 1 to
+    // 100 shots, 400 against 520 at 1000)
+    if (found && mode == 1 && faults == 0 && p.frame_words == 1 && p.peak_rank >= 8 && p.peak_rank <= 10)
+        return 1.1 * cost <= per_shot_us(p, shots);
     return found;
 }
 

@@ -1,0 +1,32 @@
+// The shared-state executor's rules of dispatch on a program's plan, for the
+// CPU test.
+#include "svm_tree_plan.h"
+#include "svm_tree_shape.h"
+
+using namespace csvm;
+
+static bool profile(const clifft_program_view* v, const int32_t* khist, TreeProfile& p) {
+    const std::vector<int32_t> kh(khist, khist + v->num_instructions);
+    const TreePlan plan = TreePlanner(v, kh).run();
+    p.ok = plan.ok;
+    p.code = (uint32_t)plan.code.size();
+    p.words = plan.words;
+    p.frame_words = v->words;
+    p.peak_rank = v->peak_rank;
+    p.instructions = (uint32_t)v->num_instructions;
+    for (uint64_t i = 0; i < v->num_instructions; ++i) p.operations += v->bytecode[i].opcode > CLIFFT_OP_FRAME_SWAP;
+    p.set_passes(plan.sizes);
+    return plan.ok;
+}
+
+// out: threads, shots a team, entries a buffer, LDS bytes, buffers in memory;
+// 0: on the per-shot executors, -1: no plan
+extern "C" int shape(const clifft_program_view* v, const int32_t* khist, uint64_t shots, uint32_t faults, uint32_t cus, int mode,
+                     int batch, uint64_t* out) {
+    TreeProfile p;
+    if (!profile(v, khist, p)) return -1;
+    TreeShape s;
+    if (!(batch ? tree_batch_shape(p, shots, mode, s) : tree_shape(p, shots, faults, cus, mode, s))) return 0;
+    out[0] = s.threads, out[1] = s.chunk, out[2] = s.elems, out[3] = s.lds, out[4] = s.global;
+    return 1;
+}
