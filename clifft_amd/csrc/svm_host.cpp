@@ -2330,9 +2330,11 @@ int batch_group(clifft_svm_batch* b, uint64_t cap) {
     std::vector<BatchGroup> groups;
     std::vector<uint32_t> group_of(b->progs.size());
     std::vector<LaunchShape> shape(b->progs.size());
-    std::vector<TreeShape> tree(b->progs.size());
+    std::vector<const TreeProfile*> profiles;
+    for (const clifft_svm_program* p : b->progs) profiles.push_back(&p->tree);
+    const std::vector<TreeShape> tree = tree_batch(profiles, b->shots, device_info().num_cus, b->shared ? shared_state_mode() : 0);
     for (size_t i = 0; i < b->progs.size(); ++i) {
-        if (b->shared && tree_batch_shape(b->progs[i]->tree, b->shots[i], shared_state_mode(), tree[i])) {
+        if (tree[i].threads) {
             shape[i] = tree_launch(tree[i]);  // (grouped by kernel and team size below)
         } else if (!batch_shape(b->progs[i], t, shape[i]))
             return fail(CLIFFT_E_UNSUPPORTED, "batch: the records of program " + std::to_string(i) +

@@ -175,33 +175,78 @@ inline bool tree_shape(const TreeProfile& p, uint64_t shots, uint32_t faults, ui
     return found;
 }
 
-// The shape in a batch, where other programs fill the device: the least
-// time of a compute unit, each team taking its part of one.  Two team sizes,
-// the larger alone for states in memory: each more is one more launch with
-// an end of its own (512 Clifford+T programs of peak 4 to 16, 1000 shots
+// Estimated time (us) of a batch's `total` shots one shot a lane, to peak 6, if
+// all its programs were like this one: one walk, or what the lanes in flight
+// give (fitted to batches of 8 to 256 random programs, 100 to 8000 shots each,
+// at peak 3 to 6: 0.7 to 1.2 times the measured time).
+inline double batch_lanes_us(const TreeProfile& p, uint64_t total, double cus) {
+    const double frames = (double)p.instructions - p.operations, amps = std::ldexp(1.0, (int)p.peak_rank);
+    const double walk = 0.1 * frames + (1.0 + 0.05 * amps) * p.operations;
+    const double shot = 0.25e-3 * frames + (0.3e-3 + 0.12e-3 * amps) * p.operations;
+    return std::max(walk, (double)total / cus * shot);
+}
+
+// The shape in a batch of `total` shots, of which `shots` are this program's,
+// and its estimated time (us): the least if the others are like it.  Teams beyond
+// what a compute unit holds at once wait for each other; fewer leave compute
+// units idle, and shots are then better spread over more teams (8 random
+// programs of peak 8 with 1000 shots, in one team each 3.6 ms, 0.58 so).  Two team
+// sizes, the larger alone for states in memory: each more is one more launch
+// with an end of its own (512 Clifford+T programs of peak 4 to 16, 1000 shots
 // each, all of 64 to 1024 threads: 766 us, 256 and 1024: 572, 1024 alone:
 // 552, 512 alone: 735); smaller ones where the records leave no room.
-inline bool tree_batch_shape(const TreeProfile& p, uint64_t shots, int mode, TreeShape& best) {
-    if (!tree_better(p, std::max<uint64_t>(shots, 4096), mode)) return false;
-    double cost = 0.0;
-    bool found = false;
+// Negative: none.
+inline double tree_batch_shape(const TreeProfile& p, uint64_t shots, uint64_t total, double cus, TreeShape& best) {
+    double cost = -1.0;
     for (uint32_t threads : {1024u, 256u, 64u}) {
-        if (found && threads == 64u) break;
+        if (cost >= 0.0 && threads == 64u) break;
         for (uint32_t chunk = threads; chunk >= 1; chunk /= 2) {
             if (chunk > 64 && chunk >= 2 * shots) continue;
             TreeShape s;
-            if (!tree_team(p, threads, chunk, 0, s) || (found && s.global && threads < best.threads)) continue;
+            if (!tree_team(p, threads, chunk, 0, s) || (cost >= 0.0 && s.global && threads < best.threads)) continue;
             if (chunk > 1 && s.elems > tree_room(p)) continue;
             const double part = std::max((double)threads / 1024.0, (double)s.lds / (double)kTreeCuLds);
-            const double c = std::ceil((double)shots / chunk) * part * tree_team_us(p, s, 1.0 / part);
-            if (!found || c < cost) {
+            const double teams = std::ceil((double)shots / chunk) * ((double)total / (double)shots) / cus;  // a compute unit
+            const double c = std::max(1.0, teams * part) * tree_team_us(p, s, std::clamp(teams, 1.0, 1.0 / part));
+            if (cost < 0.0 || c < cost) {
                 best = s;
                 cost = c;
-                found = true;
             }
         }
     }
-    return found;
+    return cost;
+}
+
+// The programs of a batch that share their states, each with its shape (0
+// threads: not).  From peak 7 on, and beyond 64 qubits, all that have a plan do;
+// the others all or none, by their estimates together: a lane group for a few
+// of them takes its whole walk beside the teams' (random programs of peak 6, 64
+// with 1000 shots: 1.15 ms with three of them on lanes, 0.61 with none).  Where
+// the device is full the estimate of the teams is low by 1.3 (peak 5, 256 random
+// programs with 1000 shots: 1.5 ms on teams, 1.25 on lanes).
+inline std::vector<TreeShape> tree_batch(const std::vector<const TreeProfile*>& progs, const std::vector<uint64_t>& shots,
+                                         double cus, int mode) {
+    std::vector<TreeShape> out(progs.size());
+    if (mode == 0) return out;
+    uint64_t total = 0;
+    for (uint64_t n : shots) total += n;
+    auto low = [&](const TreeProfile& p) { return mode == 1 && p.frame_words == 1 && p.peak_rank <= 6; };
+    double teams = 0.0, lanes = 0.0;
+    for (size_t i = 0; i < progs.size(); ++i) {
+        const TreeProfile& p = *progs[i];
+        if (!p.ok || shots[i] == 0) continue;
+        TreeShape s;
+        const double c = tree_batch_shape(p, shots[i], total, cus, s);
+        if (c < 0.0) continue;
+        out[i] = s;
+        if (!low(p)) continue;
+        teams += c * (double)shots[i];
+        lanes += batch_lanes_us(p, total, cus) * (double)shots[i];
+    }
+    if (1.3 * teams > lanes)
+        for (size_t i = 0; i < progs.size(); ++i)
+            if (low(*progs[i])) out[i] = TreeShape();
+    return out;
 }
 
 }  // namespace csvm

@@ -29,15 +29,15 @@ def lib(tmp_path_factory):
                     "-o", str(so)], check=True, timeout=120)
     L = ctypes.CDLL(str(so))
     L.shape.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_uint64, ctypes.c_uint32, ctypes.c_uint32, ctypes.c_int,
-                        ctypes.c_int, ctypes.c_void_p]
+                        ctypes.c_uint32, ctypes.c_void_p]
     return L
 
 
-def shape(lib, p, shots, faults=0, mode=1, batch=0):
+def shape(lib, p, shots, faults=0, mode=1, copies=0):
     """(threads, shots a team, entries, LDS bytes, in memory), or None on the
     per-shot executors"""
     out, kh, v = np.zeros(5, np.uint64), ranks(p), p.view()
-    n = lib.shape(ctypes.addressof(v), kh.ctypes.data, shots, faults, CUS, mode, batch, out.ctypes.data)
+    n = lib.shape(ctypes.addressof(v), kh.ctypes.data, shots, faults, CUS, mode, copies, out.ctypes.data)
     return tuple(int(x) for x in out) if n == 1 else None
 
 
@@ -78,13 +78,39 @@ def test_noiseless_programs_share(lib, t, layers):
         assert shape(lib, p, shots) is not None
 
 
+@pytest.mark.parametrize("peak,shots", [(7, 1000), (8, 1000), (9, 1000), (10, 1000)])
+def test_small_batches_use_the_whole_device(lib, peak, shots):
+    """8 programs in one team each left 248 of 256 compute units idle: 1.4 to
+    3.3 times as slow as the per-shot executors."""
+    threads, chunk = shape(lib, parting(peak, 300), shots, copies=8)[:2]
+    assert 8 * -(-shots // chunk) >= CUS
+    assert shape(lib, parting(peak, 300), shots, copies=512)[1] > chunk
+
+
+@pytest.mark.parametrize("peak,shots,copies,shared", [
+    (3, 1000, 256, False), (3, 8000, 64, False),  # up to 1.8 times as slow
+    (3, 100, 8, True), (6, 100, 8, True), (6, 8000, 64, True)])  # 1.3 to 4 times as fast
+def test_low_ranks_in_batches(lib, peak, shots, copies, shared):
+    p = parting(peak, 300, u_nodes=False)
+    assert (shape(lib, p, shots, copies=copies) is not None) == shared
+    assert shape(lib, p, shots, mode=2, copies=copies) is not None and shape(lib, p, shots, mode=0, copies=copies) is None
+
+
+@pytest.mark.parametrize("distance", [3, 5])
+def test_memories_share_in_batches(lib, distance):
+    from clifft_amd.compiler import compile as ccompile
+    from memory_circuit import memory_text
+    p = ccompile(memory_text(distance, distance, 0.002))
+    assert all(shape(lib, p, s, copies=n) is not None for s in (100, 10000, 1000000) for n in (1, 16, 512))
+
+
 @pytest.mark.parametrize("seed", range(24))
 def test_every_shape_keeps_the_limits(lib, seed):
     p = random_program(5000 + seed, num_qubits=(9, 20, 33, 90)[seed % 4], peak=(1, 6, 9, 14)[seed % 4],
                        length=(40, 200, 400)[seed % 3], u_nodes=seed % 2 == 0)
     for shots in (1, 3, 64, 1000, 1 << 20):
-        for faults, batch in ((0, 0), (8, 0), (64, 0), (0, 1)):
-            s = shape(lib, p, shots, faults, mode=2, batch=batch)
+        for faults, copies in ((0, 0), (8, 0), (64, 0), (0, 1), (0, 500)):
+            s = shape(lib, p, shots, faults, mode=2, copies=copies)
             if s is None:
                 assert faults  # (the fault lists leave no room)
                 continue
