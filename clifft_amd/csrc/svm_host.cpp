@@ -1962,8 +1962,7 @@ static int kfault_tables(clifft_svm_program* p, uint32_t k, hipStream_t st, cons
                     const double denom = dp[(size_t)i * stride + j];
                     const double hit =
                         j == n - i ? 1.0 : denom > 0.0 ? (w[i] * dp[(size_t)(i + 1) * stride + j - 1]) / denom : 0.0;
-                    // x 2^-53 < hit for the draw's top 53 bits x (scaling by 2^53 is exact)
-                    below[(size_t)i * stride + j] = (uint64_t)std::ceil(std::min(hit, 1.0) * 0x1.0p53);
+                    below[(size_t)i * stride + j] = draw_limit(hit);
                 }
         }
         auto* base = static_cast<uint8_t*>(p->kf_dev);

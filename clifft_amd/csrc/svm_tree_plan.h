@@ -38,6 +38,12 @@
 
 namespace csvm {
 
+// The draws x 2^-53 (x: 53 random bits) that are below p are those with x below
+// this; none where p is not a number (a quotient of sums that overflowed).
+inline uint64_t draw_limit(double p) {
+    return p > 0.0 ? (uint64_t)std::ceil(std::min(p, 1.0) * 0x1.0p53) : 0;  // (scaling by 2^53 is exact)
+}
+
 struct TreePlan {
     bool ok = false;
     std::vector<clifft_instruction> code, forced;  // the sampled and the forced walk
