@@ -45,9 +45,9 @@ def _run_all(cmds):
     for cmd in cmds:
         print(" ".join(cmd), flush=True)
         procs.append((cmd, subprocess.Popen(cmd)))
-    for cmd, p in procs:
-        if p.wait():
-            raise subprocess.CalledProcessError(p.returncode, cmd)
+    failed = [(p.returncode, cmd) for cmd, p in procs if p.wait()]  # (all have ended)
+    if failed:
+        raise subprocess.CalledProcessError(*failed[0])
 
 
 def build_svm(verbose: bool = True) -> str:

@@ -712,7 +712,7 @@ class TreePlanner {
         for (uint32_t b = 0; b < r; ++b) q[b] = 1u << b;
         return q;
     }
-    void emit_pass(uint32_t) { emit(blank(kTreePass)); }
+    void emit_pass() { emit(blank(kTreePass)); }
     // Write the oldest expansions, in source order, until a pass can read
     // through the rest.
     void trim_expansions() {
@@ -729,7 +729,7 @@ class TreePlanner {
             }
             out.sizes.push_back({splits, p.r});
             out.passes.push_back(p);
-            emit_pass(0);
+            emit_pass();
             r0 += (uint32_t)n;
             exps.erase(exps.begin(), exps.begin() + n);
         }
@@ -754,7 +754,7 @@ class TreePlanner {
         trim_expansions();
         const Turns rest = turns;
         const uint32_t r = rank(), p = add_pass(TREE_COPY, identity(r));
-        emit_pass(p);
+        emit_pass();
         consumed(p, identity(r), rest);
     }
     // x ^= px where popc(x & pm) is odd (its own inverse)
@@ -786,7 +786,7 @@ class TreePlanner {
         const std::vector<uint32_t> q = pair_on(rank(), a);  // its own inverse
         Turns t;
         const uint32_t p = add_pass(type, q, &t);
-        emit_pass(p);
+        emit_pass();
         consumed(p, q, t.below(rank() - 1).on(q));
         return p;
     }
@@ -915,7 +915,7 @@ class TreePlanner {
                 const uint32_t p = add_pass(TREE_U4, q, &t);
                 out.passes[p].node = in.p.u.cp_idx;
                 out.passes[p].choice = (uint32_t)c;
-                emit_pass(p);
+                emit_pass();
                 std::vector<uint32_t> stored(r);
                 for (uint32_t l = 0; l < r; ++l) stored[__builtin_ctz(q[l])] = 1u << l;
                 consumed(p, stored, t.below(r - 2).on(stored));
