@@ -1384,10 +1384,7 @@ int clifft_svm_program_create(const clifft_program_view* view, clifft_svm_progra
         p->tree.ok = plan.ok;
         p->tree.code = (uint32_t)plan.code.size();
         p->tree.words = plan.words;
-        p->tree.frame_words = view->words;
-        p->tree.peak_rank = view->peak_rank;
-        p->tree.instructions = (uint32_t)view->num_instructions;
-        for (uint64_t i = 0; i < view->num_instructions; ++i) p->tree.operations += view->bytecode[i].opcode > CLIFFT_OP_FRAME_SWAP;
+        p->tree.set_program(view);
         p->tree.set_passes(plan.sizes);
     }
     size_t o_trb = add(plan.code.data(), plan.code.size() * sizeof(clifft_instruction));

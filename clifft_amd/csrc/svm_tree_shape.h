@@ -11,6 +11,7 @@
 #include <utility>
 #include <vector>
 
+#include "clifft_svm.h"
 #include "svm_tree_args.h"
 
 namespace csvm {
@@ -38,8 +39,23 @@ struct TreeProfile {
     uint32_t peak_rank = 0;
     uint32_t instructions = 0;  // the program's
     uint32_t operations = 0;    // those that do not only move frames
+    uint32_t arrays = 0;        // those on amplitudes
+    double noise = 0.0;         // events a shot has on average
     uint32_t passes = 0;        // that write
     TreeWork work[kTreeChunks];
+
+    void set_program(const clifft_program_view* v) {
+        frame_words = v->words;
+        peak_rank = v->peak_rank;
+        instructions = (uint32_t)v->num_instructions;
+        noise = v->num_sites ? v->hazards[v->num_sites - 1] : 0.0;
+        for (uint64_t i = 0; i < v->num_instructions; ++i) {
+            const uint32_t op = v->bytecode[i].opcode;
+            operations += op > CLIFFT_OP_FRAME_SWAP;
+            arrays += (op >= CLIFFT_OP_ARRAY_CNOT && op <= CLIFFT_OP_EXPAND_ROT) || op == CLIFFT_OP_MEAS_ACTIVE_DIAGONAL ||
+                      op == CLIFFT_OP_MEAS_ACTIVE_INTERFERE || op == CLIFFT_OP_SWAP_MEAS_INTERFERE || op == CLIFFT_OP_EXP_VAL;
+        }
+    }
 
     // from (bits that may part the shots, rank) of every writing pass: over N
     // nodes of rank r it writes N 2^r, and before it at most min(chunk, 2^bits)
@@ -122,6 +138,17 @@ inline double per_shot_us(const TreeProfile& p, uint64_t shots) {
     return 20.0 + (double)p.operations * std::max(1.0, many);
 }
 
+// Estimated time (us) of `shots` shots one a lane, to peak 6: one walk, or what
+// the lanes in flight give (46 random, memory and Clifford+T programs of 100 to
+// 3300 instructions, 1 to 300000 shots: 0.6 to 1.4 times the measured time).
+inline double lanes_us(const TreeProfile& p, uint64_t shots, double cus) {
+    const double frames = (double)p.instructions - p.operations, rest = (double)p.operations - p.arrays;
+    const double amps = std::ldexp((double)p.arrays, (int)p.peak_rank);
+    const double walk = 24.0 + 0.032 * frames + 0.27 * rest + 0.6 * p.arrays + 0.0125 * amps;
+    const double shot = 0.028 + 0.45e-3 * p.operations + 0.2e-3 * amps + 0.03 * p.noise;
+    return std::max(1.1 * walk, (double)shots / cus * shot);
+}
+
 // Whether `shots` shots of a program are better off sharing their states.
 // Measured on one MI355X, per-shot executors against this one (100 to 300000
 // shots): surface-code memories 1.3 to 3 times faster to 49 qubits (25 rounds
@@ -131,8 +158,8 @@ inline double per_shot_us(const TreeProfile& p, uint64_t shots) {
 // frames part almost every shot, 1.1 to 14 times from peak 11 on.  Below that a
 // program with a pass for every few instructions can lose (random, 300
 // instructions, 60 passes: 0.72 to 0.94 times at peak 1 to 7), so it has to
-// beat the lanes' walk, 0.48 us an instruction there, and at peak 8 to 10
-// per_shot_us (tree_shape).
+// beat the lanes' walk, 0.48 us an instruction there, with more shots lanes_us,
+// and at peak 8 to 10 per_shot_us (tree_shape).
 // `mode`: CLIFFT_SHARED_STATE (0 never, 2 wherever there is a plan).
 inline bool tree_better(const TreeProfile& p, uint64_t shots, int mode) {
     if (!p.ok || mode == 0) return false;
@@ -168,11 +195,19 @@ inline bool tree_shape(const TreeProfile& p, uint64_t shots, uint32_t faults, ui
                 found = true;
             }
         }
+    if (!found || mode != 1 || faults || p.frame_words > 1) return found;
     // (random, 400 instructions, 95 passes, peak 10: 375 us against 310 at 1 to
     // 100 shots, 400 against 520 at 1000)
-    if (found && mode == 1 && faults == 0 && p.frame_words == 1 && p.peak_rank >= 8 && p.peak_rank <= 10)
-        return 1.1 * cost <= per_shot_us(p, shots);
-    return found;
+    if (p.peak_rank >= 8 && p.peak_rank <= 10) return 1.1 * cost <= per_shot_us(p, shots);
+    // The estimate leaves out the noise events and, where every compute unit has
+    // several teams, is the lower the smaller these are: by 1.4 at 64 threads,
+    // high by 1.25 at 1024 (the factors here are a tenth less).  (Random, 300
+    // instructions, 300000 shots, peak 1 to 5: 1.3 to 3 times as slow as lanes.)
+    if (p.peak_rank <= 6 && shots >= 4096) {
+        const double low = best.threads == 64 ? 1.25 : best.threads == 128 ? 1.05 : best.threads == 256 ? 0.95 : best.threads == 512 ? 0.8 : 0.7;
+        return low * cost + 0.045 * p.noise * (double)shots / cus <= lanes_us(p, shots, cus);
+    }
+    return true;
 }
 
 // Estimated time (us) of a batch's `total` shots one shot a lane, to peak 6, if

@@ -11,10 +11,7 @@ static bool profile(const clifft_program_view* v, const int32_t* khist, TreeProf
     p.ok = plan.ok;
     p.code = (uint32_t)plan.code.size();
     p.words = plan.words;
-    p.frame_words = v->words;
-    p.peak_rank = v->peak_rank;
-    p.instructions = (uint32_t)v->num_instructions;
-    for (uint64_t i = 0; i < v->num_instructions; ++i) p.operations += v->bytecode[i].opcode > CLIFFT_OP_FRAME_SWAP;
+    p.set_program(v);
     p.set_passes(plan.sizes);
     return plan.ok;
 }

@@ -78,6 +78,23 @@ def test_noiseless_programs_share(lib, t, layers):
         assert shape(lib, p, shots) is not None
 
 
+@pytest.mark.parametrize("peak", [1, 2, 3, 4, 5])
+def test_many_shots_of_many_passes_run_on_lanes(lib, peak):
+    """300 instructions, a pass for every six: 1.35 to 3.1 times as slow at
+    300000 shots, as fast or faster at a few."""
+    p = random_program(40 + peak, num_qubits=peak + 10, peak=peak, length=300, u_nodes=False, exp_vals=False)
+    assert shape(lib, p, 300000) is None and shape(lib, p, 300000, mode=2) is not None
+    assert shape(lib, p, 1) is not None
+
+
+@pytest.mark.parametrize("distance,rounds", [(3, 3), (3, 25), (5, 5), (5, 25)])
+def test_many_shots_of_memories_share(lib, distance, rounds):
+    from clifft_amd.compiler import compile as ccompile
+    from memory_circuit import memory_text
+    p = ccompile(memory_text(distance, rounds, 0.002))
+    assert all(shape(lib, p, s) is not None for s in (1, 5000, 200000))
+
+
 @pytest.mark.parametrize("peak,shots", [(7, 1000), (8, 1000), (9, 1000), (10, 1000)])
 def test_small_batches_use_the_whole_device(lib, peak, shots):
     """8 programs in one team each left 248 of 256 compute units idle: 1.4 to
