@@ -3127,21 +3127,6 @@ bool adjoint_op_ok(uint8_t op) {
     }
 }
 
-// Terms up to which their sums are taken instead of the state: half of what
-// makes the two equal.  Measured on one MI355X at 16 and at 512 angle vectors
-// (rank 6 to 14, one X probe over all axes whose terms double with every
-// second rotation): the terms take 6 us + 5.5 ns a term and parameter (1064
-// terms of 16 parameters 110 us, 4148 of 26 540), the sweeps 2 to 2.2 us an
-// operation to rank 8, 3.6 and 5.6 at rank 10 and 12 (16 vectors) and 9.5 to
-// 39 at rank 14 (16 and 512 vectors).
-size_t term_limit(const clifft_svm_program* p, uint32_t num_params) {
-    size_t ops = 0;
-    for (const clifft_instruction& in : p->host_bc) ops += in.opcode > CLIFFT_OP_FRAME_SWAP;
-    const double sweeps = (double)ops * (2.0 + std::ldexp(0.4e-3, (int)p->peak_rank));
-    const double even = (sweeps - 6.0) / (5.5e-3 * std::max(1.0, (double)num_params));
-    return (size_t)std::clamp(0.5 * even, 0.0, 65536.0);
-}
-
 int adjoint_ensure(void** ptr, size_t* cur, size_t bytes) {
     if (bytes <= *cur) return CLIFFT_OK;
     if (*ptr) {
@@ -3188,9 +3173,11 @@ int clifft_svm_adjoint_create(clifft_svm_program* p, const uint32_t* param_instr
     a->num_params = num_params;
     const size_t o_ps = align_up(std::max<size_t>(n, 1) * 4, 256);
     const size_t o_args = o_ps + align_up(psign.size() * 8, 256);
+    size_t ops = 0;
+    for (const clifft_instruction& in : p->host_bc) ops += in.opcode > CLIFFT_OP_FRAME_SWAP;
     const TermPlan plan = TermPlanner(p->host_bc.data(), n, p->khist.data(), slot_of.data(), num_params, p->num_ev, p->ev_x.data(),
                                       p->ev_z.data(), p->ev_sign.data(), p->words)
-                              .run(term_limit(p, num_params));
+                              .run(term_limit(ops, p->peak_rank, num_params));
     const size_t o_terms = o_args + align_up(kAdjArgSlots * sizeof(AdjArgs), 256);
     const size_t o_before = o_terms + align_up(plan.terms.size() * sizeof(AdjTerm), 256);
     const size_t o_first = o_before + align_up(plan.before.size() * 8, 256);

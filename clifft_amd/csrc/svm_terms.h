@@ -17,6 +17,7 @@
 #include <stdint.h>
 #include <string.h>
 
+#include <algorithm>
 #include <cmath>
 #include <vector>
 
@@ -47,6 +48,20 @@ struct TermArgs {
     uint64_t batch;
     uint32_t num_params, num_ev, num_terms, pad;
 };
+
+// Terms up to which their sums are taken instead of the state: half of what
+// makes the two equal.  Measured on one MI355X at 16 and at 512 angle vectors
+// (rank 6 to 14, one X probe over all axes whose terms double with every
+// second rotation; random programs of rank 1 to 12): the terms take 6 us and
+// 20 ns a term + 5.5 ns a term and parameter (1064 terms of 16 parameters
+// 110 us, 4148 of 26 540, 2845 of 4 171), the sweeps of `ops` operations 2 to
+// 2.2 us an operation to rank 8, 3.6 and 5.6 at rank 10 and 12 (16 vectors) and
+// 9.5 to 39 at rank 14 (16 and 512 vectors).
+inline size_t term_limit(size_t ops, uint32_t rank, uint32_t num_params) {
+    const double sweeps = (double)ops * (2.0 + std::ldexp(0.4e-3, (int)rank));
+    const double even = (sweeps - 6.0) / (20e-3 + 5.5e-3 * num_params);
+    return (size_t)std::min(std::max(0.5 * even, 0.0), 65536.0);
+}
 
 struct TermPlan {
     bool ok = false;

@@ -6,14 +6,17 @@ no number of parameters bounds."""
 
 from __future__ import annotations
 
+import ctypes
+import os
 import shutil
+import subprocess
 import time
 
 import numpy as np
 import pytest
 
 from clifft_amd import program as P
-from test_terms import lib, run  # noqa: F401  (lib: the compiled planner)
+from test_terms import ROOT, lib, run  # noqa: F401  (lib: the compiled planner)
 
 pytestmark = pytest.mark.skipif(shutil.which("g++") is None, reason="no host C++ compiler")
 
@@ -48,3 +51,17 @@ def test_few_paths_are_still_taken(lib, turns):  # noqa: F811
     p, slots, angles = vanishing(turns)
     n, ev, grad = run(lib, p, slots, angles, limit=1000)
     assert n == 0 and ev[0] == 0.0 and not grad.any()
+
+
+@pytest.mark.parametrize("ops,rank,params,terms,sums", [
+    (97, 1, 4, 2845, False),  # few parameters: 171 us against the sweeps' 153
+    (106, 2, 3, 2030, True), (210, 8, 14, 1586, True), (48, 16, 16, 32, True)])  # 117 : 122, 148 : 305, 9 : 6100
+def test_limit_of_terms(tmp_path, ops, rank, params, terms, sums):
+    so = tmp_path / "liblimit.so"
+    subprocess.run(["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-I", os.path.join(ROOT, "include"), "-I",
+                    os.path.join(ROOT, "clifft_amd", "csrc"), os.path.join(ROOT, "tests", "cpp", "term_limit_check.cpp"),
+                    "-o", str(so)], check=True, timeout=120)
+    limit = ctypes.CDLL(str(so)).limit
+    limit.restype, limit.argtypes = ctypes.c_uint64, [ctypes.c_uint64, ctypes.c_uint32, ctypes.c_uint32]
+    assert (terms <= limit(ops, rank, params)) == sums
+    assert 0 <= limit(0, rank, params) <= limit(ops, rank, params) <= 65536 and limit(10 ** 9, rank, params) == 65536
