@@ -586,10 +586,10 @@ def main():
     if os.path.exists(tpath):
         with open(tpath) as f:
             tr = json.load(f)
-        w = tr["workloads"].get(args.workload)
-        # (the profiles of the per-shot kernels, which ran these programs before)
+        # (the per-shot kernels run these programs only where they are forced)
         per_shot = os.environ.get("CLIFFT_SHARED_STATE") == "0"
-        if w and w["shots"] == shots and w["kernel"].startswith("tree_kernel") != per_shot:
+        w = tr["workloads"].get(args.workload if per_shot else args.workload + "_shared")
+        if w and w["shots"] == shots:
             traffic = (w["fetch_kib"] * tr["fetch_scale"] + w["write_kib"] * tr["write_scale"]) * 1024.0
     rec_bytes = nb(prog.num_measurements) + nb(prog.num_detectors) + nb(prog.num_observables)
     bytes_per_launch = (info["bytes_per_shot"] + rec_bytes) * shots

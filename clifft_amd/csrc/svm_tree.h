@@ -13,8 +13,9 @@
 // every node and sums both probabilities; each shot then draws its own
 // outcome from its own stream, and the (node, outcome) pairs that occur
 // become the next nodes.  Nothing is approximated or carried over from one
-// launch to the next: a shot's record is the one the per-shot executors
-// give it.
+// launch to the next: a shot draws what it draws on the per-shot executors,
+// against probabilities that agree to rounding (the order of a node's sums
+// depends on the team and on how many nodes there are).
 //
 // Why.  The per-shot tiers move the whole state once or twice per
 // measurement and shot and dispatch every opcode per shot.  Here a level
@@ -24,17 +25,18 @@
 // opcode is dispatched once per 64 shots.
 //
 // Measured on one MI355X (per call, before -> after; before: the per-shot
-// tiers): 24-qubit Clifford+T, peak 10 x 20000 shots 2304 -> 58 us, peak 16 x
-// 2000 1805 -> 276 us; 34 qubits, peak 25 x 64 shots 752 -> 67 ms; 512
-// programs x 1000 shots 54.4 -> 0.67 ms; surface-code memories, distance 3 x
-// 10^6 shots 162 -> 128 us, distance 7 (97 qubits) x 20000 7770 -> 92 us,
-// distance 5 with 4 forced faults x 20000 3940 -> 530 us (360 of them copies
-// to the host).  With a frame per shot and every opcode walked (the same
-// executor before the response) peak 10 took 82 us, its walk 35 of them.
+// tiers): 24-qubit Clifford+T, peak 10 x 20000 shots 2304 -> 55 us, peak 16 x
+// 2000 1805 -> 278 us; 34 qubits, peak 25 x 64 shots 752 -> 66.5 ms; 512
+// programs x 1000 shots 54.4 -> 0.64 to 0.70 ms; surface-code memories, distance
+// 3 x 10^6 shots 162 -> 126 us, distance 7 (97 qubits) x 20000 7770 -> 85 us,
+// distance 5 with 4 forced faults x 20000 3940 -> 210 us (135 of kernel).  With
+// a frame per shot and every opcode walked (the same executor before the
+// response) peak 10 took 82 us, its walk 35 of them.
 // What bounds it: memories, the dependent loads of a noise event (about 1.3
 // us for the slowest of 64 shots) and the draws; up to peak 12 the passes'
 // fixed part, about 2 us a measurement; from peak 14 their entries (16
-// instructions and 32 bytes each).
+// instructions and 32 bytes each).  128 VGPRs, 30 to 35 of them spilled: teams
+// of 1024 threads allow no more.
 //
 // The array work itself is planned on the host (svm_tree_plan.h): each pass
 // gathers through a linear map over GF(2), so a lane's source index is the
