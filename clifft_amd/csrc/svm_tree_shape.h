@@ -107,15 +107,21 @@ inline double tree_team_us(const TreeProfile& p, const TreeShape& s, double team
     return walk * (1.0 + 0.18 * std::max(0.0, per_simd - 1.0)) + visited * entry;
 }
 // ... and of `shots` shots on `cus` compute units: the teams' own time or, where
-// it is longer, that of the memory, which is the same for many shapes.  Two small
-// terms decide between those: a tenth of the lesser time, for teams that are
-// slow by themselves also use the memory badly, and a twentieth of the memory's
-// for each halving of the threads below 512.  (The longer time alone took 64
-// threads and the most shots where frame bits part them.  All shapes of 84
-// calls, peak 8 to 19 and 100 to 30000 shots: its choice took 1.45 times the best
-// one's time on average, 2.8 at most and up to 1.7 times the per-shot
-// executors'; with both terms 1.09, 1.67 and never that.  The sum of both times:
-// 1.15, and more where nothing parts the shots.)
+// it is longer, that of the memory, which is the same for many shapes.  A tenth
+// of the lesser time decides between those, for teams that are slow by
+// themselves also use the memory badly.  Where that is the same too, the
+// memory's time counts 0.3 % more for each halving of the threads below 512
+// and, without noise, 0.6 % for each doubling of a team's shots: all frame bits
+// count as parting these, but noise parts few of them, so that more shots are
+// fewer nodes, while outcomes and coins part them all, and smaller buffers
+// leave no compute unit idle.  (All shapes of 169 calls, peak 8 to 20, 100 to
+// 80000 shots, with noise, with resets and with neither.  The longer time alone
+// took 64 threads and the most shots where frame bits part them: 1.37 times the
+// best shape's time on average, 2.8 at most, and up to 1.7 times the per-shot
+// executors'.  With these terms 1.05 and 1.5, and nowhere more than 1 % above
+// the longer time alone.  5 % for the threads and nothing for the shots: 1.08,
+// and 22 % above where 11054 shots with resets were put 64 to a team, 512
+// threads each, so that 83 compute units had none.)
 inline double tree_cost(const TreeProfile& p, const TreeShape& s, uint64_t shots, double cus) {
     const double teams = std::ceil((double)shots / s.chunk);
     const double per_cu = std::max(1.0, std::floor(std::min((double)kTreeCuLds / (double)s.lds, 1024.0 / s.threads)));
@@ -123,8 +129,9 @@ inline double tree_cost(const TreeProfile& p, const TreeShape& s, uint64_t shots
     const double visited = (double)tree_work(p, s.chunk).visited;
     // all teams together move 32 B an entry beyond the caches
     const double bytes = s.global ? std::min(teams, cus * per_cu) * 32.0 * (double)s.elems : 0.0;
-    const double small = 1.0 + 0.05 * std::max(0.0, std::log2(512.0 / s.threads));
-    const double memory = bytes > 64e6 ? small * teams * visited * 32.0 / 4.0e6 : 0.0;
+    const double halvings = std::max(0.0, std::log2(512.0 / s.threads)), doublings = std::log2((double)s.chunk);
+    const double ties = 1.0 + 0.003 * halvings + (p.noise > 0.0 ? 0.0 : 0.006) * doublings;
+    const double memory = bytes > 64e6 ? ties * teams * visited * 32.0 / 4.0e6 : 0.0;
     const double own = rounds * tree_team_us(p, s, std::min(per_cu, std::ceil(teams / cus)));
     return std::max(own, memory) + 0.1 * std::min(own, memory);
 }
