@@ -107,33 +107,43 @@ inline double tree_team_us(const TreeProfile& p, const TreeShape& s, double team
     return walk * (1.0 + 0.18 * std::max(0.0, per_simd - 1.0)) + visited * entry;
 }
 // ... and of `shots` shots on `cus` compute units: the teams' own time or, where
-// it is longer, that of the memory, which is the same for many shapes.  A tenth
-// of the lesser time decides between those, for teams that are slow by
-// themselves also use the memory badly.  Where that is the same too, the
-// memory's time counts 0.3 % more for each halving of the threads below 512
-// and, without noise, 0.6 % for each doubling of a team's shots: all frame bits
-// count as parting these, but noise parts few of them, so that more shots are
-// fewer nodes, while outcomes and coins part them all, and smaller buffers
-// leave no compute unit idle.  (All shapes of 169 calls, peak 8 to 20, 100 to
-// 80000 shots, with noise, with resets and with neither.  The longer time alone
-// took 64 threads and the most shots where frame bits part them: 1.37 times the
+// it is longer, that of the memory, which is the same for many shapes; `tie`
+// then decides between those (0: the teams' own is the longer).
+struct TreeTime {
+    double us = 0.0, tie = 0.0;
+};
+
+// The tie: shapes whose teams are the faster by themselves use the memory the
+// better, so 5.5 % of the difference is taken off (the last round without its
+// idle places, which the memory fills).  Where that is the same too, the memory's
+// time counts 0.2 % more for each halving of the threads below 512 and, without
+// noise, 0.26 % for each doubling of a team's shots: all frame bits count as
+// parting these, but noise parts few of them, so that more shots are fewer nodes,
+// while outcomes and coins part them all, and smaller buffers leave no compute
+// unit idle.  (All shapes of 222 calls, peak 8 to 21, 100 to 80000 shots, with
+// noise, with resets and with neither.  The first shape of the least time, 64
+// threads and the most shots where frame bits part them, took 1.35 times the
 // best shape's time on average, 2.8 at most, and up to 1.7 times the per-shot
-// executors'.  With these terms 1.05 and 1.5, and nowhere more than 1 % above
-// the longer time alone.  5 % for the threads and nothing for the shots: 1.08,
-// and 22 % above where 11054 shots with resets were put 64 to a team, 512
-// threads each, so that 83 compute units had none.)
-inline double tree_cost(const TreeProfile& p, const TreeShape& s, uint64_t shots, double cus) {
+// executors'.  With the tie 1.06 and 2.0, and nowhere above the first shape; at
+// 4.5 to 9 %, all three in proportion, by 1 % at most.  If the tie also takes
+// shapes whose own time is longer, up to 20 % above it where both times are
+// alike.  5 % for the threads and nothing for the shots: 22 % above it where
+// 11054 shots with resets were put 64 to a team, so that 83 compute units had
+// none.)
+inline TreeTime tree_time(const TreeProfile& p, const TreeShape& s, uint64_t shots, double cus) {
     const double teams = std::ceil((double)shots / s.chunk);
     const double per_cu = std::max(1.0, std::floor(std::min((double)kTreeCuLds / (double)s.lds, 1024.0 / s.threads)));
-    const double rounds = std::ceil(teams / (cus * per_cu));
+    const double rounds = std::max(1.0, teams / (cus * per_cu));
     const double visited = (double)tree_work(p, s.chunk).visited;
     // all teams together move 32 B an entry beyond the caches
     const double bytes = s.global ? std::min(teams, cus * per_cu) * 32.0 * (double)s.elems : 0.0;
+    const double memory = bytes > 64e6 ? teams * visited * 32.0 / 4.0e6 : 0.0;
+    const double team = tree_team_us(p, s, std::min(per_cu, std::ceil(teams / cus)));
+    const double own = std::ceil(rounds) * team;
+    if (own >= memory) return {own, 0.0};
     const double halvings = std::max(0.0, std::log2(512.0 / s.threads)), doublings = std::log2((double)s.chunk);
-    const double ties = 1.0 + 0.003 * halvings + (p.noise > 0.0 ? 0.0 : 0.006) * doublings;
-    const double memory = bytes > 64e6 ? ties * teams * visited * 32.0 / 4.0e6 : 0.0;
-    const double own = rounds * tree_team_us(p, s, std::min(per_cu, std::ceil(teams / cus)));
-    return std::max(own, memory) + 0.1 * std::min(own, memory);
+    const double even = memory * (1.0 + 0.002 * halvings + (p.noise > 0.0 ? 0.0 : 0.0026) * doublings);
+    return {memory, even - 0.055 * (even - rounds * team)};
 }
 
 // Estimated time (us) of `shots` shots on the per-shot executors at peak 8 to
@@ -184,34 +194,36 @@ inline bool tree_better(const TreeProfile& p, uint64_t shots, int mode) {
 inline uint64_t tree_room(const TreeProfile& p) { return std::max<uint64_t>(1ull << 18, 1ull << p.peak_rank); }
 
 // The shape for a launch of `shots` shots: the team size and the shots per
-// team of the lowest estimate.  False: the program has no plan, or the
-// per-shot executors are faster.
+// team of the least time or, if that is the memory's, of the least tie.  False:
+// the program has no plan, or the per-shot executors are faster.
 inline bool tree_shape(const TreeProfile& p, uint64_t shots, uint32_t faults, uint32_t cus, int mode, TreeShape& best) {
     if (!tree_better(p, shots, mode)) return false;
-    double cost = 0.0;
+    TreeTime least, tied;
+    TreeShape even;
     bool found = false;
     for (uint32_t threads : {64u, 128u, 256u, 512u, 1024u})
         for (uint32_t chunk = threads; chunk >= 1; chunk /= 2) {
             if (chunk > 2 * shots && chunk > 1) continue;
             TreeShape s;
             if (!tree_team(p, threads, chunk, faults, s) || (chunk > 1 && s.elems > tree_room(p))) continue;
-            const double c = tree_cost(p, s, shots, cus);
-            if (!found || c < cost) {
-                best = s;
-                cost = c;
-                found = true;
-            }
+            const TreeTime t = tree_time(p, s, shots, cus);
+            if (!found || t.us < least.us) best = s, least = t;
+            if (t.tie > 0.0 && (tied.tie == 0.0 || t.tie < tied.tie)) even = s, tied = t;
+            found = true;
         }
+    if (least.tie > 0.0) best = even, least = tied;
+    const double cost = least.us;
     if (!found || mode != 1 || faults || p.frame_words > 1) return found;
     // (random, 400 instructions, 95 passes, peak 10: 375 us against 310 at 1 to
     // 100 shots, 400 against 520 at 1000)
     if (p.peak_rank >= 8 && p.peak_rank <= 10) return 1.1 * cost <= per_shot_us(p, shots);
     // The estimate leaves out the noise events and, where every compute unit has
     // several teams, is the lower the smaller these are: by 1.4 at 64 threads,
-    // high by 1.25 at 1024 (the factors here are a tenth less).  (Random, 300
-    // instructions, 300000 shots, peak 1 to 5: 1.3 to 3 times as slow as lanes.)
+    // high by 1.25 at 1024, but not in memory (the others' factors here are a
+    // tenth less).  (Random, 300 instructions, 300000 shots, peak 1 to 5: 1.3 to
+    // 3 times as slow as lanes.)
     if (p.peak_rank <= 6 && shots >= 4096) {
-        const double low = best.threads == 64 ? 1.25 : best.threads == 128 ? 1.05 : best.threads == 256 ? 0.95 : best.threads == 512 ? 0.8 : 0.7;
+        const double low = best.threads == 64 ? 1.25 : best.threads == 128 ? 1.05 : best.threads == 256 ? 0.95 : best.global ? 1.0 : best.threads == 512 ? 0.8 : 0.7;
         return low * cost + 0.045 * p.noise * (double)shots / cus <= lanes_us(p, shots, cus);
     }
     return true;
